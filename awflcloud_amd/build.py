@@ -77,7 +77,7 @@ def build_parity():
     for name, (mask, nocontract) in PARITY_BUILDS.items():
         obj = os.path.join(objdir, "parity_%s.o" % name)
         cmd = [HIPCC] + HIP_FLAGS + ["-DAWFL_LEAN", "-DAWFL_PARITY=%d" % mask] + \
-            (["-ffp-contract=off"] if nocontract or name == "contract" else []) + \
+            (["-ffp-contract=off", "-DAWFL_NOFMA"] if nocontract or name == "contract" else []) + \
             ["-c", os.path.join(CSRC, "awfl_dycore.hip"), "-o", obj]
         print("+", " ".join(cmd), flush=True)
         procs.append((name, obj, subprocess.Popen(cmd)))

@@ -68,6 +68,13 @@ AWFL_HD Dual sqrt_g(const Dual& x) {
   return Dual(s, 0.5 * x.d * rcp(s));
 }
 
+// a b + c d with the value rounded as the production face averages round it
+// (face_averages in awfl_cell.hpp), so that the upwind test sees the same sign
+AWFL_HD double dot2(double a, double b, double c, double d) { return fma(a, b, c * d); }
+AWFL_HD Dual dot2(const Dual& a, const Dual& b, const Dual& c, const Dual& d) {
+  return Dual(fma(a.v, b.v, c.v * d.v), a.d * b.v + a.v * b.d + c.d * d.v + c.v * d.d);
+}
+
 // the WENO of weno_coefs for T = Dual takes its generic (non-double) branch,
 // which calls rcp_t (found here by argument-dependent lookup)
 AWFL_HD Dual rcp_t(const Dual& x) { return rcp_g(x); }
@@ -229,49 +236,44 @@ AWFL_HD void riemann_fwd(const T (&L)[5], const T (&R)[5], const FaceRef& fr, do
   constexpr int T1 = DIR == 0 ? 2 : 1;
   constexpr int T2 = DIR == 2 ? 2 : 3;
   T r = T(0.5) * (L[0] + R[0]);
-  T un, ut1, ut2, t;
+  T un, ut1, ut2, t, ir, hit;          // averages (face_averages), 1/r, 1/(2 t)
   if constexpr (DIR == 1) {
     un = T(0.5) * (L[NM] + R[NM]);
     ut1 = T(0.5) * (L[T1] + R[T1]);
     ut2 = T(0.5) * (L[T2] + R[T2]);
     t = T(0.5) * (L[4] + R[4]);
+    const T z = rcp_g(r * t);
+    ir = t * z;
+    hit = (T(0.5) * r) * z;
   } else {
-    T iL = rcp_g(L[0]), iR = rcp_g(R[0]);
-    un = T(0.5) * (L[NM] * iL + R[NM] * iR);
-    ut1 = T(0.5) * (L[T1] * iL + R[T1] * iR);
-    ut2 = T(0.5) * (L[T2] * iL + R[T2] * iR);
-    t = T(0.5) * (L[4] * iL + R[4] * iR);
+    const T LR = L[0] * R[0];
+    const T x4 = dot2(L[4], R[0], R[4], L[0]);
+    const T y = LR * x4, z = rcp_g(y * r), iy = z * r;
+    ir = z * y;
+    hit = LR * (iy * LR);
+    const T h = T(0.5) * (iy * x4);
+    un = dot2(L[NM], R[0], R[NM], L[0]) * h;
+    ut1 = dot2(L[T1], R[0], R[T1], L[0]) * h;
+    ut2 = dot2(L[T2], R[0], R[T2], L[0]) * h;
+    t = x4 * h;
   }
-  T p = T(C0) * pow_at(r * t, fr.rt);
-  T cs = sqrt_g(T(GAMMA) * p * rcp_g(r));
-  T it = rcp_g(t);
+  T cs = sqrt_g(T(GAMMA * C0) * pow_at(r * t, fr.rt) * ir);
   T i2c = T(0.5) * rcp_g(cs);
-  T w1, w2, w3;
-  if (val(un) > 0) {
-    T a = L[4] * it;
-    w1 = L[0] - a;
-    w2 = L[T1] - ut1 * a;
-    w3 = L[T2] - ut2 * a;
-  } else {
-    T a = R[4] * it;
-    w1 = R[0] - a;
-    w2 = R[T1] - ut1 * a;
-    w3 = R[T2] - ut2 * a;
-  }
-  T w5 = (un * R[0] - R[NM]) * i2c + T(0.5) * R[4] * it;
-  T w6 = (L[NM] - un * L[0]) * i2c + T(0.5) * L[4] * it;
-  T q1 = w1 + w5 + w6;
-  T qn = un * w1 + (un - cs) * w5 + (un + cs) * w6;
-  T qt1 = w2 + ut1 * w5 + ut1 * w6;
-  T qt2 = w3 + ut2 * w5 + ut2 * w6;
-  T q5 = t * w5 + t * w6;
-  T iq1 = rcp_g(q1);
+  const bool up = val(un) > 0;
+  const T(&U)[5] = up ? L : R;
+  T D = (un * (R[0] - L[0]) + (L[NM] - R[NM])) * i2c;
+  T d = (R[4] - L[4]) * hit;
+  T v = up ? D + d : D - d;
+  T q1 = U[0] + v;
+  T qn = (un * (q1 - r) + T(0.5) * (L[NM] + R[NM])) - cs * d;
+  T q5 = T(0.5) * (L[4] + R[4]) + t * D;
+  T un1 = qn * rcp_g(q1);
   F[0] = qn;
-  F[NM] = qn * qn * iq1 + T(C0) * pow_at(q5, fr.q5);
+  F[NM] = qn * un1 + T(C0) * pow_at(q5, fr.q5);
   if constexpr (DIR == 2) F[NM] -= T(p_face);
-  F[T1] = qn * qt1 * iq1;
-  F[T2] = qn * qt2 * iq1;
-  F[4] = qn * q5 * iq1;
+  F[T1] = un1 * (U[T1] + ut1 * v);
+  F[T2] = un1 * (U[T2] + ut2 * v);
+  F[4] = un1 * q5;
 }
 
 // ---------------------------------------------------------------------------
@@ -286,30 +288,15 @@ AWFL_HD void riemann_adj(const double (&L)[5], const double (&R)[5], const FaceR
   constexpr int T1 = DIR == 0 ? 2 : 1;
   constexpr int T2 = DIR == 2 ? 2 : 3;
   // primal
-  double r = 0.5 * (L[0] + R[0]);
-  double un, ut1, ut2, t, iL = 0, iR = 0;
-  if constexpr (DIR == 1) {
-    un = 0.5 * (L[NM] + R[NM]);
-    ut1 = 0.5 * (L[T1] + R[T1]);
-    ut2 = 0.5 * (L[T2] + R[T2]);
-    t = 0.5 * (L[4] + R[4]);
-  } else {
-    iL = rcp(L[0]);
-    iR = rcp(R[0]);
-    un = 0.5 * (L[NM] * iL + R[NM] * iR);
-    ut1 = 0.5 * (L[T1] * iL + R[T1] * iR);
-    ut2 = 0.5 * (L[T2] * iL + R[T2] * iR);
-    t = 0.5 * (L[4] * iL + R[4] * iR);
-  }
-  double rt = r * t;
-  double p = C0 * pow_at(rt, fr.rt);
-  // 1/r, 1/t and 1/(r t) from one reciprocal
-  const double irt = rcp(rt);
-  double ir = t * irt;
+  const FaceAvg av = face_averages<DIR>(L, R);
+  const double r = av.r, un = av.un, ut1 = av.ut1, ut2 = av.ut2, t = av.t;
+  const double iL = R[0] * av.iLR, iR = L[0] * av.iLR;   // 1/L_0, 1/R_0 (x and z)
+  const double ir = av.ir, it = 2.0 * av.hit, irt = ir * it;
+  const double rt = r * t;
+  const double p = C0 * pow_at(rt, fr.rt);
   double cs2 = GAMMA * p * ir;
   double cs, i2c;
   sqrt_halfrsqrt(cs2, cs, i2c);     // as the forward riemann
-  double it = r * irt;
   double ics = 2.0 * i2c;
   const bool up = un > 0;
   const double(&U)[5] = up ? L : R;

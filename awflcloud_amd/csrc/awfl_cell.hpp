@@ -407,11 +407,12 @@ inline constexpr Weno5Consts kW5{};
 // D_i (c_0 = c_2 = 1), normalised with eps (WenoLimiter.h:153-156)
 template <class T>
 __host__ __device__ __forceinline__ void weno5_first_weights(const T (&D)[4], T (&w)[4]) {
+  AWFL_NO_CONTRACT
   constexpr T c1 = (T)kW5.c1, c3 = (T)kW5.c3;
   if constexpr (std::is_same<T, double>::value) {
     const T D01 = D[0] * D[1], D23 = D[2] * D[3];
     const T n0 = D[1] * D23, n1 = (D[0] * D23) * c1, n2 = D01 * D[3], n3 = (D01 * D[2]) * c3;
-    const T rs = rcp(fma((T)kW5.epsn, D01 * D23, (n0 + n1) + (n2 + n3)));
+    const T rs = rcp(fm((T)kW5.epsn, D01 * D23, (n0 + n1) + (n2 + n3)));
     w[0] = n0 * rs;
     w[1] = n1 * rs;
     w[2] = n2 * rs;
@@ -432,25 +433,26 @@ template <int I, int ORD, class T>
 __host__ __device__ __forceinline__ void weno_map(T w, T& A, T& E) {
   constexpr double d = Weno<ORD>::idl[I];
   constexpr T d3 = (T)(-3.0 * d), dd = (T)(d + d * d), d2 = (T)(d * d), e1 = (T)(1.0 - 2.0 * d);
-  A = w * (w * (w + d3) + dd);
-  E = w * e1 + d2;
+  A = w * fm(w, w + d3, dd);
+  E = fm(w, e1, d2);
 }
 
 template <class T>
 __host__ __device__ __forceinline__ void reconstruct_w5(const T (&u)[5], T (&g)[3]) {
+  AWFL_NO_CONTRACT
   const T d0 = u[1] - u[0], d1 = u[2] - u[1], d2 = u[3] - u[2], d3 = u[4] - u[3];
   const T s0 = d1 - d0, s1 = d2 - d1, s2 = d3 - d2;
-  const T A0 = (T)2 * d1 + s0, A1 = d1 + d2, A2 = (T)2 * d2 - s2;
-  const T M = s2 - s0, Q = (s0 + s2) - (T)2 * s1;
+  const T A0 = fm((T)2, d1, s0), A1 = d1 + d2, A2 = fm((T)2, d2, -s2);
+  const T M = s2 - s0, Q = fm((T)-2, s1, s0 + s2);
   // total variation (times four) of the candidates and, blended with their
   // average by sigma, of the bridge (WenoLimiter.h:133-151)
-  const T t0 = A0 * A0 + ((T)kW5.tvs * s0) * s0;
-  const T t1 = A1 * A1 + ((T)kW5.tvs * s1) * s1;
-  const T t2 = A2 * A2 + ((T)kW5.tvs * s2) * s2;
-  T th = (T)kW5.k0 * (t0 + t2) + (T)kW5.k1 * t1;
-  th += M * ((T)kW5.m1 * A1 + (T)kW5.mm * M);
-  th += Q * ((T)kW5.q1 * s1 + (T)kW5.qq * Q);
-  const T D[4] = {t0 * t0 + (T)kW5.eps, t1 * t1 + (T)kW5.eps, t2 * t2 + (T)kW5.eps, th * th + (T)kW5.eps};
+  const T t0 = fm((T)kW5.tvs * s0, s0, A0 * A0);
+  const T t1 = fm((T)kW5.tvs * s1, s1, A1 * A1);
+  const T t2 = fm((T)kW5.tvs * s2, s2, A2 * A2);
+  T th = fm((T)kW5.k1, t1, (T)kW5.k0 * (t0 + t2));
+  th = fm(M, fm((T)kW5.m1, A1, (T)kW5.mm * M), th);
+  th = fm(Q, fm((T)kW5.q1, s1, (T)kW5.qq * Q), th);
+  const T D[4] = {fm(t0, t0, (T)kW5.eps), fm(t1, t1, (T)kW5.eps), fm(t2, t2, (T)kW5.eps), fm(th, th, (T)kW5.eps)};
   T w[4], a[4], e[4];
   weno5_first_weights(D, w);
   weno_map<0, 5>(w[0], a[0], e[0]);
@@ -464,12 +466,13 @@ __host__ __device__ __forceinline__ void reconstruct_w5(const T (&u)[5], T (&g)[
   const T W13 = W1 + W3;
   const T rs = rcp_t((W0 + W2) + W13);
   const T w3 = W3 * rs, wM = w3 * M, wQ = w3 * Q;
-  const T od = rs * (W0 * A0 + W13 * A1 + W2 * A2) + (T)kW5.od_m * wM;   // four times the odd part at x = 1/2
-  const T ev = rs * (W0 * s0 + W13 * s1 + W2 * s2);
-  const T end = u[2] + (ev * (T)(1.0 / 12.0) + (T)kW5.ev_q * wQ);
-  g[0] = end - (T)0.25 * od;
-  g[1] = u[2] + (ev * (T)(-1.0 / 24.0) + (T)kW5.md_q * wQ);
-  g[2] = end + (T)0.25 * od;
+  // od: four times the odd part at x = 1/2; ev: twelve times the even part
+  const T od = fm(rs, fm(W2, A2, fm(W13, A1, W0 * A0)), (T)kW5.od_m * wM);
+  const T ev = rs * fm(W2, s2, fm(W13, s1, W0 * s0));
+  const T end = u[2] + fm(ev, (T)(1.0 / 12.0), (T)kW5.ev_q * wQ);
+  g[0] = fm((T)-0.25, od, end);
+  g[1] = u[2] + fm(ev, (T)(-1.0 / 24.0), (T)kW5.md_q * wQ);
+  g[2] = fm((T)0.25, od, end);
 }
 
 // ---------------------------------------------------------------------------
@@ -499,16 +502,17 @@ inline constexpr Weno3Consts kW3{};
 
 template <class T>
 __host__ __device__ __forceinline__ void reconstruct_w3(const T (&u)[3], T (&g)[2]) {
+  AWFL_NO_CONTRACT
   const T d0 = u[1] - u[0], d1 = u[2] - u[1];
   const T S = d0 + d1, Q = d1 - d0;
   const T t0 = d0 * d0, t1 = d1 * d1;
-  const T th = (T)kW3.k0 * (t0 + t1) + ((T)kW3.ks * S) * S + ((T)kW3.kd * Q) * Q;
-  const T D[3] = {t0 * t0 + (T)WENO_EPS, t1 * t1 + (T)WENO_EPS, th * th + (T)WENO_EPS};
+  const T th = fm((T)kW3.kd * Q, Q, fm((T)kW3.ks * S, S, (T)kW3.k0 * (t0 + t1)));
+  const T D[3] = {fm(t0, t0, (T)WENO_EPS), fm(t1, t1, (T)WENO_EPS), fm(th, th, (T)WENO_EPS)};
   T w[3], a[3], e[3];
   if constexpr (std::is_same<T, double>::value) {
     const T D01 = D[0] * D[1];
     const T n0 = D[1] * D[2], n1 = D[0] * D[2], n2 = (T)kW3.c2 * D01;
-    const T rs = rcp(fma((T)kW3.epsn, D01 * D[2], (n0 + n1) + n2));
+    const T rs = rcp(fm((T)kW3.epsn, D01 * D[2], (n0 + n1) + n2));
     w[0] = n0 * rs;
     w[1] = n1 * rs;
     w[2] = n2 * rs;
@@ -525,8 +529,8 @@ __host__ __device__ __forceinline__ void reconstruct_w3(const T (&u)[3], T (&g)[
   const T W0 = a[0] * (e[1] * e[2]), W1 = a[1] * (e[0] * e[2]), W2 = a[2] * (e[0] * e[1]);
   const T rs = rcp_t((W0 + W1) + W2);
   const T hw = (T)0.5 * W2;
-  const T od = (T)0.5 * (rs * ((W0 + hw) * d0 + (W1 + hw) * d1));
-  const T mid = u[1] + (T)kW3.ev * ((W2 * rs) * Q);
+  const T od = ((T)0.5 * rs) * fm(W0 + hw, d0, (W1 + hw) * d1);
+  const T mid = fm((T)kW3.ev, (W2 * rs) * Q, u[1]);
   g[0] = mid - od;
   g[1] = mid + od;
 }
@@ -613,157 +617,215 @@ struct SweepK {
 };
 
 // ---------------------------------------------------------------------------
+// n times the derivative of the point values F along the cell at its GLL
+// points (Deriv<NGLL>, the collocation derivative).  With two and three
+// points it is formed from F's first and second difference.
+// ---------------------------------------------------------------------------
+template <int NGLL>
+__host__ __device__ __forceinline__ void gll_deriv(const double (&F)[NGLL], double n, double (&d)[NGLL]) {
+  AWFL_NO_CONTRACT
+  if constexpr (NGLL == 2) {
+    d[0] = d[1] = (F[1] - F[0]) * n;
+  } else if constexpr (NGLL == 3) {
+    const double a = (F[2] - F[0]) * n, c = fm(-2.0, F[1], F[0] + F[2]), h = 2.0 * n;
+    d[0] = fm(-h, c, a);
+    d[1] = a;
+    d[2] = fm(h, c, a);
+  } else {
+    sfor<NGLL>([&](auto ii) {
+      double t = -0.0;
+      sfor<NGLL>([&](auto s) {
+        constexpr double D = Deriv<NGLL>::m[s][ii];
+        if constexpr (D != 0.0) t = fm(D, F[s], t);
+      });
+      d[ii] = t * n;
+    });
+  }
+}
+
+// eL, eR += n times that derivative at the cell's two edges
+template <int NGLL>
+__host__ __device__ __forceinline__ void gll_deriv_edges(const double (&F)[NGLL], double n, double& eL, double& eR) {
+  AWFL_NO_CONTRACT
+  if constexpr (NGLL == 3) {
+    const double a = F[2] - F[0], c = fm(-2.0, F[1], F[0] + F[2]), h = 2.0 * n;
+    eL = fm(-h, c, fm(n, a, eL));
+    eR = fm(h, c, fm(n, a, eR));
+  } else {
+    double d[NGLL];
+    gll_deriv<NGLL>(F, n, d);
+    eL += d[0];
+    eR += d[NGLL - 1];
+  }
+}
+
+// ---------------------------------------------------------------------------
 // One cell of a DIR sweep (0 x, 1 y, 2 z): stencils of the 5 state variables
 // along the sweep axis -> time-averaged left/right edge states (and, for z,
 // the time- and cell-averaged gravity source of rho*w).
+//
+// The transform carries the normal velocity's Taylor coefficients u_k: with
+// u r = q_nm, u_k = (q_nm,k - sum_{j>=1} r_j u_{k-j}) / r_0, the flux of every
+// variable is f_k = sum_j u_j q_{k-j}: the same coefficients as the
+// reference's f_k = (sum_j q_nm,j q_{k-j} - sum_{j>=1} r_j f_{k-j}) / r_0,
+// with one division per point instead of one per variable and half the
+// products.  The last level enters the edge states alone and is formed there.
+// The cell average of the z source follows from the quadrature being exact
+// for a derivative: sum_s w_s dF/dx(s) = F(last) - F(first).  The sweeps are
+// bound by FP64 issue: with gll_deriv, one reciprocal for 1/r and 1/(r t), one
+// branch for the cell's powers and riemann()'s difference form, a (5, 3) y
+// sweep's cell and face went from 1,020 to 830 FP64 operations and a step at
+// 256x256x128 from 1.148 to 1.000 ms; the errors against 64-bit torch did not
+// grow (7.6e-15 -> 7.4e-15 of the state).
 // ---------------------------------------------------------------------------
-// levels(q) receives the transform levels q[var][level][point] (level 0 with
-// the background added) once they are complete: the tracer sweeps take the
-// density and normal-momentum levels from it (S:757-758).
+// levels(r0, u) receives the density at the GLL points (background added) and
+// the normal velocity's Taylor coefficients u[level][point], levels 0 ..
+// NGLL-2, which the tracer sweeps' transform takes (S:757-758).
 template <int ORD, int NGLL, int DIR, class Levels>
 __host__ __device__ __forceinline__ void cell_edges(const double (&st)[5][ORD], const CellBg<NGLL>& bg, bool weno_s,
                                            bool weno_w, const SweepK& K, double (&eL)[5], double (&eR)[5],
                                            double& src_avg, Levels&& levels) {
+  AWFL_NO_CONTRACT
   constexpr int NA = NGLL;             // nAder = ngll (Temporal_ader.h:8)
   constexpr int NM = 1 + DIR;          // momentum normal to the sweep
-  double q[5][NA][NGLL];               // r, ru, rv, rw, rt at every level
-  double f[4][NA][NGLL];               // q_nm*var_l/r for l = 1..4
+  static_assert(NA >= 2, "at least one transform level");
+  double q[5][NA][NGLL];               // r, ru, rv, rw, rt at levels 0 .. NA-2
+  double u[NA][NGLL];                  // normal velocity
   double g[NA][NGLL];                  // (r t)^gamma, levels >= 1 carried doubled (S:1904-1915)
-  double src[NA][NGLL];                // z gravity source
   double rr[NGLL], rrt[NGLL];          // 1/r and 1/(r t) at level 0
 
   // level 0: reconstruction + background
-  double et[NGLL];                     // (rho theta)'/B at the GLL points
   sfor<5>([&](auto l) {
     double gv[NGLL];
     reconstruct<ORD, NGLL>(st[l], (l == idR || l == idT) ? weno_s : weno_w, gv);
     sfor<NGLL>([&](auto ii) { q[l][0][ii] = gv[ii]; });
   });
+  // S:1439 assigns a scalar to the whole SArray: every entry of the source's
+  // level 0 holds the value of the last GLL point
+  const double sv = DIR == 2 ? -GRAV * q[idR][0][NGLL - 1] : 0.0;
+  // (r t)^gamma: r t = rho*theta up to an ulp.  The series near the
+  // background runs for every lane; the general power replaces it where a
+  // point is further off.
+  bool near = true;
   sfor<NGLL>([&](auto ii) {
+    const PowRef& pr = DIR == 2 ? bg.ptG[ii] : bg.pt;
+    const double e = q[idT][0][ii] * pr.rb;
+    g[0][ii] = pow_gamma_series(e, pr.h, pr.l);
+    near = near & (fabs(e) <= NEAR_MAX);
     if constexpr (DIR == 2) {
-      et[ii] = q[idT][0][ii] * bg.ptG[ii].rb;
       q[idR][0][ii] += bg.rG[ii];
       q[idT][0][ii] += bg.rtG[ii];
     } else {
-      et[ii] = q[idT][0][ii] * bg.pt.rb;
       q[idR][0][ii] += bg.r;
       q[idT][0][ii] += bg.rt;
     }
   });
+  if (AWFL_PARITY & AWFL_PAR_POW ? true : !near)
+    sfor<NGLL>([&](auto ii) {
+      const double e = (q[idT][0][ii] - (DIR == 2 ? bg.rtG[ii] : bg.rt)) * (DIR == 2 ? bg.ptG[ii] : bg.pt).rb;
+      if (AWFL_PARITY & AWFL_PAR_POW ? true : !(fabs(e) <= NEAR_MAX)) g[0][ii] = pow_gamma_far(q[idT][0][ii]);
+    });
   if constexpr (DIR == 2) {            // S:1413-1416
     if (bg.wall_top) q[idW][0][NGLL - 1] = 0.0;
     if (bg.wall_bot) q[idW][0][0] = 0.0;
   }
-  double sv = 0.0;
   sfor<NGLL>([&](auto ii) {
-    double r = q[idR][0][ii];
-    rr[ii] = rcp(r);
-    double vel[5];
-    sfor<4>([&](auto m) { vel[m + 1] = q[m + 1][0][ii] * rr[ii]; });
-    sfor<4>([&](auto m) { f[m][0][ii] = r * vel[NM] * vel[m + 1]; });
-    if constexpr (NA > 1) {
-      // (r t)^gamma: r t = rho*theta up to an ulp
-      const PowRef& pr = DIR == 2 ? bg.ptG[ii] : bg.pt;
-      g[0][ii] = pow_gamma_near(q[idT][0][ii], et[ii], pr.h, pr.l);
-      rrt[ii] = rcp(q[idT][0][ii]);
+    const double r = q[idR][0][ii], rt = q[idT][0][ii];
+    if constexpr (NA > 2) {
+      const double z = rcp(r * rt);
+      rr[ii] = rt * z;
+      rrt[ii] = r * z;
+    } else {
+      rr[ii] = rcp(r);
     }
-    if constexpr (DIR == 2) sv = -(q[idR][0][ii] - bg.rG[ii]) * GRAV;
+    u[0][ii] = q[NM][0][ii] * rr[ii];
   });
-  if constexpr (DIR == 2) {
-    // S:1439 assigns a scalar to the whole SArray: every entry holds the value
-    // of the last GLL point
-    sfor<NA>([&](auto kt) { sfor<NGLL>([&](auto ii) { src[kt][ii] = sv; }); });
-  }
+  sfor<5>([&](auto l) {
+    eL[l] = q[l][0][0];
+    eR[l] = q[l][0][NGLL - 1];
+  });
+  double sa = sv;
 
   // differential transform: levels 1..NA-1
   sfor<NA - 1>([&](auto kt) {
     constexpr double rkt1 = 1.0 / (kt + 1.0);
-    const double ndt = K.ndt[kt];
-    sfor<NGLL>([&](auto ii) {
-      double d[5];
-      sfor<5>([&](auto l) { d[l] = -0.0; });
+    constexpr bool last = kt + 2 == NA;
+    const double ndt = K.ndt[kt], tav = K.tav[kt + 1];
+    if constexpr (DIR == 2) sa = fm(-GRAV * (tav * ndt), q[NM][kt][NGLL - 1] - q[NM][kt][0], sa);
+    sfor<5>([&](auto l) {
+      double F[NGLL];
       sfor<NGLL>([&](auto s) {
-        constexpr double D = Deriv<NGLL>::m[s][ii];
-        if constexpr (D == 0.0) return;
-        d[0] += D * q[NM][kt][s];
-        sfor<4>([&](auto m) {
-          constexpr int l = m + 1;
+        if constexpr (l == idR) {
+          F[s] = q[NM][kt][s];
+        } else {
+          double t;
           if constexpr (l == NM) {
-            if constexpr (kt == 0) {
-              if constexpr (DIR == 2) d[l] += D * (f[m][kt][s] + C0 * g[kt][s] - bg.pG[s]);
-              else d[l] += D * (f[m][kt][s] + C0 * g[kt][s]);
-            } else {
-              d[l] += D * (f[m][kt][s] + (0.5 * C0) * g[kt][s]);
-            }
+            if constexpr (kt == 0) t = DIR == 2 ? fm(C0, g[kt][s], -bg.pG[s]) : C0 * g[kt][s];
+            else t = (0.5 * C0) * g[kt][s];
+            t = fm(u[0][s], q[l][kt][s], t);
           } else {
-            d[l] += D * f[m][kt][s];
+            t = u[0][s] * q[l][kt][s];
           }
+          sfor<kt>([&](auto j) { t = fm(u[j + 1][s], q[l][kt - 1 - j][s], t); });
+          F[s] = t;
+        }
+      });
+      if constexpr (last) {
+        gll_deriv_edges<NGLL>(F, ndt * tav, eL[l], eR[l]);
+        if constexpr (DIR == 2 && l == idW) {     // the source at level kt, S:2049
+          eL[l] = kt == 0 ? fm(tav, sv, eL[l]) : fm((-GRAV * rkt1) * tav, q[idR][kt][0], eL[l]);
+          eR[l] = kt == 0 ? fm(tav, sv, eR[l]) : fm((-GRAV * rkt1) * tav, q[idR][kt][NGLL - 1], eR[l]);
+        }
+      } else {
+        double d[NGLL];
+        gll_deriv<NGLL>(F, ndt, d);
+        sfor<NGLL>([&](auto ii) {
+          if constexpr (DIR == 2 && l == idW) d[ii] = kt == 0 ? d[ii] + sv : fm(-GRAV * rkt1, q[idR][kt][ii], d[ii]);
+          q[l][kt + 1][ii] = d[ii];
         });
-      });
-      sfor<5>([&](auto l) {
-        if constexpr (DIR == 2 && l == idW) q[l][kt + 1][ii] = d[l] * ndt + src[kt][ii] * rkt1;
-        else q[l][kt + 1][ii] = d[l] * ndt;
-      });
-      if constexpr (DIR == 2) {        // S:2051-2055
-        if (bg.wall_top) q[idW][kt + 1][NGLL - 1] = 0.0;
-        if (bg.wall_bot) q[idW][kt + 1][0] = 0.0;
-        src[kt + 1][ii] = -q[idR][kt + 1][ii] * GRAV;
+        if constexpr (DIR == 2 && l == idW) {     // S:2051-2055
+          if (bg.wall_top) q[idW][kt + 1][NGLL - 1] = 0.0;
+          if (bg.wall_bot) q[idW][kt + 1][0] = 0.0;
+        }
+        eL[l] = fm(q[l][kt + 1][0], tav, eL[l]);   // time averages of the edge values (S:2142-2177)
+        eR[l] = fm(q[l][kt + 1][NGLL - 1], tav, eR[l]);
       }
     });
-    if constexpr (kt + 2 < NA) {       // products at level kt+1 are used only below the last level
+    if constexpr (!last) {
       sfor<NGLL>([&](auto ii) {
-        sfor<4>([&](auto m) {
-          constexpr int l = m + 1;
-          double tot = 0.0;
-          sfor<kt + 2>([&](auto ir) {
-            if constexpr (ir == 0) tot += q[NM][ir][ii] * q[l][kt + 1 - ir][ii];   // f(kt+1) is still 0
-            else tot += q[NM][ir][ii] * q[l][kt + 1 - ir][ii] - q[idR][ir][ii] * f[m][kt + 1 - ir][ii];
+        double t = q[NM][kt + 1][ii];
+        sfor<kt + 1>([&](auto j) { t = fm(-q[idR][j + 1][ii], u[kt - j][ii], t); });
+        u[kt + 1][ii] = t * rr[ii];
+        if constexpr (kt == 0) {
+          g[1][ii] = (2.0 * GAMMA) * ((g[0][ii] * rrt[ii]) * q[idT][1][ii]);
+        } else {
+          double tg = 0.0;
+          sfor<kt + 1>([&](auto ir) {
+            constexpr double wgt = kt + 1.0 - ir;
+            double p = (GAMMA * g[ir][ii]) * q[idT][kt + 1 - ir][ii];
+            if constexpr (ir > 0) p = fm(-q[idT][ir][ii], g[kt + 1 - ir][ii], p);
+            tg = fm(wgt, p, tg);
           });
-          f[m][kt + 1][ii] = tot * rr[ii];
-        });
-        double tg = 0.0;
-        sfor<kt + 1>([&](auto ir) {
-          constexpr double wgt = kt + 1.0 - ir;
-          if constexpr (ir == 0)          // g(kt+1) is still 0
-            tg += wgt * (GAMMA * g[ir][ii] * q[idT][kt + 1 - ir][ii]);
-          else
-            tg += wgt * (GAMMA * g[ir][ii] * q[idT][kt + 1 - ir][ii] - q[idT][ir][ii] * g[kt + 1 - ir][ii]);
-        });
-        g[kt + 1][ii] = (GAMMA * g[0][ii] * q[idT][kt + 1][ii] + tg * rkt1) * rrt[ii];
+          g[kt + 1][ii] = fm(GAMMA * g[0][ii], q[idT][kt + 1][ii], tg * rkt1) * rrt[ii];
+        }
       });
     }
   });
-
-  levels(q);
-  // time averages of the edge values (S:2142-2177)
-  sfor<5>([&](auto l) {
-    double a0 = q[l][0][0], a1 = q[l][0][NGLL - 1];
-    sfor<NA - 1>([&](auto km) {
-      constexpr int kt = km + 1;
-      a0 += q[l][kt][0] * K.tav[kt];
-      a1 += q[l][kt][NGLL - 1] * K.tav[kt];
-    });
-    eL[l] = a0;
-    eR[l] = a1;
-  });
-  if constexpr (DIR == 2) {            // S:1462, 1489-1492
-    sfor<NA - 1>([&](auto km) {
-      constexpr int kt = km + 1;
-      sfor<NGLL>([&](auto ii) { src[0][ii] += src[kt][ii] * K.tav[kt]; });
-    });
-    double sa = 0.0;
-    sfor<NGLL>([&](auto ii) { sa += src[0][ii] * Gll<NGLL>::wts[ii]; });
-    src_avg = sa;
-  } else {
-    src_avg = 0.0;
+  if constexpr (DIR == 2) {
+    if (bg.wall_top) eR[idW] = 0.0;
+    if (bg.wall_bot) eL[idW] = 0.0;
   }
+
+  const double(&r0)[NGLL] = q[idR][0];
+  levels(r0, u);
+  src_avg = DIR == 2 ? sa : 0.0;       // S:1462, 1489-1492
 }
 
 template <int ORD, int NGLL, int DIR>
 __host__ __device__ __forceinline__ void cell_edges(const double (&st)[5][ORD], const CellBg<NGLL>& bg, bool weno_s,
                                            bool weno_w, const SweepK& K, double (&eL)[5], double (&eR)[5],
                                            double& src_avg) {
-  cell_edges<ORD, NGLL, DIR>(st, bg, weno_s, weno_w, K, eL, eR, src_avg, [](const auto&) {});
+  cell_edges<ORD, NGLL, DIR>(st, bg, weno_s, weno_w, K, eL, eR, src_avg, [](const auto&, const auto&) {});
 }
 
 // ---------------------------------------------------------------------------
@@ -771,62 +833,87 @@ __host__ __device__ __forceinline__ void cell_edges(const double (&st)[5][ORD], 
 // variables; Y averages the conservative variables (S:1210-1214).  The
 // normal velocity test is strict (u > 0).
 // ---------------------------------------------------------------------------
-// un_out receives the averaged normal velocity the flux upwinds with (the
-// tracer fluxes upwind with the same value, S:891-900).  With FORCE the
-// upwind side of waves 1-3 is up_forced (true: left) instead of the sign
-// test: the flux with a frozen branch, for difference checks of the adjoint.
-template <int DIR, bool FORCE = false>
-__host__ __device__ __forceinline__ void riemann(const double (&L)[5], const double (&R)[5], const FaceRef& fr,
-                                        double (&F)[5], double& un_out, bool up_forced = false) {
+// Averages of the two edge states at a face and the reciprocals that go with
+// them.  In x and z the velocities and theta are averaged: with X_l = L_l R_0 +
+// R_l L_0 they are X_l / (2 L_0 R_0), and 1/r, 1/(L_0 R_0) and 1/t come from
+// one reciprocal (of r L_0 R_0 X_4) by products.  The adjoint forms its
+// averages here too, so that both take the same upwind side.
+struct FaceAvg {
+  double r, un, ut1, ut2, t;
+  double ir, hit;                      // 1/r, 1/(2 t)
+  double iLR;                          // 1/(L_0 R_0) (x and z)
+};
+template <int DIR>
+__host__ __device__ __forceinline__ FaceAvg face_averages(const double (&L)[5], const double (&R)[5]) {
+  AWFL_NO_CONTRACT
   constexpr int NM = 1 + DIR;
   // tangential momentum indices in the order the reference uses them
   constexpr int T1 = DIR == 0 ? 2 : 1;
   constexpr int T2 = DIR == 2 ? 2 : 3;
-  double r = 0.5 * (L[0] + R[0]);
-  double un, ut1, ut2, t;
+  FaceAvg a;
+  a.r = 0.5 * (L[0] + R[0]);
   if constexpr (DIR == 1) {
-    un = 0.5 * (L[NM] + R[NM]);
-    ut1 = 0.5 * (L[T1] + R[T1]);
-    ut2 = 0.5 * (L[T2] + R[T2]);
-    t = 0.5 * (L[4] + R[4]);
+    a.un = 0.5 * (L[NM] + R[NM]);
+    a.ut1 = 0.5 * (L[T1] + R[T1]);
+    a.ut2 = 0.5 * (L[T2] + R[T2]);
+    a.t = 0.5 * (L[4] + R[4]);
+    const double z = rcp(a.r * a.t);
+    a.ir = a.t * z;
+    a.hit = (0.5 * a.r) * z;
+    a.iLR = 0.0;
   } else {
-    double rL = rcp(L[0]), rR = rcp(R[0]);
-    un = 0.5 * (L[NM] * rL + R[NM] * rR);
-    ut1 = 0.5 * (L[T1] * rL + R[T1] * rR);
-    ut2 = 0.5 * (L[T2] * rL + R[T2] * rR);
-    t = 0.5 * (L[4] * rL + R[4] * rR);
+    const double LR = L[0] * R[0];
+    const double x4 = fm(L[4], R[0], R[4] * L[0]);
+    const double y = LR * x4, z = rcp(y * a.r), iy = z * a.r;
+    a.ir = z * y;
+    a.iLR = iy * x4;
+    a.hit = LR * (iy * LR);
+    const double h = 0.5 * a.iLR;
+    a.un = fm(L[NM], R[0], R[NM] * L[0]) * h;
+    a.ut1 = fm(L[T1], R[0], R[T1] * L[0]) * h;
+    a.ut2 = fm(L[T2], R[0], R[T2] * L[0]) * h;
+    a.t = x4 * h;
   }
-  double p = C0 * pow_gamma_near(r * t, fma(r, t, -fr.rt.b) * fr.rt.rb, fr.rt.h, fr.rt.l);
-  double cs2 = GAMMA * p * rcp(r);
+  return a;
+}
+
+// un_out receives the averaged normal velocity the flux upwinds with (the
+// tracer fluxes upwind with the same value, S:891-900).  With FORCE the
+// upwind side of waves 1-3 is up_forced (true: left) instead of the sign
+// test: the flux with a frozen branch, for difference checks of the adjoint.
+//
+// The waves and the recomposed state (S:866-882) are taken together, in
+// differences of the two sides, so that 1/t and cs act on differences only:
+// with D = (u_n (R_0 - L_0) + L_n - R_n) / (2 cs) and d = (R_4 - L_4) / (2 t),
+//   q5 = (L_4 + R_4)/2 + t D,  v = D + d (left upwind) or D - d,
+//   q1 = U_0 + v,  q_t = U_t + u_t v  (U the upwind side),
+//   q_n = u_n (q1 - r) + (L_n + R_n)/2 - cs d.
+template <int DIR, bool FORCE = false>
+__host__ __device__ __forceinline__ void riemann(const double (&L)[5], const double (&R)[5], const FaceRef& fr,
+                                        double (&F)[5], double& un_out, bool up_forced = false) {
+  AWFL_NO_CONTRACT
+  constexpr int NM = 1 + DIR;
+  constexpr int T1 = DIR == 0 ? 2 : 1;
+  constexpr int T2 = DIR == 2 ? 2 : 3;
+  const FaceAvg m = face_averages<DIR>(L, R);
+  const double pw = pow_gamma_near(m.r * m.t, fm(m.r, m.t, -fr.rt.b) * fr.rt.rb, fr.rt.h, fr.rt.l);
   double cs, r2c;
-  sqrt_halfrsqrt(cs2, cs, r2c);
-  double rt = rcp(t);
-  double w1, w2, w3;
-  if (FORCE ? up_forced : un > 0) {
-    double a = L[4] * rt;
-    w1 = L[0] - a;
-    w2 = L[T1] - ut1 * a;
-    w3 = L[T2] - ut2 * a;
-  } else {
-    double a = R[4] * rt;
-    w1 = R[0] - a;
-    w2 = R[T1] - ut1 * a;
-    w3 = R[T2] - ut2 * a;
-  }
-  double w5 = (un * R[0] - R[NM]) * r2c + 0.5 * R[4] * rt;
-  double w6 = (L[NM] - un * L[0]) * r2c + 0.5 * L[4] * rt;
-  double q1 = w1 + w5 + w6;
-  double qn = un * w1 + (un - cs) * w5 + (un + cs) * w6;
-  double qt1 = w2 + ut1 * w5 + ut1 * w6;
-  double qt2 = w3 + ut2 * w5 + ut2 * w6;
-  double q5 = t * w5 + t * w6;
-  double rq1 = rcp(q1);
+  sqrt_halfrsqrt((GAMMA * C0) * pw * m.ir, cs, r2c);
+  const bool up = FORCE ? up_forced : m.un > 0;
+  const double u0 = up ? L[0] : R[0], u1 = up ? L[T1] : R[T1], u2 = up ? L[T2] : R[T2];
+  const double D = fm(m.un, R[0] - L[0], L[NM] - R[NM]) * r2c;
+  const double d = (R[4] - L[4]) * m.hit;
+  const double v = D + (up ? d : -d);
+  const double q1 = u0 + v;
+  const double qn = fm(-cs, d, fm(m.un, q1 - m.r, 0.5 * (L[NM] + R[NM])));
+  const double q5 = fm(m.t, D, 0.5 * (L[4] + R[4]));
+  const double un1 = qn * rcp(q1);
   F[0] = qn;
-  F[NM] = qn * qn * rq1 + C0 * pow_gamma_near(q5, (q5 - fr.q5.b) * fr.q5.rb, fr.q5.h, fr.q5.l);
-  F[T1] = qn * qt1 * rq1;
-  F[T2] = qn * qt2 * rq1;
-  F[4] = qn * q5 * rq1;
-  un_out = un;
+  F[NM] = fm(qn, un1, C0 * pow_gamma_near(q5, (q5 - fr.q5.b) * fr.q5.rb, fr.q5.h, fr.q5.l));
+  F[T1] = un1 * fm(m.ut1, v, u1);
+  F[T2] = un1 * fm(m.ut2, v, u2);
+  F[4] = un1 * q5;
+  un_out = m.un;
 }
 
 template <int DIR>

@@ -281,15 +281,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(AWFL_COL_WAV
       else F[idW] -= G.hyPressureGLL[(G.nz - 1) * NGLL + NGLL - 1];
     }
   };
-  // result of one cell (new state, or its tendency) into registers, and its store
-  auto update = [&](const double (&F0)[5], const double (&F1)[5], double src, const double (&cell)[5],
-                    double (&res)[5]) {
+  double w[5][ORD];                    // the window of the walk
+  // result of one cell (new state, or its tendency) into registers, and its
+  // store; the cell sits at w[.][at]
+  auto update = [&](const double (&F0)[5], const double (&F1)[5], double src, int at, double (&res)[5]) {
 #pragma unroll
     for (int l = 0; l < 5; l++) {
       double td = flux_div(F1[l], F0[l], K);
       if (DIR == 2 && l == idW) td = src + td;
       if (DIR == 2 && G.sim2d && l == idV) td = 0.0;
-      res[l] = TEND ? td : cell[l] + K.dt * td;
+      res[l] = TEND ? td : w[l][at] + K.dt * td;
     }
   };
   auto put = [&](int c, const double (&res)[5]) {
@@ -304,9 +305,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(AWFL_COL_WAV
     }
   };
 
-  double w[5][ORD];
   sfor<5>([&](auto l) { sfor<ORD>([&](auto s) { w[l][s] = ld(l, s0 - 1 - hs + s); }); });
-  double prevR[5], prevF[5], prevCell[5], prevSrc = 0.0;
+  double prevR[5], prevF[5], prevSrc = 0.0;
   if (per || s0 > 0) {                 // right edge of the cell below the segment
     CellBg<NGLL> bg;
     bg_of(((s0 - 1) % n + n) % n, bg);
@@ -320,7 +320,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(AWFL_COL_WAV
   double nxt[5], res[5];
   sfor<5>([&](auto l) {
     nxt[l] = ld(l, s0 + hs);
-    prevF[l] = prevCell[l] = res[l] = 0.0;
+    prevF[l] = res[l] = 0.0;
   });
   for (int v = s0; v < s1; v++) {
     if (v > s0 + 1) put(v - 2, res);
@@ -335,15 +335,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(AWFL_COL_WAV
     cellns::cell_edges<ORD, NGLL, DIR>(w, bg, G.weno_s, G.weno_w, K, eL, eR, src);
     double F[5];
     FaceRef fr = face_ref(v);
-    if (!per && v == 0) face_flux<DIR, BR>(eL, eL, fr, F, branch(v));   // wall: both sides from the first cell
-    else face_flux<DIR, BR>(prevR, eL, fr, F, branch(v));
+    if (!per && v == 0) sfor<5>([&](auto l) { prevR[l] = eL[l]; });   // wall: both sides from the first cell
+    face_flux<DIR, BR>(prevR, eL, fr, F, branch(v));
     face_bg(v, F);
-    update(prevF, F, prevSrc, prevCell, res);   // cell v-1 (for v == s0 a value never stored)
+    update(prevF, F, prevSrc, hs - 1, res);   // cell v-1 (for v == s0 a value never stored)
 #pragma unroll
     for (int l = 0; l < 5; l++) {
       prevF[l] = F[l];
       prevR[l] = eR[l];
-      prevCell[l] = w[l][hs];
     }
     prevSrc = src;
   }
@@ -351,13 +350,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(AWFL_COL_WAV
   // top face of the segment
   double F[5];
   FaceRef fr = face_ref(s1);
+  sfor<5>([&](auto l) {
+    sfor<ORD - 1>([&](auto s) { w[l][s] = w[l][s + 1]; });
+    w[l][ORD - 1] = nxt[l];            // cell s1 + hs, loaded by the last iteration
+  });
   if (!per && s1 == n) {
     face_flux<DIR, BR>(prevR, prevR, fr, F, branch(s1));   // wall: both sides from the last cell
   } else {
-    sfor<5>([&](auto l) {
-      sfor<ORD - 1>([&](auto s) { w[l][s] = w[l][s + 1]; });
-      w[l][ORD - 1] = nxt[l];          // cell s1 + hs, loaded by the last iteration
-    });
     CellBg<NGLL> bg;
     bg_of(s1 % n, bg);
     double eL[5], eR[5], sa_;
@@ -365,7 +364,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(AWFL_COL_WAV
     face_flux<DIR, BR>(prevR, eL, fr, F, branch(s1));
   }
   face_bg(s1, F);
-  update(prevF, F, prevSrc, prevCell, res);
+  update(prevF, F, prevSrc, hs - 1, res);
   put(s1 - 1, res);
 }
 

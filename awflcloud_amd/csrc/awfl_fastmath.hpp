@@ -1,7 +1,8 @@
 // awfl_fastmath.hpp -- FP64 building blocks of the sweep kernels.
 //
 // * rcp(x): 1/x for positive (or negative) normal x from the hardware
-//   reciprocal estimate refined by two Newton-Raphson steps (|err| <~ 1 ulp).
+//   reciprocal estimate (good to 2^-23) refined by one third-order step
+//   (|err| <~ 1 ulp).
 // * pow_gamma(x): x^GAMMA for positive normal x, GAMMA the FP64 constant
 //   CP/CV of the equation of state p = C0 (rho theta)^GAMMA.  Computed as
 //   exp(GAMMA * log(x)) with log in double-double (atanh series after
@@ -22,6 +23,7 @@
 // the device library's pow; AWFL_PAR_BRIDGE forms the WENO bridge polynomial
 // by its three statements instead of the folded map; AWFL_PAR_ORDER runs the
 // cell and face bodies in the reference's operation order (awfl_cell_ref.hpp).
+// AWFL_NOFMA makes fm() a product and a sum.
 #pragma once
 #define AWFL_PAR_DIV 1
 #define AWFL_PAR_POW 2
@@ -49,6 +51,27 @@ using std::rint;
 using std::fabs;
 
 
+// a b + c, rounded once.  The sweeps' cell and face bodies write their
+// multiply-adds with it and switch the compiler's own contraction off
+// (AWFL_NO_CONTRACT): left to itself the compiler picks which product of a b + c
+// d it fuses by each kernel's instruction order, and the same statements then
+// round differently in the recording, tendency, tracer and production kernels.
+#if defined(__clang__)
+#define AWFL_NO_CONTRACT _Pragma("clang fp contract(off)")
+#else
+#define AWFL_NO_CONTRACT
+#endif
+#ifdef AWFL_NOFMA
+template <class T>
+__host__ __device__ __forceinline__ T fm(T a, T b, T c) {
+  AWFL_NO_CONTRACT
+  return a * b + c;
+}
+#else
+__host__ __device__ __forceinline__ double fm(double a, double b, double c) { return fma(a, b, c); }
+__host__ __device__ __forceinline__ float fm(float a, float b, float c) { return std::fma(a, b, c); }
+#endif
+
 constexpr double POW_GAMMA = 1.40027894002789400278940027894;
 
 __host__ __device__ __forceinline__ double rcp(double x) {
@@ -60,11 +83,10 @@ __host__ __device__ __forceinline__ double rcp(double x) {
 #else
   double r = 1.0 / x;
 #endif
-  double e = fma(-x, r, 1.0);
-  r = fma(r, e, r);
-  e = fma(-x, r, 1.0);
-  r = fma(r, e, r);
-  return r;
+  // r (1 + e + e^2), e = 1 - x r: the error e^3 is below 2^-69, one operation
+  // fewer than two Newton-Raphson steps
+  const double e = fma(-x, r, 1.0);
+  return fma(r, fma(e, e, e), r);
 }
 
 // sqrt(x) and 1/(2 sqrt(x)) for a positive normal x: two Goldschmidt steps from
@@ -174,40 +196,52 @@ __host__ __device__ __forceinline__ double pow_gamma(double x) {
   return ldexp(er, (int)k);
 }
 
-// (1+e)^GAMMA by its binomial series, degree 12: truncation < 3e-19 relative
-// for |e| <= 1/16.  Coefficients c_n = binom(GAMMA, n), c_0 = 1.
+// Binomial coefficients c_n = binom(GAMMA, n) of (1+e)^GAMMA (the FP32 form's
+// series).
 struct BinomGamma {
-  double c[13];
+  double c[6];
   constexpr BinomGamma() : c() {
     c[0] = 1.0;
-    for (int n = 1; n <= 12; n++) c[n] = c[n - 1] * (POW_GAMMA - (n - 1)) / n;
+    for (int n = 1; n <= 5; n++) c[n] = c[n - 1] * (POW_GAMMA - (n - 1)) / n;
   }
 };
 constexpr BinomGamma BINOM_GAMMA{};
+
+// ((1+e)^GAMMA - 1)/e for |e| <= 1/16 by its degree-8 interpolant at the
+// Chebyshev nodes of that interval (solved in 400-bit arithmetic, rounded to
+// double): 7.4e-18 of (1+e)^GAMMA at most, the accuracy that the binomial
+// series reaches with three more terms.
 constexpr double NEAR_MAX = 0.0625;
+constexpr double POWQ[9] = {0x1.6678ae3cb2859p+0,  0x1.1efa23f1c07b4p-2, -0x1.caf32d76b876cp-5,
+                            0x1.6f188e4832539p-6,  -0x1.7dbd21f235928p-7, 0x1.ca0c4b6827194p-8,
+                            -0x1.2cfbfec853229p-8, 0x1.a76e8eee2355cp-9,  -0x1.369ab21a1d5e9p-9};
 
 // x^GAMMA for x = B (1 + e) near a reference value B whose power is known as
 // a double-double Bh + Bl = B^GAMMA: B^GAMMA (1 + s) with s = (1+e)^GAMMA - 1
-// from the series, added as Bh + (Bh s + Bl (1+s)) so only the last addition
-// rounds at full size (~0.6 ulp).  Outside |e| <= 1/16 the general
-// pow_gamma(x) is used.
-// out-of-line general path, so the five inlined uses of the fast path do not
-// each carry its code and constants
+// from the interpolant, added as Bh + (Bh s + Bl (1+s)) so only the last
+// addition rounds at full size (~0.6 ulp).
+__host__ __device__ __forceinline__ double pow_gamma_series(double e, double Bh, double Bl) {
+  double q = POWQ[8];
+#pragma unroll
+  for (int n = 7; n >= 0; n--) q = fma(q, e, POWQ[n]);
+  const double sv = q * e;
+  return Bh + fma(Bh, sv, fma(Bl, sv, Bl));
+}
+
+// out-of-line general path, so the inlined uses of the fast path do not each
+// carry its code and constants
 __host__ __device__ __attribute__((noinline)) inline double pow_gamma_far(double x) { return pow_gamma(x); }
 
+// The series near the reference value, computed unconditionally (it then sits
+// in straight-line code, free to be scheduled with its neighbours), and the
+// general pow_gamma(x) in its place outside |e| <= 1/16.
 __host__ __device__ __forceinline__ double pow_gamma_near(double x, double e, double Bh, double Bl) {
 #if AWFL_PARITY & AWFL_PAR_POW
   return pow_gamma_far(x);
 #endif
-  if (fabs(e) <= NEAR_MAX) {
-    double q = BINOM_GAMMA.c[12];
-#pragma unroll
-    for (int n = 11; n >= 1; n--) q = fma(q, e, BINOM_GAMMA.c[n]);
-    double sv = q * e;
-    double t = fma(Bl, sv, Bl);
-    return Bh + fma(Bh, sv, t);
-  }
-  return pow_gamma_far(x);
+  double r = pow_gamma_series(e, Bh, Bl);
+  if (!(fabs(e) <= NEAR_MAX)) r = pow_gamma_far(x);
+  return r;
 }
 
 }  // namespace awfl

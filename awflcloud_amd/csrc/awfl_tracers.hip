@@ -73,6 +73,46 @@ __device__ __forceinline__ int wrap_axis(int a, int n, bool per, bool& zn) {
   return a;
 }
 
+// Time-averaged edge values of rho*q of one cell from the mixing ratio's GLL
+// values gv, the density r0 there and the normal velocity's Taylor
+// coefficients ul of the cell's transform: diffTransformTracer (S:2095-2126)
+// with the flux of level k as sum_j u_j rt_{k-j} (awfl_cell.hpp:
+// cell_edges), clipped at zero before and after for a positive tracer
+// (S:760-809).
+template <int NGLL>
+__device__ __forceinline__ void tracer_edges(const double (&gv)[NGLL], const double (&r0)[NGLL],
+                                             const double (&ul)[NGLL - 1][NGLL], bool positive, const SweepK& K,
+                                             double& a0, double& a1) {
+  AWFL_NO_CONTRACT
+  constexpr int NA = NGLL;
+  double rt[NA][NGLL];
+  sfor<NGLL>([&](auto ii) {
+    rt[0][ii] = gv[ii] * r0[ii];
+    if (positive) rt[0][ii] = fmax(0.0, rt[0][ii]);
+  });
+  a0 = rt[0][0];
+  a1 = rt[0][NGLL - 1];
+  sfor<NA - 1>([&](auto kt) {
+    double F[NGLL];
+    sfor<NGLL>([&](auto s) {
+      double t = ul[0][s] * rt[kt][s];
+      sfor<kt>([&](auto j) { t = fm(ul[j + 1][s], rt[kt - 1 - j][s], t); });
+      F[s] = t;
+    });
+    if constexpr (kt + 2 == NA) {
+      gll_deriv_edges<NGLL>(F, K.ndt[kt] * K.tav[kt + 1], a0, a1);
+    } else {
+      gll_deriv<NGLL>(F, K.ndt[kt], rt[kt + 1]);
+      a0 = fm(rt[kt + 1][0], K.tav[kt + 1], a0);
+      a1 = fm(rt[kt + 1][NGLL - 1], K.tav[kt + 1], a1);
+    }
+  });
+  if (positive) {
+    a0 = fmax(0.0, a0);
+    a1 = fmax(0.0, a1);
+  }
+}
+
 // One line of a DIR sweep with ntr tracers.  LDS (doubles), n cells, W =
 // n + 2hs, NF = n + 1 faces:
 //   state line [5][W] (then the state fluxes [5][NF]), mixing ratios
@@ -218,14 +258,12 @@ __device__ __forceinline__ void sweep_tr(const double* __restrict__ in, const do
       bg.wall_bot = bg.wall_top = false;
     }
     double st[5][ORD], eL[5], eR[5], sa;
-    double rl[NA][NGLL], nl[NA][NGLL];
+    double rl[NGLL], ul[NA - 1][NGLL];
     sfor<5>([&](auto l) { sfor<ORD>([&](auto s) { st[l][s] = s_st[l * W + c + s]; }); });
-    cell_edges<ORD, NGLL, DIR>(st, bg, G.weno_s, G.weno_w, K, eL, eR, sa, [&](const auto& q) {
-      sfor<NA>([&](auto kt) {
-        sfor<NGLL>([&](auto ii) {
-          rl[kt][ii] = q[idR][kt][ii];
-          nl[kt][ii] = q[NM][kt][ii];
-        });
+    cell_edges<ORD, NGLL, DIR>(st, bg, G.weno_s, G.weno_w, K, eL, eR, sa, [&](const auto& r0, const auto& u) {
+      sfor<NGLL>([&](auto ii) {
+        rl[ii] = r0[ii];
+        sfor<NA - 1>([&](auto kt) { ul[kt][ii] = u[kt][ii]; });
       });
     });
     sfor<5>([&](auto l) {
@@ -233,47 +271,13 @@ __device__ __forceinline__ void sweep_tr(const double* __restrict__ in, const do
       s_e[(5 + l) * n + c] = eR[l];
     });
     if constexpr (DIR == 2) s_src[c] = sa;
-    double rr0[NGLL];
-    sfor<NGLL>([&](auto ii) { rr0[ii] = rcp(rl[0][ii]); });
     for (int t = 0; t < ntr; t++) {
       const bool tp = (pos >> t) & 1u;
       double u[ORD], g[NGLL];
       sfor<ORD>([&](auto s) { u[s] = s_tq[t * W + c + s]; });
       reconstruct<ORD, NGLL>(u, G.weno_s, g);
-      double rt[NA][NGLL], rnt[NA][NGLL];
-      sfor<NGLL>([&](auto ii) {
-        rt[0][ii] = g[ii] * rl[0][ii];
-        if (tp) rt[0][ii] = fmax(0.0, rt[0][ii]);
-        rnt[0][ii] = rt[0][ii] * nl[0][ii] * rr0[ii];
-      });
-      // diffTransformTracer (S:2095-2126)
-      sfor<NA - 1>([&](auto kt) {
-        sfor<NGLL>([&](auto ii) {
-          double df = 0.0;
-          sfor<NGLL>([&](auto s) { df += Deriv<NGLL>::m[s][ii] * rnt[kt][s]; });
-          rt[kt + 1][ii] = df * K.ndt[kt];
-        });
-        if constexpr (kt + 2 < NA) {     // the flux at the last level is not used
-          sfor<NGLL>([&](auto ii) {
-            double tot = 0.0;
-            sfor<kt + 2>([&](auto ir) {
-              if constexpr (ir == 0) tot += nl[ir][ii] * rt[kt + 1 - ir][ii];
-              else tot += nl[ir][ii] * rt[kt + 1 - ir][ii] - rl[ir][ii] * rnt[kt + 1 - ir][ii];
-            });
-            rnt[kt + 1][ii] = tot * rr0[ii];
-          });
-        }
-      });
-      double a0 = rt[0][0], a1 = rt[0][NGLL - 1];
-      sfor<NA - 1>([&](auto km) {
-        constexpr int kt = km + 1;
-        a0 += rt[kt][0] * K.tav[kt];
-        a1 += rt[kt][NGLL - 1] * K.tav[kt];
-      });
-      if (tp) {
-        a0 = fmax(0.0, a0);
-        a1 = fmax(0.0, a1);
-      }
+      double a0, a1;
+      tracer_edges<NGLL>(g, rl, ul, tp, K, a0, a1);
       s_te[(2 * t) * n + c] = a0;
       s_te[(2 * t + 1) * n + c] = a1;
     }
@@ -727,7 +731,7 @@ __device__ __forceinline__ void walk(const WalkArgs& A, int mode, int s) {
     // (a) cell X: state edges, the source, and the density and normal
     // momentum levels the tracer transform reads
     double eL[5], eR[5], sa;
-    double rl[NA][NGLL], nl[NA][NGLL];
+    double rl[NGLL], ul[NA - 1][NGLL];
     {
       const int Xc = X < n ? X : n - 1;
       CellBg<NGLL> bg{};
@@ -752,12 +756,10 @@ __device__ __forceinline__ void walk(const WalkArgs& A, int mode, int s) {
         const int sk = s0 + k < R ? s0 + k : s0 + k - R;
         sfor<5>([&](auto l) { st[l][k] = rg[l * R + sk]; });
       });
-      cell_edges<ORD, NGLL, DIR>(st, bg, G.weno_s, G.weno_w, K, eL, eR, sa, [&](const auto& q) {
-        sfor<NA>([&](auto kt) {
-          sfor<NGLL>([&](auto ii) {
-            rl[kt][ii] = q[idR][kt][ii];
-            nl[kt][ii] = q[NM][kt][ii];
-          });
+      cell_edges<ORD, NGLL, DIR>(st, bg, G.weno_s, G.weno_w, K, eL, eR, sa, [&](const auto& r0, const auto& u) {
+        sfor<NGLL>([&](auto ii) {
+          rl[ii] = r0[ii];
+          sfor<NA - 1>([&](auto kt) { ul[kt][ii] = u[kt][ii]; });
         });
       });
     }
@@ -831,8 +833,6 @@ __device__ __forceinline__ void walk(const WalkArgs& A, int mode, int s) {
     // update.  Neighbouring lanes' values come by shuffles; lane 0 takes the
     // previous step's last cell from the carry area, which lane cw then
     // overwrites for the next step.
-    double rr0[NGLL];
-    sfor<NGLL>([&](auto ii) { rr0[ii] = rcp(rl[0][ii]); });
     const int sm1 = slot(X - 1);
     const double dns = pos ? rg[idR * R + sm1] + bg_dens(X - 1) : 0.0;
     for (int t = 0; t < ntr; t++) {
@@ -844,40 +844,8 @@ __device__ __forceinline__ void walk(const WalkArgs& A, int mode, int s) {
         u[kk] = mr[t * R + sk];
       });
       reconstruct<ORD, NGLL>(u, G.weno_s, g);
-      double rt[NA][NGLL], rnt[NA][NGLL];
-      sfor<NGLL>([&](auto ii) {
-        rt[0][ii] = g[ii] * rl[0][ii];
-        if (tp) rt[0][ii] = fmax(0.0, rt[0][ii]);
-        rnt[0][ii] = rt[0][ii] * nl[0][ii] * rr0[ii];
-      });
-      // diffTransformTracer (S:2095-2126)
-      sfor<NA - 1>([&](auto kt) {
-        sfor<NGLL>([&](auto ii) {
-          double df = 0.0;
-          sfor<NGLL>([&](auto s2) { df += Deriv<NGLL>::m[s2][ii] * rnt[kt][s2]; });
-          rt[kt + 1][ii] = df * K.ndt[kt];
-        });
-        if constexpr (kt + 2 < NA) {
-          sfor<NGLL>([&](auto ii) {
-            double tot = 0.0;
-            sfor<kt + 2>([&](auto ir) {
-              if constexpr (ir == 0) tot += nl[ir][ii] * rt[kt + 1 - ir][ii];
-              else tot += nl[ir][ii] * rt[kt + 1 - ir][ii] - rl[ir][ii] * rnt[kt + 1 - ir][ii];
-            });
-            rnt[kt + 1][ii] = tot * rr0[ii];
-          });
-        }
-      });
-      double a0 = rt[0][0], a1 = rt[0][NGLL - 1];
-      sfor<NA - 1>([&](auto km) {
-        constexpr int kt = km + 1;
-        a0 += rt[kt][0] * K.tav[kt];
-        a1 += rt[kt][NGLL - 1] * K.tav[kt];
-      });
-      if (tp) {
-        a0 = fmax(0.0, a0);
-        a1 = fmax(0.0, a1);
-      }
+      double a0, a1;
+      tracer_edges<NGLL>(g, rl, ul, tp, K, a0, a1);
       if (s == 0 && c == 0) h_tlo0[t] = a0;
       // face X: rho*q of the upwind side, the high edge of cell X-1 or the low edge of cell X
       const double a1s = __shfl_up(a1, 1);
