@@ -678,13 +678,16 @@ __host__ __device__ __forceinline__ void gll_deriv_edges(const double (&F)[NGLL]
 // 256x256x128 from 1.148 to 1.000 ms; the errors against 64-bit torch did not
 // grow (7.6e-15 -> 7.4e-15 of the state).
 // ---------------------------------------------------------------------------
+// load_bg() returns the cell's background; it is called after the
+// reconstructions, so that a background that differs between lanes is not
+// held in registers through them.
 // levels(r0, u) receives the density at the GLL points (background added) and
 // the normal velocity's Taylor coefficients u[level][point], levels 0 ..
 // NGLL-2, which the tracer sweeps' transform takes (S:757-758).
-template <int ORD, int NGLL, int DIR, class Levels>
-__host__ __device__ __forceinline__ void cell_edges(const double (&st)[5][ORD], const CellBg<NGLL>& bg, bool weno_s,
-                                           bool weno_w, const SweepK& K, double (&eL)[5], double (&eR)[5],
-                                           double& src_avg, Levels&& levels) {
+template <int ORD, int NGLL, int DIR, class LoadBg, class Levels>
+__host__ __device__ __forceinline__ void cell_edges_of(const double (&st)[5][ORD], LoadBg&& load_bg, bool weno_s,
+                                              bool weno_w, const SweepK& K, double (&eL)[5], double (&eR)[5],
+                                              double& src_avg, Levels&& levels) {
   AWFL_NO_CONTRACT
   constexpr int NA = NGLL;             // nAder = ngll (Temporal_ader.h:8)
   constexpr int NM = 1 + DIR;          // momentum normal to the sweep
@@ -700,6 +703,7 @@ __host__ __device__ __forceinline__ void cell_edges(const double (&st)[5][ORD], 
     reconstruct<ORD, NGLL>(st[l], (l == idR || l == idT) ? weno_s : weno_w, gv);
     sfor<NGLL>([&](auto ii) { q[l][0][ii] = gv[ii]; });
   });
+  const CellBg<NGLL> bg = load_bg();
   // S:1439 assigns a scalar to the whole SArray: every entry of the source's
   // level 0 holds the value of the last GLL point
   const double sv = DIR == 2 ? -GRAV * q[idR][0][NGLL - 1] : 0.0;
@@ -821,6 +825,12 @@ __host__ __device__ __forceinline__ void cell_edges(const double (&st)[5][ORD], 
   src_avg = DIR == 2 ? sa : 0.0;       // S:1462, 1489-1492
 }
 
+template <int ORD, int NGLL, int DIR, class Levels>
+__host__ __device__ __forceinline__ void cell_edges(const double (&st)[5][ORD], const CellBg<NGLL>& bg, bool weno_s,
+                                           bool weno_w, const SweepK& K, double (&eL)[5], double (&eR)[5],
+                                           double& src_avg, Levels&& levels) {
+  cell_edges_of<ORD, NGLL, DIR>(st, [&]() { return bg; }, weno_s, weno_w, K, eL, eR, src_avg, levels);
+}
 template <int ORD, int NGLL, int DIR>
 __host__ __device__ __forceinline__ void cell_edges(const double (&st)[5][ORD], const CellBg<NGLL>& bg, bool weno_s,
                                            bool weno_w, const SweepK& K, double (&eL)[5], double (&eR)[5],
@@ -921,6 +931,22 @@ __host__ __device__ __forceinline__ void riemann(const double (&L)[5], const dou
                                         double (&F)[5]) {
   double un;
   riemann<DIR>(L, R, fr, F, un);
+}
+
+// riemann(L, L): both sides of a wall face (S:822-823) are the cell's edge
+// state, whose differences vanish; the remaining statements, bit for bit
+template <int DIR>
+__host__ __device__ __forceinline__ void wall_flux(const double (&L)[5], const FaceRef& fr, double (&F)[5]) {
+  AWFL_NO_CONTRACT
+  constexpr int NM = 1 + DIR;
+  constexpr int T1 = DIR == 0 ? 2 : 1;
+  constexpr int T2 = DIR == 2 ? 2 : 3;
+  const double un1 = L[NM] * rcp(L[0]);
+  F[0] = L[NM];
+  F[NM] = fm(L[NM], un1, C0 * pow_gamma_near(L[4], (L[4] - fr.q5.b) * fr.q5.rb, fr.q5.h, fr.q5.l));
+  F[T1] = un1 * L[T1];
+  F[T2] = un1 * L[T2];
+  F[4] = un1 * L[4];
 }
 
 }  // namespace awfl

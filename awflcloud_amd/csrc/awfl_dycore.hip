@@ -8,13 +8,9 @@
 //    edge states, computes the upwind flux at every face and writes
 //    out = in + dt * tendency (or the tendency itself).  No intermediate
 //    (edge states, fluxes) touches HBM.
-//  * x sweep (contiguous axis): one workgroup per x-line; the line and its
-//    boundary cells are staged in LDS with coalesced loads, edge states and
-//    face fluxes are exchanged through LDS.
-//  * y and z sweeps (strided axes): one lane per x-column walks a segment of
-//    its column along the sweep axis with a register window of ord cells, so
-//    every wavefront load/store is 64 consecutive doubles along x and no LDS
-//    or barrier is needed.
+//  * A work-group takes a tile of lines along the sweep, one lane per cell;
+//    the cells, edge states and face fluxes pass between lanes through LDS
+//    (k_sweep_tile).
 //  * Sweeps run out of place; a fused time step ping-pongs through two
 //    context-owned buffers and ends in the caller's state buffer.
 #include <hip/hip_runtime.h>
@@ -37,15 +33,13 @@
 #endif
 #include "awfl_sweep_line.hpp"
 
-// Cell body of the sweeps: the production numerics, or (reference-order
-// parity builds) the reference's operation order.
-namespace cellns {
+// Cell body of the sweeps: the production numerics, or (reference-order parity
+// builds) the reference's operation order.
 #if AWFL_PARITY & AWFL_PAR_ORDER
-using awfl::ref::cell_edges;
+#define AWFL_CELL awfl::ref
 #else
-using awfl::cell_edges;
+#define AWFL_CELL awfl
 #endif
-}  // namespace cellns
 
 // Flux divergence -(F_high - F_low)/d of one cell along the sweep.
 __device__ __forceinline__ double flux_div(double F1, double F0, const awfl::SweepK& K) {
@@ -65,15 +59,8 @@ __device__ __forceinline__ int64_t tend_index(const Grid& G, int l, int k, int j
 }
 
 // ---------------------------------------------------------------------------
-// x sweep: one workgroup per x-line
+// the sweep kernel
 // ---------------------------------------------------------------------------
-#ifndef AWFL_X_WAVES
-#define AWFL_X_WAVES 1
-#endif
-#ifndef AWFL_COL_WAVES
-#define AWFL_COL_WAVES 1
-#endif
-
 // BR: 0 production; 1 also records each face's upwind branch (un > 0) in
 // K.br; 2 takes the branch from K.br instead of the sign test (frozen-branch
 // forward for difference checks of the adjoint).  Branch bytes: x face f of
@@ -99,115 +86,231 @@ __device__ __forceinline__ void face_flux(const double (&qL)[5], const double (&
   }
 }
 
-// INPLACE: in == out is allowed.  Every global read of the line happens in
-// the staging loop, before the first barrier; the face fluxes get LDS of
-// their own, so the update takes each cell's old value from the staged line
-// instead of reading it again.  (The line belongs to this work-group alone.)
-template <int ORD, int NGLL, bool TEND, int BR = 0, bool INPLACE = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AWFL_X_WAVES))) void k_sweep_x(const double* __restrict__ in, double* __restrict__ out, Grid G,
-                                                 SweepK K) {
+// How a sweep's grid is cut into work-groups (tile_plan).  A work-group holds
+// `cols` lines and of each the rows lo .. lo + rows - 1 along the sweep: the
+// whole line (nseg == 1), or a segment of seglen cells with the neighbouring
+// cell at either end, whose edge state the segment's end faces need and which
+// is reconstructed twice.
+struct TilePlan {
+  int cols, rows, nseg, seglen;
+};
+
+// One lane per cell.  The tile's cells and hs cells beyond either end go
+// through LDS (periodic wrap or wall clamp applied at the load, so there is no
+// halo pass); a lane reconstructs its cell and hands its right edge state to
+// the lane of the next cell through LDS, forms the flux of its low face and
+// hands that back to the previous cell in the same place (the only lane that
+// reads a slot before it is overwritten is the one that overwrites it), and
+// updates its cell.  Every global read happens before the first barrier, so
+// whole lines may be updated in place.
+//
+// What bounds it: FP64 issue (and the clock the FP64 load leaves).  One cell
+// per lane takes 96-106 registers, four or five waves per SIMD, and gives
+// small grids as many waves as they have cells; the column walker
+// (k_sweep_col) needs 203-245 registers, two waves per SIMD, and at 64x64x32
+// fills an eighth of the chip.  LDS holds a cell's 5 values contiguously (40
+// bytes): every stencil address is one base plus a constant, and 32 lanes 10
+// dwords apart touch 64 distinct banks.  Measured against the walkers (y, z)
+// and the former line kernel (x), whose edge states all went through LDS: a
+// step at 64x64x32 123 -> 30 us, a 301x1x75 slice 74 -> 16 us, 128x128x64
+// 190 -> 134 us; x at 256x256x128 346 -> 310 us.
+//
+// TX: lines of a y or z tile, neighbours in x (the lanes of a load run along
+// x); an x tile's lines are neighbours in y.
+constexpr int TILE_THREADS = 1024;
+template <int ORD, int NGLL, int DIR, int TX, bool TEND, int BR = 0>
+__global__ __launch_bounds__(TILE_THREADS) void k_sweep_tile(const double* in, double* out, Grid G, SweepK K,
+                                                             TilePlan T) {
   constexpr int hs = (ORD - 1) / 2;
+  constexpr int NM = 1 + DIR;
   extern __shared__ double sm[];
-  const int nx = G.nx;
-  const int W = nx + 2 * hs;
-  const unsigned line = tile_index();
-  const int j = line % G.ny;
-  const int k = line / G.ny;
-  double* s_st = sm;              // [5][W]   state of the line with boundary cells
-  double* s_L = sm + 5 * W;       // [5][nx]  left edge states
-  double* s_R = s_L + 5 * nx;     // [5][nx]  right edge states
-  // [5][nx+1] face fluxes: over s_st once the edges are formed, or after s_R
-  double* s_F = INPLACE ? s_R + 5 * nx : sm;
-  const int64_t row = (int64_t)(hs + k) * G.sz + (int64_t)(hs + j) * G.sy + hs;
-  const bool per = G.bc[0] == AWFL_BC_PERIODIC;
+  const int n = DIR == 0 ? G.nx : DIR == 1 ? G.ny : G.nz;
+  const int cols = DIR == 0 ? T.cols : TX;
+  const int rows = T.rows;
+  const bool per = G.bc[DIR] == AWFL_BC_PERIODIC;
+  const bool full = T.nseg == 1;
+  // tile -> lines (line index along x or, for x tiles, y; o: the other axis), segment
+  const dim3 tb = tile_coords();
+  const int o = tb.y;                      // x, y tiles: level k; z tiles: j
+  const int s0 = tb.z * T.seglen, s1 = min(n, s0 + T.seglen);
+  const int lo = full || (!per && s0 == 0) ? s0 : s0 - 1;
+  const int nrow = (full || (!per && s1 == n) ? s1 : s1 + 1) - lo;
+  // lane -> column c, row r (cell a of the line)
+  const int t = threadIdx.x;
+  int c, r;
+  if constexpr (DIR == 0) {
+    c = cols == 1 ? 0 : t / rows;
+    r = t - c * rows;
+  } else {
+    c = t % TX;
+    r = t / TX;
+  }
+  const int line = tb.x * cols + c;
+  const int nline = DIR == 0 ? G.ny : G.nx;
+  const bool act = c < cols && r < nrow && line < nline;
+  const int a = lo + r;
+  const int64_t sa = DIR == 0 ? 1 : DIR == 1 ? G.sy : G.sz;
+  auto line_base = [&](int l) -> int64_t {
+    if constexpr (DIR == 0) return (int64_t)(hs + o) * G.sz + (int64_t)(hs + l) * G.sy + hs;
+    else if constexpr (DIR == 1) return (int64_t)(hs + o) * G.sz + (int64_t)hs * G.sy + hs + l;
+    else return (int64_t)hs * G.sz + (int64_t)(hs + o) * G.sy + hs + l;
+  };
+  // LDS slot of row p of column c: staged cells (p from -hs) and edges
+  auto st_slot = [&](int cc, int p) { return 5 * (DIR == 0 ? cc * (rows + 2 * hs) + p + hs : (p + hs) * TX + cc); };
+  auto e_slot = [&](int cc, int p) { return 5 * (DIR == 0 ? cc * rows + p : p * TX + cc); };
+  double* s_st = sm;                                   // [cols][rows + 2hs][5]
+  double* s_e = sm + 5 * cols * (rows + 2 * hs);       // [cols][rows][5]: right edge states, then fluxes
 
-  for (int c = threadIdx.x; c < W; c += blockDim.x) {
-    int ci = c - hs, src;
-    bool zn = false;
+  // stage: a cell of the line or one beyond its ends (S:631-662, 994-1025, 1351-1382)
+  auto source = [&](int v, bool& zn) {
+    zn = false;
+    if (v >= 0 && v < n) return v;
     if (per) {
-      src = ci % nx;
-      if (src < 0) src += nx;
-    } else if (ci < 0) {
-      src = 0; zn = true;
-    } else if (ci >= nx) {
-      src = nx - 1; zn = true;
-    } else {
-      src = ci;
+      if (n > hs + 1) return v < 0 ? v + n : v - n;    // a tile reaches at most hs + 1 cells past the line
+      const int m = v % n;
+      return m < 0 ? m + n : m;
     }
-#pragma unroll
-    for (int l = 0; l < 5; l++) {
-      double v = in[l * G.sl + row + src];
-      s_st[l * W + c] = (zn && l == idU) ? 0.0 : v;
+    zn = true;
+    return v < 0 ? 0 : n - 1;
+  };
+  double own[5];
+  if (act) {
+    bool zn;
+    const int64_t g = line_base(line) + source(a, zn) * sa;
+    sfor<5>([&](auto l) { own[l] = in[l * G.sl + g]; });
+  }
+  for (int h = t; h < 2 * hs * cols; h += blockDim.x) {
+    int hc, hp;                                        // column, and which of the 2 hs cells beyond the tile
+    if constexpr (DIR == 0) {
+      hc = h / (2 * hs);
+      hp = h % (2 * hs);
+    } else {
+      hc = h % TX;
+      hp = h / TX;
+    }
+    if ((int)tb.x * cols + hc < nline) {
+      const int p = hp < hs ? hp - hs : nrow + hp - hs;
+      bool zn;
+      const int64_t g = line_base(tb.x * cols + hc) + source(lo + p, zn) * sa;
+      double v[5];
+      sfor<5>([&](auto l) { v[l] = in[l * G.sl + g]; });
+      if (zn) v[NM] = 0.0;
+      sfor<5>([&](auto l) { s_st[st_slot(hc, p) + l] = v[l]; });
     }
   }
+  if (act) sfor<5>([&](auto l) { s_st[st_slot(c, r) + l] = own[l]; });
   __syncthreads();
 
-  CellBg<NGLL> bg;
-  bg.r = G.hyDensCells[hs + k];
-  bg.rt = G.hyDensThetaCells[hs + k];
-  bg.pt = G.prT[k];
-  bg.wall_bot = bg.wall_top = false;
-  FaceRef fr;
-  fr.rt = bg.pt;
-  fr.q5 = bg.pt;
-  for (int c = threadIdx.x; c < nx; c += blockDim.x) {
+  double eL[5], eR[5], src = 0.0;
+  const int ac = a < 0 ? a + n : a >= n ? a - n : a;   // the cell itself (a line's end wraps)
+  if (act) {
     double st[5][ORD];
-    sfor<5>([&](auto l) { sfor<ORD>([&](auto s) { st[l][s] = s_st[l * W + c + s]; }); });
-    double eL[5], eR[5], sa;
-    cellns::cell_edges<ORD, NGLL, 0>(st, bg, G.weno_s, G.weno_w, K, eL, eR, sa);
-#pragma unroll
-    for (int l = 0; l < 5; l++) {
-      s_L[l * nx + c] = eL[l];
-      s_R[l * nx + c] = eR[l];
-    }
+    const double* w = s_st + st_slot(c, r - hs);
+    constexpr int step = DIR == 0 ? 5 : 5 * TX;
+    sfor<5>([&](auto l) { sfor<ORD>([&](auto s) { st[l][s] = w[s * step + l]; }); });
+    auto load_bg = [&]() {
+      CellBg<NGLL> bg;
+      if constexpr (DIR < 2) {
+        bg.r = G.hyDensCells[hs + o];
+        bg.rt = G.hyDensThetaCells[hs + o];
+        bg.pt = G.prT[o];
+        bg.wall_bot = bg.wall_top = false;
+      } else {
+        sfor<NGLL>([&](auto ii) {
+          bg.rG[ii] = G.hyDensGLL[ac * NGLL + ii];
+          bg.rtG[ii] = G.hyDensThetaGLL[ac * NGLL + ii];
+          bg.pG[ii] = G.hyPressureGLL[ac * NGLL + ii];
+          bg.ptG[ii] = G.prG[ac * NGLL + ii];
+        });
+        bg.wall_bot = !per && ac == 0;
+        bg.wall_top = !per && ac == n - 1;
+      }
+      return bg;
+    };
+#if AWFL_PARITY & AWFL_PAR_ORDER
+    awfl::ref::cell_edges<ORD, NGLL, DIR>(st, load_bg(), G.weno_s, G.weno_w, K, eL, eR, src);
+#else
+    cell_edges_of<ORD, NGLL, DIR>(st, load_bg, G.weno_s, G.weno_w, K, eL, eR, src, [](const auto&, const auto&) {});
+#endif
+    sfor<5>([&](auto l) { s_e[e_slot(c, r) + l] = eR[l]; });
   }
   __syncthreads();
 
-  // periodic: face nx has the inputs of face 0 (S:819-820), so it is not recomputed
-  const int nfaces = per ? nx : nx + 1;
-  for (int f = threadIdx.x; f < nfaces; f += blockDim.x) {
-    int a, b;                 // qL from the right edge of cell a, qR from the left edge of cell b
-    bool aL = false, bR = false;
-    if (per) {
-      a = f == 0 ? nx - 1 : f - 1;
-      b = f == nx ? 0 : f;
-    } else if (f == 0) {      // wall: both sides from the first cell's left edge (S:822)
-      a = 0; b = 0; aL = true;
-    } else if (f == nx) {     // wall: both sides from the last cell's right edge (S:823)
-      a = nx - 1; b = nx - 1; bR = true;
+  // the flux of the low face, from the previous cell's right edge state (a
+  // line's first face: wrapped, or both sides from the cell at a wall), into
+  // that state's slot; the last cell of a walled line also takes its high face
+  auto face_ref = [&](int f) {
+    FaceRef fr;
+    if constexpr (DIR == 0) fr.rt = fr.q5 = G.prT[o];
+    else if constexpr (DIR == 1) {
+      fr.rt = G.prRT[o];
+      fr.q5 = G.prT[o];
     } else {
-      a = f - 1; b = f;
+      fr.rt = fr.q5 = G.prF[f];
     }
-    double qL[5], qR[5], F[5];
-#pragma unroll
-    for (int l = 0; l < 5; l++) {
-      qL[l] = aL ? s_L[l * nx + a] : s_R[l * nx + a];
-      qR[l] = bR ? s_R[l * nx + b] : s_L[l * nx + b];
+    return fr;
+  };
+  auto branch = [&](int f) -> unsigned char* {
+    if constexpr (BR == 0) return nullptr;
+    else if constexpr (DIR == 0) return K.br + ((int64_t)o * G.ny + line) * (G.nx + 1) + f;
+    else if constexpr (DIR == 1) return K.br + ((int64_t)o * (G.ny + 1) + f) * G.nx + line;
+    else return K.br + ((int64_t)f * G.ny + o) * G.nx + line;
+  };
+  auto face_p = [&](int f) {               // background pressure of a z face (S:1628-1629)
+    return f < n ? G.hyPressureGLL[f * NGLL] : G.hyPressureGLL[(n - 1) * NGLL + NGLL - 1];
+  };
+  double F[5];
+  if (act && a >= 0) {
+    const bool wall_lo = !per && a == 0;
+    const bool wrap = full && per && r == 0;
+    if (r > 0 || wrap || wall_lo) {
+      const int prev = e_slot(c, wrap ? nrow - 1 : r > 0 ? r - 1 : 0);
+      double qL[5];
+      sfor<5>([&](auto l) { qL[l] = wall_lo ? eL[l] : s_e[prev + l]; });
+      face_flux<DIR, BR>(qL, eL, face_ref(a), F, branch(a));
+      if constexpr (DIR == 2) {
+        // a periodic z line's face n is face 0 with the top's background pressure
+        const double raw = F[idW];
+        F[idW] = raw - face_p(a);
+        if (wrap) s_e[prev + idW] = raw - face_p(n);
+      }
+      if (!wall_lo)
+        sfor<5>([&](auto l) {
+          if (!(DIR == 2 && l == idW && wrap)) s_e[prev + l] = F[l];
+        });
     }
-    face_flux<0, BR>(qL, qR, fr, F, BR ? K.br + ((int64_t)k * G.ny + j) * (nx + 1) + f : nullptr);
-#pragma unroll
-    for (int l = 0; l < 5; l++) s_F[l * (nx + 1) + f] = F[l];
+    if (!per && a == n - 1) {
+      double Fn[5];
+      const FaceRef fr = face_ref(n);
+      if constexpr (BR == 0 && !(AWFL_PARITY & AWFL_PAR_ORDER)) wall_flux<DIR>(eR, fr, Fn);
+      else face_flux<DIR, BR>(eR, eR, fr, Fn, branch(n));
+      if constexpr (DIR == 2) Fn[idW] -= face_p(n);
+      sfor<5>([&](auto l) { s_e[e_slot(c, r) + l] = Fn[l]; });
+    }
   }
   __syncthreads();
 
-  for (int c = threadIdx.x; c < nx; c += blockDim.x) {
-#pragma unroll
-    for (int l = 0; l < 5; l++) {
-      const int cp = (per && c + 1 == nx) ? 0 : c + 1;
-      double td = flux_div(s_F[l * (nx + 1) + cp], s_F[l * (nx + 1) + c], K);
-      if (G.sim2d && l == idV) td = 0.0;
-      if constexpr (TEND) out[tend_index(G, l, k, j, c)] = td;
-      else if constexpr (INPLACE) out[l * G.sl + row + c] = s_st[l * W + hs + c] + K.dt * td;
-      else out[l * G.sl + row + c] = in[l * G.sl + row + c] + K.dt * td;
-    }
+  if (act && a >= s0 && a < s1) {
+    int64_t g;
+    if constexpr (!TEND) g = line_base(line) + a * sa;
+    else if constexpr (DIR == 0) g = tend_index(G, 0, o, line, a);
+    else if constexpr (DIR == 1) g = tend_index(G, 0, o, a, line);
+    else g = tend_index(G, 0, a, o, line);
+    const int64_t gl = TEND ? (int64_t)G.nz * G.ny * G.nx : G.sl;
+    sfor<5>([&](auto l) {
+      double td = flux_div(s_e[e_slot(c, r) + l], F[l], K);
+      if (DIR == 2 && l == idW) td = src + td;
+      if (DIR != 1 && G.sim2d && l == idV) td = 0.0;
+      out[g + l * gl] = TEND ? td : s_st[st_slot(c, r) + l] + K.dt * td;
+    });
   }
 }
 
 // ---------------------------------------------------------------------------
 // y / z sweeps: one lane per x-column walking a segment of its column
 // ---------------------------------------------------------------------------
-template <int ORD, int NGLL, int DIR, bool TEND, int BR = 0>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(AWFL_COL_WAVES))) void k_sweep_col(const double* __restrict__ in, double* __restrict__ out, Grid G,
+template <int ORD, int NGLL, int DIR, bool TEND>
+__global__ __launch_bounds__(64) void k_sweep_col(const double* __restrict__ in, double* __restrict__ out, Grid G,
                                                   SweepK K, int seglen) {
   constexpr int hs = (ORD - 1) / 2;
   constexpr int NM = 1 + DIR;
@@ -271,10 +374,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(AWFL_COL_WAV
     }
     return fr;
   };
-  auto branch = [&](int f) -> unsigned char* {
-    if constexpr (BR == 0) return nullptr;
-    return K.br + (DIR == 1 ? ((int64_t)o * (G.ny + 1) + f) * G.nx + i : ((int64_t)f * G.ny + o) * G.nx + i);
-  };
   auto face_bg = [&](int f, double (&F)[5]) {   // S:1628-1629
     if constexpr (DIR == 2) {
       if (f < G.nz) F[idW] -= G.hyPressureGLL[f * NGLL + 0];
@@ -311,7 +410,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(AWFL_COL_WAV
     CellBg<NGLL> bg;
     bg_of(((s0 - 1) % n + n) % n, bg);
     double eL[5], sa_;
-    cellns::cell_edges<ORD, NGLL, DIR>(w, bg, G.weno_s, G.weno_w, K, eL, prevR, sa_);
+    AWFL_CELL::cell_edges<ORD, NGLL, DIR>(w, bg, G.weno_s, G.weno_w, K, eL, prevR, sa_);
   }
   // software pipeline: the stencil cell of the next iteration is loaded one
   // iteration ahead, and the result of an iteration is stored at the top of
@@ -332,11 +431,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(AWFL_COL_WAV
     CellBg<NGLL> bg;
     bg_of(v, bg);
     double eL[5], eR[5], src;
-    cellns::cell_edges<ORD, NGLL, DIR>(w, bg, G.weno_s, G.weno_w, K, eL, eR, src);
+    AWFL_CELL::cell_edges<ORD, NGLL, DIR>(w, bg, G.weno_s, G.weno_w, K, eL, eR, src);
     double F[5];
     FaceRef fr = face_ref(v);
     if (!per && v == 0) sfor<5>([&](auto l) { prevR[l] = eL[l]; });   // wall: both sides from the first cell
-    face_flux<DIR, BR>(prevR, eL, fr, F, branch(v));
+    face_flux<DIR, 0>(prevR, eL, fr, F, nullptr);
     face_bg(v, F);
     update(prevF, F, prevSrc, hs - 1, res);   // cell v-1 (for v == s0 a value never stored)
 #pragma unroll
@@ -355,13 +454,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(AWFL_COL_WAV
     w[l][ORD - 1] = nxt[l];            // cell s1 + hs, loaded by the last iteration
   });
   if (!per && s1 == n) {
-    face_flux<DIR, BR>(prevR, prevR, fr, F, branch(s1));   // wall: both sides from the last cell
+    face_flux<DIR, 0>(prevR, prevR, fr, F, nullptr);   // wall: both sides from the last cell
   } else {
     CellBg<NGLL> bg;
     bg_of(s1 % n, bg);
     double eL[5], eR[5], sa_;
-    cellns::cell_edges<ORD, NGLL, DIR>(w, bg, G.weno_s, G.weno_w, K, eL, eR, sa_);
-    face_flux<DIR, BR>(prevR, eL, fr, F, branch(s1));
+    AWFL_CELL::cell_edges<ORD, NGLL, DIR>(w, bg, G.weno_s, G.weno_w, K, eL, eR, sa_);
+    face_flux<DIR, 0>(prevR, eL, fr, F, nullptr);
   }
   face_bg(s1, F);
   update(prevF, F, prevSrc, hs - 1, res);
@@ -596,55 +695,58 @@ __global__ void k_init(double* __restrict__ st, Grid G, InitDev S) {
 // ---------------------------------------------------------------------------
 // compiled (ord, ngll) variants
 // ---------------------------------------------------------------------------
-// the in-place x kernel of awfl_time_step_noalloc: the per-cell x kernel, or
-// for (9, 5) the x line kernel
-template <int O, int N>
-constexpr void (*inplace_x())(const double*, double*, Grid, SweepK) {
-  if constexpr (O == 9) return awfl_line::k_sweep_line<O, N, 0, false, true>;
-  else return k_sweep_x<O, N, false, 0, true>;
-}
-
 // the lane-split line sweeps (awfl_sweep_line.hpp), used for (9, 5), whose
-// per-cell kernels need more registers than a lane has
+// cell takes more registers than a lane has; [dir][tend], and the in-place x
+// kernel of awfl_time_step_noalloc
 using LineFn = void (*)(const double*, double*, Grid, SweepK);
-template <int O, int N, int D, bool T>
-constexpr LineFn line_fn() {
-  if constexpr (O == 9) return awfl_line::k_sweep_line<O, N, D, T>;
-  else return nullptr;
-}
+// the tile kernels: x, then y and z with 4, 8 and 16 lines a tile
+using TileFn = void (*)(const double*, double*, Grid, SweepK, TilePlan);
+constexpr int TILE_TX[3] = {4, 8, 16};
+struct TileFns {
+  TileFn x, yz[2][3];
+};
+
+using ColFn = void (*)(const double*, double*, Grid, SweepK, int);
 
 struct Variant {
   int ord, ngll;
-  void (*sweep_x[2])(const double*, double*, Grid, SweepK);
-  void (*sweep_x_inplace)(const double*, double*, Grid, SweepK);
-  void (*sweep_y[2])(const double*, double*, Grid, SweepK, int);
-  void (*sweep_z[2])(const double*, double*, Grid, SweepK, int);
+  TileFns tile[2];                     // [tend]; null at (9, 5)
+  ColFn col[2][2];                     // [y, z][tend]
   void (*init)(double*, Grid, InitDev);
-  LineFn sweep_line[3][2];             // [dir][tend]; null: the per-cell kernels above
+  LineFn sweep_line[3][2];             // null: the tile kernels
+  LineFn line_x_inplace;
 };
 
-// per-cell sweep kernels, for the orders that do not use the line kernels
-template <int O, int N, bool T>
-constexpr void (*cell_x())(const double*, double*, Grid, SweepK) {
-  if constexpr (O == 9) return nullptr;
-  else return k_sweep_x<O, N, T>;
+template <int O, int N, bool T, int BR = 0>
+constexpr TileFns tile_fns() {
+  if constexpr (O == 9) return TileFns{};
+  else
+    return TileFns{k_sweep_tile<O, N, 0, 1, T, BR>,
+                   {{k_sweep_tile<O, N, 1, 4, T, BR>, k_sweep_tile<O, N, 1, 8, T, BR>, k_sweep_tile<O, N, 1, 16, T, BR>},
+                    {k_sweep_tile<O, N, 2, 4, T, BR>, k_sweep_tile<O, N, 2, 8, T, BR>, k_sweep_tile<O, N, 2, 16, T, BR>}}};
 }
+template <int O, int N, int D, bool T, bool INPLACE = false>
+constexpr LineFn line_fn() {
+  if constexpr (O == 9) return awfl_line::k_sweep_line<O, N, D, T, INPLACE>;
+  else return nullptr;
+}
+
 template <int O, int N, int D, bool T>
-constexpr void (*cell_col())(const double*, double*, Grid, SweepK, int) {
+constexpr ColFn col_fn() {
   if constexpr (O == 9) return nullptr;
   else return k_sweep_col<O, N, D, T>;
 }
 
-#define AWFL_VARIANT(O, N)                                                                        \
-  Variant{O, N,                                                                                   \
-          {cell_x<O, N, false>(), cell_x<O, N, true>()},                                          \
-          inplace_x<O, N>(),                                                                      \
-          {cell_col<O, N, 1, false>(), cell_col<O, N, 1, true>()},                                \
-          {cell_col<O, N, 2, false>(), cell_col<O, N, 2, true>()},                                \
-          k_init<O>,                                                                              \
-          {{line_fn<O, N, 0, false>(), line_fn<O, N, 0, true>()},                                 \
-           {line_fn<O, N, 1, false>(), line_fn<O, N, 1, true>()},                                 \
-           {line_fn<O, N, 2, false>(), line_fn<O, N, 2, true>()}}}
+#define AWFL_VARIANT(O, N)                                          \
+  Variant{O, N,                                                     \
+          {tile_fns<O, N, false>(), tile_fns<O, N, true>()},        \
+          {{col_fn<O, N, 1, false>(), col_fn<O, N, 1, true>()},     \
+           {col_fn<O, N, 2, false>(), col_fn<O, N, 2, true>()}},    \
+          k_init<O>,                                                \
+          {{line_fn<O, N, 0, false>(), line_fn<O, N, 0, true>()},   \
+           {line_fn<O, N, 1, false>(), line_fn<O, N, 1, true>()},   \
+           {line_fn<O, N, 2, false>(), line_fn<O, N, 2, true>()}},  \
+          line_fn<O, N, 0, false, true>()}
 
 #ifdef AWFL_LEAN
 // parity builds: the FP64 (5, 3) sweeps only, no FP32 form in the library
@@ -1001,39 +1103,68 @@ int awfl_state_sums(awfl_ctx* c, const double* d_state, double* h_out) {
 }  // extern "C"
 
 
-using SweepXFn = void (*)(const double*, double*, Grid, SweepK);
-using SweepColFn = void (*)(const double*, double*, Grid, SweepK, int);
-
-// launch one sweep with the given kernels (x: kx; y, z: kcol)
-// (x_flux_lds: the in-place x kernel keeps its face fluxes apart from the line)
-static int launch_sweep_with(awfl_ctx* c, const double* in, double* out, const SweepK& K, int dir, SweepXFn kx,
-                             SweepColFn kcol, bool x_flux_lds = false) {
-  Grid G = c->grid();
+// Cut of a sweep of n-cell lines, nline of them side by side (x: along y; y
+// and z: along x): TX index for y and z (-1: x) and the plan.  The cut with
+// the fewest waves (idle lanes and twice-reconstructed cells both cost waves)
+// among whole lines and segments in work-groups of at most 512 lanes, x lines
+// whole up to 1024 cells.
+struct TileCut {
+  int tx;
+  TilePlan p;
+  int threads;
+};
+static TileCut tile_plan(int dir, int n, int nline, bool per) {
+  TileCut best{};
+  int64_t best_cost = INT64_MAX;
+  auto consider = [&](int tx, int cols, int nseg, int limit) {
+    const int seglen = (n + nseg - 1) / nseg;
+    if ((n + seglen - 1) / seglen != nseg) return;
+    // rows of the longest segment with the cells at its ends that it needs
+    const int rows = nseg == 1 ? n : !per && nseg == 2 ? seglen + 1 : seglen + 2;
+    const int64_t lanes = (int64_t)rows * cols;
+    if (lanes > limit) return;
+    const int64_t waves = (lanes + 63) / 64;
+    const int64_t cost = waves * nseg * ((nline + cols - 1) / cols);
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = TileCut{tx, TilePlan{cols, rows, nseg, seglen}, (int)waves * 64};
+    }
+  };
   if (dir == 0) {
-    int nx = c->cfg.nx;
-    int threads = line_threads(nx);
-    size_t lds = sizeof(double) * (size_t)(5 * (nx + 2 * c->hs) + 10 * nx + (x_flux_lds ? 5 * (nx + 1) : 0));
-    if (lds > 64 * 1024)
-      HIP_TRY(c, hipFuncSetAttribute((const void*)kx, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    kx<<<c->cfg.ny * c->cfg.nz, threads, lds, c->stream>>>(in, out, G, K);
-    LAUNCH_CHECK(c);
-    return AWFL_OK;
+    for (int cols = 1; cols <= std::max(1, std::min(nline, 512 / n)); cols++) consider(-1, cols, 1, TILE_THREADS);
+    for (int nseg = 2; best_cost == INT64_MAX; nseg++) consider(-1, 1, nseg, TILE_THREADS);
+  } else {
+    const int max_seg = (n + 13) / 14;                 // segments of at least 14 cells
+    for (int x = 0; x < 3; x++)
+      for (int nseg = 1; nseg <= max_seg; nseg++) consider(x, TILE_TX[x], nseg, 512);
   }
-  int n = dir == 1 ? c->cfg.ny : c->cfg.nz;
-  int other = dir == 1 ? c->cfg.nz : c->cfg.ny;
-  int bx = (c->cfg.nx + 63) / 64;
-  // segments of at most 32 cells, and shorter (down to 16 cells) where that
-  // is needed for ~4 waves per SIMD (256 CUs x 4 SIMDs).  Longer segments on
-  // large grids (256 cells at 512x512x256) measured 4-7% slower.
-  int64_t layer = (int64_t)bx * other;
-  int nseg = (int)std::max<int64_t>(1, std::min<int64_t>(std::max<int64_t>((4096 + layer - 1) / layer, (n + 31) / 32),
-                                                           std::max(1, n / 16)));
-  int seglen = (n + nseg - 1) / nseg;
-  nseg = (n + seglen - 1) / seglen;
-  dim3 grid(bx, other, nseg);
-  kcol<<<grid, 64, 0, c->stream>>>(in, out, G, K, seglen);
+  return best;
+}
+
+// launch one tile sweep with the given kernels
+static int launch_tile(awfl_ctx* c, const double* in, double* out, const SweepK& K, int dir, const TileFns& f) {
+  const int n = dir == 0 ? c->cfg.nx : dir == 1 ? c->cfg.ny : c->cfg.nz;
+  const int nline = dir == 0 ? c->cfg.ny : c->cfg.nx;
+  const int bc = dir == 0 ? c->cfg.bc_x : dir == 1 ? c->cfg.bc_y : c->cfg.bc_z;
+  const TileCut cut = tile_plan(dir, n, nline, bc == AWFL_BC_PERIODIC);
+  const TileFn k = dir == 0 ? f.x : f.yz[dir - 1][cut.tx];
+  const size_t lds = sizeof(double) * 5 * cut.p.cols * (size_t)(2 * cut.p.rows + 2 * c->hs);
+  if (lds > 64 * 1024)
+    HIP_TRY(c, hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  const dim3 grid((nline + cut.p.cols - 1) / cut.p.cols, dir == 2 ? c->cfg.ny : c->cfg.nz, cut.p.nseg);
+  k<<<grid, cut.threads, lds, c->stream>>>(in, out, c->grid(), K, cut.p);
   LAUNCH_CHECK(c);
   return AWFL_OK;
+}
+
+// Whether a y or z sweep runs the column walker: with 4 million cells or more
+// its waves fill the chip, and it reads whole 512-byte rows and reconstructs
+// 6% of the cells twice where a tile is cut into segments with more (256x256x128:
+// y 324 against 362, z 337 against 391 us; 192x192x96: 158 against 147, 167 against
+// 192; 128x128x64: 58 against 43, 62 against 44; 96x300x200: 318 against 262, 362
+// against 318)
+static bool walks(const awfl_ctx* c, int dir) {
+  return (int64_t)c->cfg.nx * c->cfg.ny * c->cfg.nz >= 4000000;
 }
 
 // one lane-split line sweep: a work-group of awfl_line::LS_THREADS per line
@@ -1050,13 +1181,29 @@ static int launch_line(awfl_ctx* c, const double* in, double* out, const SweepK&
   return AWFL_OK;
 }
 
+// launch one column-walker sweep (y or z): segments of at most 32 cells, and
+// shorter (down to 16 cells) where that is needed for ~4 waves per SIMD
+static int launch_col(awfl_ctx* c, const double* in, double* out, const SweepK& K, int dir, ColFn k) {
+  const int n = dir == 1 ? c->cfg.ny : c->cfg.nz;
+  const int other = dir == 1 ? c->cfg.nz : c->cfg.ny;
+  const int bx = (c->cfg.nx + 63) / 64;
+  const int64_t layer = (int64_t)bx * other;
+  int nseg = (int)std::max<int64_t>(1, std::min<int64_t>(std::max<int64_t>((4096 + layer - 1) / layer, (n + 31) / 32),
+                                                         std::max(1, n / 16)));
+  const int seglen = (n + nseg - 1) / nseg;
+  nseg = (n + seglen - 1) / seglen;
+  k<<<dim3(bx, other, nseg), 64, 0, c->stream>>>(in, out, c->grid(), K, seglen);
+  LAUNCH_CHECK(c);
+  return AWFL_OK;
+}
+
 // launch one sweep; tend selects the tendency output (layout [5][nz][ny][nx])
 static int launch_sweep(awfl_ctx* c, const double* in, double* out, double dt, int dir, bool tend) {
   const Variant* v = static_cast<const Variant*>(c->var);
   if (v->sweep_line[dir][0])
     return launch_line(c, in, out, sweep_constants(c, dt, dir), dir, v->sweep_line[dir][tend ? 1 : 0]);
-  return launch_sweep_with(c, in, out, sweep_constants(c, dt, dir), dir, v->sweep_x[tend ? 1 : 0],
-                           dir == 1 ? v->sweep_y[tend ? 1 : 0] : v->sweep_z[tend ? 1 : 0]);
+  if (dir > 0 && walks(c, dir)) return launch_col(c, in, out, sweep_constants(c, dt, dir), dir, v->col[dir - 1][tend ? 1 : 0]);
+  return launch_tile(c, in, out, sweep_constants(c, dt, dir), dir, v->tile[tend ? 1 : 0]);
 }
 
 static int fill(awfl_ctx* c, double* p, int64_t n, double v) {
@@ -1136,10 +1283,8 @@ int awfl_time_step_branches(awfl_ctx* c, double* d_state, double dt, unsigned ch
     double* dst = (s == nd - 1) ? d_state : (cur == c->d_buf[0] ? c->d_buf[1] : c->d_buf[0]);
     SweepK K = sweep_constants(c, dt, dirs[s]);
     K.br = d_branch + per_split * slot[s];
-    int rc = mode == 1 ? launch_sweep_with(c, cur, dst, K, dirs[s], k_sweep_x<5, 3, false, 1>,
-                                           dirs[s] == 1 ? k_sweep_col<5, 3, 1, false, 1> : k_sweep_col<5, 3, 2, false, 1>)
-                       : launch_sweep_with(c, cur, dst, K, dirs[s], k_sweep_x<5, 3, false, 2>,
-                                           dirs[s] == 1 ? k_sweep_col<5, 3, 1, false, 2> : k_sweep_col<5, 3, 2, false, 2>);
+    static const TileFns record = tile_fns<5, 3, false, 1>(), replay = tile_fns<5, 3, false, 2>();
+    int rc = launch_tile(c, cur, dst, K, dirs[s], mode == 1 ? record : replay);
     if (rc != AWFL_OK) return rc;
     cur = dst;
   }
@@ -1194,12 +1339,11 @@ int awfl_time_step_noalloc(awfl_ctx* c, double* d_state, double dt) {
     SweepK K = sweep_constants(c, dt, d);
     int rc;
     if (v->sweep_line[d][0])          // (9, 5): line kernels
-      rc = (d == 0 && src == dst) ? launch_line(c, src, dst, K, 0, v->sweep_x_inplace, true)
+      rc = (d == 0 && src == dst) ? launch_line(c, src, dst, K, 0, v->line_x_inplace, true)
                                   : launch_line(c, src, dst, K, d, v->sweep_line[d][0]);
     else
-      rc = (d == 0 && src == dst)
-               ? launch_sweep_with(c, src, dst, K, 0, v->sweep_x_inplace, nullptr, true)
-               : launch_sweep_with(c, src, dst, K, d, v->sweep_x[0], d == 1 ? v->sweep_y[0] : v->sweep_z[0]);
+      rc = d > 0 && walks(c, d) ? launch_col(c, src, dst, K, d, v->col[d - 1][0])
+                                : launch_tile(c, src, dst, K, d, v->tile[0]);   // (x lines are whole up to the limit above: in place)
     if (rc != AWFL_OK) return rc;
   }
   c->dimSwitch = !c->dimSwitch;
