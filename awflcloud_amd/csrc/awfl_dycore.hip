@@ -32,6 +32,7 @@
 #include "awfl_cell_ref.hpp"
 #endif
 #include "awfl_sweep_line.hpp"
+#include "awfl_tile.hpp"
 
 // Cell body of the sweeps: the production numerics, or (reference-order parity
 // builds) the reference's operation order.
@@ -86,224 +87,101 @@ __device__ __forceinline__ void face_flux(const double (&qL)[5], const double (&
   }
 }
 
-// How a sweep's grid is cut into work-groups (tile_plan).  A work-group holds
-// `cols` lines and of each the rows lo .. lo + rows - 1 along the sweep: the
-// whole line (nseg == 1), or a segment of seglen cells with the neighbouring
-// cell at either end, whose edge state the segment's end faces need and which
-// is reconstructed twice.
-struct TilePlan {
-  int cols, rows, nseg, seglen;
-};
+// The FP64 sweep's numerics for the tile sweep (awfl_tile.hpp)
+template <int ORD_, int NGLL, int DIR_, int TX_, bool TEND, int BR>
+struct Sweep64 {
+  using real = double;
+  static constexpr int ORD = ORD_, DIR = DIR_, TX = TX_;
+  static constexpr int hs = (ORD - 1) / 2;
+  const double* src;
+  double* out;
+  const Grid& g;
+  const SweepK& K;
+  __device__ const Grid& G() const { return g; }
+  __device__ const double* in() const { return src; }
 
-// One lane per cell.  The tile's cells and hs cells beyond either end go
-// through LDS (periodic wrap or wall clamp applied at the load, so there is no
-// halo pass); a lane reconstructs its cell and hands its right edge state to
-// the lane of the next cell through LDS, forms the flux of its low face and
-// hands that back to the previous cell in the same place (the only lane that
-// reads a slot before it is overwritten is the one that overwrites it), and
-// updates its cell.  Every global read happens before the first barrier, so
-// whole lines may be updated in place.
-//
-// What bounds it: FP64 issue (and the clock the FP64 load leaves).  One cell
-// per lane takes 96-106 registers, four or five waves per SIMD, and gives
-// small grids as many waves as they have cells; the column walker
-// (k_sweep_col) needs 203-245 registers, two waves per SIMD, and at 64x64x32
-// fills an eighth of the chip.  LDS holds a cell's 5 values contiguously (40
-// bytes): every stencil address is one base plus a constant, and 32 lanes 10
-// dwords apart touch 64 distinct banks.  Measured against the walkers (y, z)
-// and the former line kernel (x), whose edge states all went through LDS: a
-// step at 64x64x32 123 -> 30 us, a 301x1x75 slice 74 -> 16 us, 128x128x64
-// 190 -> 134 us; x at 256x256x128 346 -> 310 us.
-//
-// TX: lines of a y or z tile, neighbours in x (the lanes of a load run along
-// x); an x tile's lines are neighbours in y.
-constexpr int TILE_THREADS = 1024;
-template <int ORD, int NGLL, int DIR, int TX, bool TEND, int BR = 0>
-__global__ __launch_bounds__(TILE_THREADS) void k_sweep_tile(const double* in, double* out, Grid G, SweepK K,
-                                                             TilePlan T) {
-  constexpr int hs = (ORD - 1) / 2;
-  constexpr int NM = 1 + DIR;
-  extern __shared__ double sm[];
-  const int n = DIR == 0 ? G.nx : DIR == 1 ? G.ny : G.nz;
-  const int cols = DIR == 0 ? T.cols : TX;
-  const int rows = T.rows;
-  const bool per = G.bc[DIR] == AWFL_BC_PERIODIC;
-  const bool full = T.nseg == 1;
-  // tile -> lines (line index along x or, for x tiles, y; o: the other axis), segment
-  const dim3 tb = tile_coords();
-  const int o = tb.y;                      // x, y tiles: level k; z tiles: j
-  const int s0 = tb.z * T.seglen, s1 = min(n, s0 + T.seglen);
-  const int lo = full || (!per && s0 == 0) ? s0 : s0 - 1;
-  const int nrow = (full || (!per && s1 == n) ? s1 : s1 + 1) - lo;
-  // lane -> column c, row r (cell a of the line)
-  const int t = threadIdx.x;
-  int c, r;
-  if constexpr (DIR == 0) {
-    c = cols == 1 ? 0 : t / rows;
-    r = t - c * rows;
-  } else {
-    c = t % TX;
-    r = t / TX;
-  }
-  const int line = tb.x * cols + c;
-  const int nline = DIR == 0 ? G.ny : G.nx;
-  const bool act = c < cols && r < nrow && line < nline;
-  const int a = lo + r;
-  const int64_t sa = DIR == 0 ? 1 : DIR == 1 ? G.sy : G.sz;
-  auto line_base = [&](int l) -> int64_t {
-    if constexpr (DIR == 0) return (int64_t)(hs + o) * G.sz + (int64_t)(hs + l) * G.sy + hs;
-    else if constexpr (DIR == 1) return (int64_t)(hs + o) * G.sz + (int64_t)hs * G.sy + hs + l;
-    else return (int64_t)hs * G.sz + (int64_t)(hs + o) * G.sy + hs + l;
-  };
-  // LDS slot of row p of column c: staged cells (p from -hs) and edges
-  auto st_slot = [&](int cc, int p) { return 5 * (DIR == 0 ? cc * (rows + 2 * hs) + p + hs : (p + hs) * TX + cc); };
-  auto e_slot = [&](int cc, int p) { return 5 * (DIR == 0 ? cc * rows + p : p * TX + cc); };
-  double* s_st = sm;                                   // [cols][rows + 2hs][5]
-  double* s_e = sm + 5 * cols * (rows + 2 * hs);       // [cols][rows][5]: right edge states, then fluxes
-
-  // stage: a cell of the line or one beyond its ends (S:631-662, 994-1025, 1351-1382)
-  auto source = [&](int v, bool& zn) {
-    zn = false;
-    if (v >= 0 && v < n) return v;
-    if (per) {
-      if (n > hs + 1) return v < 0 ? v + n : v - n;    // a tile reaches at most hs + 1 cells past the line
-      const int m = v % n;
-      return m < 0 ? m + n : m;
-    }
-    zn = true;
-    return v < 0 ? 0 : n - 1;
-  };
-  double own[5];
-  if (act) {
-    bool zn;
-    const int64_t g = line_base(line) + source(a, zn) * sa;
-    sfor<5>([&](auto l) { own[l] = in[l * G.sl + g]; });
-  }
-  for (int h = t; h < 2 * hs * cols; h += blockDim.x) {
-    int hc, hp;                                        // column, and which of the 2 hs cells beyond the tile
-    if constexpr (DIR == 0) {
-      hc = h / (2 * hs);
-      hp = h % (2 * hs);
-    } else {
-      hc = h % TX;
-      hp = h / TX;
-    }
-    if ((int)tb.x * cols + hc < nline) {
-      const int p = hp < hs ? hp - hs : nrow + hp - hs;
-      bool zn;
-      const int64_t g = line_base(tb.x * cols + hc) + source(lo + p, zn) * sa;
-      double v[5];
-      sfor<5>([&](auto l) { v[l] = in[l * G.sl + g]; });
-      if (zn) v[NM] = 0.0;
-      sfor<5>([&](auto l) { s_st[st_slot(hc, p) + l] = v[l]; });
-    }
-  }
-  if (act) sfor<5>([&](auto l) { s_st[st_slot(c, r) + l] = own[l]; });
-  __syncthreads();
-
-  double eL[5], eR[5], src = 0.0;
-  const int ac = a < 0 ? a + n : a >= n ? a - n : a;   // the cell itself (a line's end wraps)
-  if (act) {
-    double st[5][ORD];
-    const double* w = s_st + st_slot(c, r - hs);
-    constexpr int step = DIR == 0 ? 5 : 5 * TX;
-    sfor<5>([&](auto l) { sfor<ORD>([&](auto s) { st[l][s] = w[s * step + l]; }); });
+  __device__ __forceinline__ void cell(int o, int a, const double (&st)[5][ORD], double (&eL)[5], double (&eR)[5],
+                                       double& sa) const {
     auto load_bg = [&]() {
       CellBg<NGLL> bg;
       if constexpr (DIR < 2) {
-        bg.r = G.hyDensCells[hs + o];
-        bg.rt = G.hyDensThetaCells[hs + o];
-        bg.pt = G.prT[o];
+        bg.r = g.hyDensCells[hs + o];
+        bg.rt = g.hyDensThetaCells[hs + o];
+        bg.pt = g.prT[o];
         bg.wall_bot = bg.wall_top = false;
       } else {
         sfor<NGLL>([&](auto ii) {
-          bg.rG[ii] = G.hyDensGLL[ac * NGLL + ii];
-          bg.rtG[ii] = G.hyDensThetaGLL[ac * NGLL + ii];
-          bg.pG[ii] = G.hyPressureGLL[ac * NGLL + ii];
-          bg.ptG[ii] = G.prG[ac * NGLL + ii];
+          bg.rG[ii] = g.hyDensGLL[a * NGLL + ii];
+          bg.rtG[ii] = g.hyDensThetaGLL[a * NGLL + ii];
+          bg.pG[ii] = g.hyPressureGLL[a * NGLL + ii];
+          bg.ptG[ii] = g.prG[a * NGLL + ii];
         });
-        bg.wall_bot = !per && ac == 0;
-        bg.wall_top = !per && ac == n - 1;
+        const bool per = g.bc[2] == AWFL_BC_PERIODIC;
+        bg.wall_bot = !per && a == 0;
+        bg.wall_top = !per && a == g.nz - 1;
       }
       return bg;
     };
 #if AWFL_PARITY & AWFL_PAR_ORDER
-    awfl::ref::cell_edges<ORD, NGLL, DIR>(st, load_bg(), G.weno_s, G.weno_w, K, eL, eR, src);
+    awfl::ref::cell_edges<ORD, NGLL, DIR>(st, load_bg(), g.weno_s, g.weno_w, K, eL, eR, sa);
 #else
-    cell_edges_of<ORD, NGLL, DIR>(st, load_bg, G.weno_s, G.weno_w, K, eL, eR, src, [](const auto&, const auto&) {});
+    cell_edges_of<ORD, NGLL, DIR>(st, load_bg, g.weno_s, g.weno_w, K, eL, eR, sa, [](const auto&, const auto&) {});
 #endif
-    sfor<5>([&](auto l) { s_e[e_slot(c, r) + l] = eR[l]; });
   }
-  __syncthreads();
-
-  // the flux of the low face, from the previous cell's right edge state (a
-  // line's first face: wrapped, or both sides from the cell at a wall), into
-  // that state's slot; the last cell of a walled line also takes its high face
-  auto face_ref = [&](int f) {
+  __device__ __forceinline__ FaceRef face_ref(int o, int f) const {
     FaceRef fr;
-    if constexpr (DIR == 0) fr.rt = fr.q5 = G.prT[o];
+    if constexpr (DIR == 0) fr.rt = fr.q5 = g.prT[o];
     else if constexpr (DIR == 1) {
-      fr.rt = G.prRT[o];
-      fr.q5 = G.prT[o];
+      fr.rt = g.prRT[o];
+      fr.q5 = g.prT[o];
     } else {
-      fr.rt = fr.q5 = G.prF[f];
+      fr.rt = fr.q5 = g.prF[f];
     }
     return fr;
-  };
-  auto branch = [&](int f) -> unsigned char* {
-    if constexpr (BR == 0) return nullptr;
-    else if constexpr (DIR == 0) return K.br + ((int64_t)o * G.ny + line) * (G.nx + 1) + f;
-    else if constexpr (DIR == 1) return K.br + ((int64_t)o * (G.ny + 1) + f) * G.nx + line;
-    else return K.br + ((int64_t)f * G.ny + o) * G.nx + line;
-  };
-  auto face_p = [&](int f) {               // background pressure of a z face (S:1628-1629)
-    return f < n ? G.hyPressureGLL[f * NGLL] : G.hyPressureGLL[(n - 1) * NGLL + NGLL - 1];
-  };
-  double F[5];
-  if (act && a >= 0) {
-    const bool wall_lo = !per && a == 0;
-    const bool wrap = full && per && r == 0;
-    if (r > 0 || wrap || wall_lo) {
-      const int prev = e_slot(c, wrap ? nrow - 1 : r > 0 ? r - 1 : 0);
-      double qL[5];
-      sfor<5>([&](auto l) { qL[l] = wall_lo ? eL[l] : s_e[prev + l]; });
-      face_flux<DIR, BR>(qL, eL, face_ref(a), F, branch(a));
-      if constexpr (DIR == 2) {
-        // a periodic z line's face n is face 0 with the top's background pressure
-        const double raw = F[idW];
-        F[idW] = raw - face_p(a);
-        if (wrap) s_e[prev + idW] = raw - face_p(n);
-      }
-      if (!wall_lo)
-        sfor<5>([&](auto l) {
-          if (!(DIR == 2 && l == idW && wrap)) s_e[prev + l] = F[l];
-        });
-    }
-    if (!per && a == n - 1) {
-      double Fn[5];
-      const FaceRef fr = face_ref(n);
-      if constexpr (BR == 0 && !(AWFL_PARITY & AWFL_PAR_ORDER)) wall_flux<DIR>(eR, fr, Fn);
-      else face_flux<DIR, BR>(eR, eR, fr, Fn, branch(n));
-      if constexpr (DIR == 2) Fn[idW] -= face_p(n);
-      sfor<5>([&](auto l) { s_e[e_slot(c, r) + l] = Fn[l]; });
-    }
   }
-  __syncthreads();
-
-  if (act && a >= s0 && a < s1) {
-    int64_t g;
-    if constexpr (!TEND) g = line_base(line) + a * sa;
-    else if constexpr (DIR == 0) g = tend_index(G, 0, o, line, a);
-    else if constexpr (DIR == 1) g = tend_index(G, 0, o, a, line);
-    else g = tend_index(G, 0, a, o, line);
-    const int64_t gl = TEND ? (int64_t)G.nz * G.ny * G.nx : G.sl;
+  __device__ unsigned char* branch(int o, int line, int f) const {
+    if constexpr (BR == 0) return nullptr;
+    else if constexpr (DIR == 0) return K.br + ((int64_t)o * g.ny + line) * (g.nx + 1) + f;
+    else if constexpr (DIR == 1) return K.br + ((int64_t)o * (g.ny + 1) + f) * g.nx + line;
+    else return K.br + ((int64_t)f * g.ny + o) * g.nx + line;
+  }
+  // background pressure of a z face (S:1628-1629)
+  __device__ __forceinline__ void subtract_p(int f, double (&F)[5]) const {
+    if constexpr (DIR == 2)
+      F[idW] -= f < g.nz ? g.hyPressureGLL[f * NGLL] : g.hyPressureGLL[(g.nz - 1) * NGLL + NGLL - 1];
+  }
+  __device__ __forceinline__ void face(int o, int line, int f, const double (&qL)[5], const double (&qR)[5],
+                                       double (&F)[5]) const {
+    face_flux<DIR, BR>(qL, qR, face_ref(o, f), F, branch(o, line, f));
+    subtract_p(f, F);
+  }
+  __device__ __forceinline__ void wall(int o, int line, int f, const double (&q)[5], double (&F)[5]) const {
+    if constexpr (BR == 0 && !(AWFL_PARITY & AWFL_PAR_ORDER)) wall_flux<DIR>(q, face_ref(o, f), F);
+    else face_flux<DIR, BR>(q, q, face_ref(o, f), F, branch(o, line, f));
+    subtract_p(f, F);
+  }
+  __device__ __forceinline__ void put(int o, int line, int a, int64_t at, const double (&cell)[5],
+                                      const double (&F0)[5], const double (&F1)[5], double sa) const {
+    int64_t i = at, step = g.sl;
+    if constexpr (TEND) {
+      step = (int64_t)g.nz * g.ny * g.nx;
+      if constexpr (DIR == 0) i = tend_index(g, 0, o, line, a);
+      else if constexpr (DIR == 1) i = tend_index(g, 0, o, a, line);
+      else i = tend_index(g, 0, a, o, line);
+    }
     sfor<5>([&](auto l) {
-      double td = flux_div(s_e[e_slot(c, r) + l], F[l], K);
-      if (DIR == 2 && l == idW) td = src + td;
-      if (DIR != 1 && G.sim2d && l == idV) td = 0.0;
-      out[g + l * gl] = TEND ? td : s_st[st_slot(c, r) + l] + K.dt * td;
+      double td = flux_div(F1[l], F0[l], K);
+      if (DIR == 2 && l == idW) td = sa + td;
+      if (DIR != 1 && g.sim2d && l == idV) td = 0.0;
+      out[i + l * step] = TEND ? td : cell[l] + K.dt * td;
     });
   }
+};
+
+template <int ORD, int NGLL, int DIR, int TX, bool TEND, int BR = 0>
+__global__ __launch_bounds__(awfl_tile::MAX_THREADS) void k_sweep_tile(const double* in, double* out, Grid G,
+                                                                       SweepK K, awfl_tile::TilePlan T) {
+  awfl_tile::sweep(Sweep64<ORD, NGLL, DIR, TX, TEND, BR>{in, out, G, K}, T);
 }
 
 // ---------------------------------------------------------------------------
@@ -700,8 +578,7 @@ __global__ void k_init(double* __restrict__ st, Grid G, InitDev S) {
 // kernel of awfl_time_step_noalloc
 using LineFn = void (*)(const double*, double*, Grid, SweepK);
 // the tile kernels: x, then y and z with 4, 8 and 16 lines a tile
-using TileFn = void (*)(const double*, double*, Grid, SweepK, TilePlan);
-constexpr int TILE_TX[3] = {4, 8, 16};
+using TileFn = void (*)(const double*, double*, Grid, SweepK, awfl_tile::TilePlan);
 struct TileFns {
   TileFn x, yz[2][3];
 };
@@ -1103,68 +980,55 @@ int awfl_state_sums(awfl_ctx* c, const double* d_state, double* h_out) {
 }  // extern "C"
 
 
-// Cut of a sweep of n-cell lines, nline of them side by side (x: along y; y
-// and z: along x): TX index for y and z (-1: x) and the plan.  The cut with
-// the fewest waves (idle lanes and twice-reconstructed cells both cost waves)
-// among whole lines and segments in work-groups of at most 512 lanes, x lines
-// whole up to 1024 cells.
-struct TileCut {
-  int tx;
-  TilePlan p;
-  int threads;
-};
-static TileCut tile_plan(int dir, int n, int nline, bool per) {
-  TileCut best{};
-  int64_t best_cost = INT64_MAX;
-  auto consider = [&](int tx, int cols, int nseg, int limit) {
-    const int seglen = (n + nseg - 1) / nseg;
-    if ((n + seglen - 1) / seglen != nseg) return;
-    // rows of the longest segment with the cells at its ends that it needs
-    const int rows = nseg == 1 ? n : !per && nseg == 2 ? seglen + 1 : seglen + 2;
-    const int64_t lanes = (int64_t)rows * cols;
-    if (lanes > limit) return;
-    const int64_t waves = (lanes + 63) / 64;
-    const int64_t cost = waves * nseg * ((nline + cols - 1) / cols);
-    if (cost < best_cost) {
-      best_cost = cost;
-      best = TileCut{tx, TilePlan{cols, rows, nseg, seglen}, (int)waves * 64};
-    }
-  };
-  if (dir == 0) {
-    for (int cols = 1; cols <= std::max(1, std::min(nline, 512 / n)); cols++) consider(-1, cols, 1, TILE_THREADS);
-    for (int nseg = 2; best_cost == INT64_MAX; nseg++) consider(-1, 1, nseg, TILE_THREADS);
-  } else {
-    const int max_seg = (n + 13) / 14;                 // segments of at least 14 cells
-    for (int x = 0; x < 3; x++)
-      for (int nseg = 1; nseg <= max_seg; nseg++) consider(x, TILE_TX[x], nseg, 512);
-  }
-  return best;
+// Rates of the (5, 3) kernels, which the cuts of the other orders share (a
+// ratio of the two kernels' times is all that they decide).  Fitted to sweeps
+// of 64x64x32 to 512x512x256 cells, every cut timed: best tiles 9 us at 64x64x32
+// (y and z; the walkers 55), 43 and 45 at 128x128x64 (57 and 62), 84 and 92 at
+// 160x160x80 (124 and 131), 147 and 161 at 192x192x96 (160 and 167), 228 and 271
+// at 96x300x200 (319 and 364), 340 and 393 at 256x256x128 (330 and 340).  The z
+// kernel has 112 registers, four waves per SIMD, which work-groups of five to
+// eight waves fill badly.
+static const awfl_tile::Rates& rates_of(int dir) {
+  static const awfl_tile::Rates xy{2.55, 1.03, {1.15, 1.18, 1.12, 1.07}, 2.3, 0.8, 3.2};
+  static const awfl_tile::Rates z{2.6, 1.03, {1.4, 1.33, 1.2, 1.15}, 2.35, 0.9, 3.4};
+  return dir == 2 ? z : xy;
 }
 
 // launch one tile sweep with the given kernels
-static int launch_tile(awfl_ctx* c, const double* in, double* out, const SweepK& K, int dir, const TileFns& f) {
+static int launch_tile(awfl_ctx* c, const double* in, double* out, const SweepK& K, int dir, const TileFns& f,
+                       const awfl_tile::TileCut* known = nullptr) {
   const int n = dir == 0 ? c->cfg.nx : dir == 1 ? c->cfg.ny : c->cfg.nz;
   const int nline = dir == 0 ? c->cfg.ny : c->cfg.nx;
+  const int other = dir == 2 ? c->cfg.ny : c->cfg.nz;
   const int bc = dir == 0 ? c->cfg.bc_x : dir == 1 ? c->cfg.bc_y : c->cfg.bc_z;
-  const TileCut cut = tile_plan(dir, n, nline, bc == AWFL_BC_PERIODIC);
+  const awfl_tile::TileCut cut =
+      known ? *known : awfl_tile::tile_cut(dir, n, nline, other, bc == AWFL_BC_PERIODIC, rates_of(dir));
   const TileFn k = dir == 0 ? f.x : f.yz[dir - 1][cut.tx];
-  const size_t lds = sizeof(double) * 5 * cut.p.cols * (size_t)(2 * cut.p.rows + 2 * c->hs);
+  const size_t lds = sizeof(double) * awfl_tile::lds_elems(cut.p, c->hs);
   if (lds > 64 * 1024)
     HIP_TRY(c, hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  const dim3 grid((nline + cut.p.cols - 1) / cut.p.cols, dir == 2 ? c->cfg.ny : c->cfg.nz, cut.p.nseg);
+  const dim3 grid((nline + cut.p.cols - 1) / cut.p.cols, other, cut.p.nseg);
   k<<<grid, cut.threads, lds, c->stream>>>(in, out, c->grid(), K, cut.p);
   LAUNCH_CHECK(c);
   return AWFL_OK;
 }
 
-// Whether a y or z sweep runs the column walker: with 4 million cells or more
-// its waves fill the chip, and it reads whole 512-byte rows and reconstructs
-// 6% of the cells twice where a tile is cut into segments with more (256x256x128:
-// y 324 against 362, z 337 against 391 us; 192x192x96: 158 against 147, 167 against
-// 192; 128x128x64: 58 against 43, 62 against 44; 96x300x200: 318 against 262, 362
-// against 318)
-static bool walks(const awfl_ctx* c, int dir) {
-  return (int64_t)c->cfg.nx * c->cfg.ny * c->cfg.nz >= 4000000;
+// One sweep of the per-cell kernels.  y and z run the column walker where its
+// modelled time is the smaller: on large grids, where its waves fill the chip
+// and it reads whole rows and cuts lines into longer segments.
+static int launch_cells(awfl_ctx* c, const double* in, double* out, const SweepK& K, int dir, const Variant* v,
+                        bool tend) {
+  if (dir == 0) return launch_tile(c, in, out, K, dir, v->tile[tend]);
+  const int n = dir == 1 ? c->cfg.ny : c->cfg.nz;
+  const int other = dir == 1 ? c->cfg.nz : c->cfg.ny;
+  const int bc = dir == 1 ? c->cfg.bc_y : c->cfg.bc_z;
+  const awfl_tile::Rates& rate = rates_of(dir);
+  const awfl_tile::TileCut cut = awfl_tile::tile_cut(dir, n, c->cfg.nx, other, bc == AWFL_BC_PERIODIC, rate);
+  const awfl_tile::WalkCut walk = awfl_tile::walk_cut(n, c->cfg.nx, other, rate);
+  if (cut.us <= walk.us) return launch_tile(c, in, out, K, dir, v->tile[tend], &cut);
+  v->col[dir - 1][tend]<<<dim3(walk.bx, other, walk.nseg), 64, 0, c->stream>>>(in, out, c->grid(), K, walk.seglen);
+  LAUNCH_CHECK(c);
+  return AWFL_OK;
 }
 
 // one lane-split line sweep: a work-group of awfl_line::LS_THREADS per line
@@ -1181,29 +1045,12 @@ static int launch_line(awfl_ctx* c, const double* in, double* out, const SweepK&
   return AWFL_OK;
 }
 
-// launch one column-walker sweep (y or z): segments of at most 32 cells, and
-// shorter (down to 16 cells) where that is needed for ~4 waves per SIMD
-static int launch_col(awfl_ctx* c, const double* in, double* out, const SweepK& K, int dir, ColFn k) {
-  const int n = dir == 1 ? c->cfg.ny : c->cfg.nz;
-  const int other = dir == 1 ? c->cfg.nz : c->cfg.ny;
-  const int bx = (c->cfg.nx + 63) / 64;
-  const int64_t layer = (int64_t)bx * other;
-  int nseg = (int)std::max<int64_t>(1, std::min<int64_t>(std::max<int64_t>((4096 + layer - 1) / layer, (n + 31) / 32),
-                                                         std::max(1, n / 16)));
-  const int seglen = (n + nseg - 1) / nseg;
-  nseg = (n + seglen - 1) / seglen;
-  k<<<dim3(bx, other, nseg), 64, 0, c->stream>>>(in, out, c->grid(), K, seglen);
-  LAUNCH_CHECK(c);
-  return AWFL_OK;
-}
-
 // launch one sweep; tend selects the tendency output (layout [5][nz][ny][nx])
 static int launch_sweep(awfl_ctx* c, const double* in, double* out, double dt, int dir, bool tend) {
   const Variant* v = static_cast<const Variant*>(c->var);
   if (v->sweep_line[dir][0])
     return launch_line(c, in, out, sweep_constants(c, dt, dir), dir, v->sweep_line[dir][tend ? 1 : 0]);
-  if (dir > 0 && walks(c, dir)) return launch_col(c, in, out, sweep_constants(c, dt, dir), dir, v->col[dir - 1][tend ? 1 : 0]);
-  return launch_tile(c, in, out, sweep_constants(c, dt, dir), dir, v->tile[tend ? 1 : 0]);
+  return launch_cells(c, in, out, sweep_constants(c, dt, dir), dir, v, tend);
 }
 
 static int fill(awfl_ctx* c, double* p, int64_t n, double v) {
@@ -1342,8 +1189,7 @@ int awfl_time_step_noalloc(awfl_ctx* c, double* d_state, double dt) {
       rc = (d == 0 && src == dst) ? launch_line(c, src, dst, K, 0, v->line_x_inplace, true)
                                   : launch_line(c, src, dst, K, d, v->sweep_line[d][0]);
     else
-      rc = d > 0 && walks(c, d) ? launch_col(c, src, dst, K, d, v->col[d - 1][0])
-                                : launch_tile(c, src, dst, K, d, v->tile[0]);   // (x lines are whole up to the limit above: in place)
+      rc = launch_cells(c, src, dst, K, d, v, false);   // (x lines are whole up to the limit above: in place)
     if (rc != AWFL_OK) return rc;
   }
   c->dimSwitch = !c->dimSwitch;

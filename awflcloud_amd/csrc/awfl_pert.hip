@@ -1,9 +1,9 @@
 // awfl_pert.hip -- FP32 perturbation-form split sweeps with Kahan-compensated
 // updates, and their C ABI (awfl_*_f32 in include/awfl_dycore.h).
 //
-// Same kernel organisation as the FP64 sweeps (awfl_dycore.hip): a workgroup
-// per x-line staged in LDS for the x sweep, one lane per x-column walking a
-// segment for y and z.  Storage is two FP32 arrays per state in the FP64
+// Kernels: a workgroup per x-line staged in LDS for the x sweep; for y and z
+// tiles with one lane per cell (awfl_tile.hpp), or on large grids one lane per
+// x-column walking a segment of it.  Storage is two FP32 arrays per state in the FP64
 // layout: the value s and its Kahan compensation c; the represented value is
 // s - c.  Each sweep reads (s, c) and writes (s', c') with
 //   y = dt*tend - c;  t = s + y;  c' = (t - s) - y;  s' = t.
@@ -18,6 +18,7 @@
 
 #include "awfl_cell_pert.hpp"
 #include "awfl_internal.hpp"
+#include "awfl_tile.hpp"
 
 using namespace awfl;
 using namespace awfl::pert;
@@ -42,6 +43,11 @@ __device__ __forceinline__ void kahan(float s, float c, float inc, float& so, fl
   so = t;
 }
 
+// x lines: one work-group of up to 256 lanes per line, each variable a row of
+// LDS.  The tile sweep (below) runs x lines no faster in FP32: 28 us against 28
+// at 128x128x64, 23 against 21 at 120x100x60, 53 against 48 at 300x100x60, 1697
+// against 1632 at 512x512x256 (lines of more than 256 cells loop here, and are
+// work-groups of up to 16 waves there).
 template <int ORD, int NGLL>
 __global__ __launch_bounds__(256) void k_sweep_x_f32(const float* __restrict__ in, const float* __restrict__ cin,
                                                      float* __restrict__ out, float* __restrict__ cout, GridF G,
@@ -133,6 +139,62 @@ __global__ __launch_bounds__(256) void k_sweep_x_f32(const float* __restrict__ i
       kahan(in[o], cin[o], K.dt * td, out[o], cout[o]);   // s again: an L2 hit, and LDS stays small
     }
   }
+}
+
+// The FP32 sweep's numerics for the tile sweep (awfl_tile.hpp).  The stencils
+// see s; the compensation c (below 1/2 ulp of s) enters only the update.
+template <int ORD_, int NGLL, int DIR_, int TX_>
+struct Sweep32 {
+  using real = float;
+  static constexpr int ORD = ORD_, DIR = DIR_, TX = TX_;
+  const float *s, *c;
+  float *so, *co;
+  const GridF& g;
+  const SweepKF& K;
+  __device__ const GridF& G() const { return g; }
+  __device__ const float* in() const { return s; }
+
+  __device__ __forceinline__ void cell(int o, int a, const float (&st)[5][ORD], float (&eL)[5], float (&eR)[5],
+                                       float& src) const {
+    CellBgP<NGLL> bg;
+    if constexpr (DIR < 2) {
+      const PointBg b = g.bgL[o];
+      sfor<NGLL>([&](auto ii) { bg.pt[ii] = b; });
+      bg.wall_bot = bg.wall_top = false;
+    } else {
+      sfor<NGLL>([&](auto ii) { bg.pt[ii] = g.bgG[a * NGLL + ii]; });
+      const bool per = g.bc[2] == AWFL_BC_PERIODIC;
+      bg.wall_bot = !per && a == 0;
+      bg.wall_top = !per && a == g.nz - 1;
+    }
+    cell_edges_pert<ORD, NGLL, DIR>(st, bg, g.weno_s, g.weno_w, K, eL, eR, src);
+  }
+  __device__ __forceinline__ void face(int o, int, int f, const float (&qL)[5], const float (&qR)[5],
+                                       float (&F)[5]) const {
+    riemann_pert<DIR>(qL, qR, DIR < 2 ? g.fbL[o] : g.fbF[f], F);
+  }
+  __device__ __forceinline__ void wall(int o, int line, int f, const float (&q)[5], float (&F)[5]) const {
+    face(o, line, f, q, q, F);
+  }
+  __device__ __forceinline__ void put(int, int, int, int64_t at, const float (&cell)[5], const float (&F0)[5],
+                                      const float (&F1)[5], float src) const {
+    float cc[5];
+    sfor<5>([&](auto l) { cc[l] = c[at + l * g.sl]; });
+    sfor<5>([&](auto l) {
+      float td = -(F1[l] - F0[l]) * K.rd;
+      if (DIR == 2 && l == idW) td = src + td;
+      if (DIR != 1 && g.sim2d && l == idV) td = 0.0f;
+      const int64_t i = at + l * g.sl;
+      kahan(cell[l], cc[l], K.dt * td, so[i], co[i]);
+    });
+  }
+};
+
+template <int ORD, int NGLL, int DIR, int TX>
+__global__ __launch_bounds__(awfl_tile::MAX_THREADS) void k_sweep_tile_f32(const float* s, const float* c, float* so,
+                                                                           float* co, GridF G, SweepKF K,
+                                                                           awfl_tile::TilePlan T) {
+  awfl_tile::sweep(Sweep32<ORD, NGLL, DIR, TX>{s, c, so, co, G, K}, T);
 }
 
 template <int ORD, int NGLL, int DIR>
@@ -294,15 +356,22 @@ __global__ void k_from_f32(const float* __restrict__ s, const float* __restrict_
     d[t] = (double)s[t] - (double)c[t];
 }
 
+using TileFnF = void (*)(const float*, const float*, float*, float*, GridF, SweepKF, awfl_tile::TilePlan);
+using ColFnF = void (*)(const float*, const float*, float*, float*, GridF, SweepKF, int);
 struct VariantF {
   int ord, ngll;
   void (*sweep_x)(const float*, const float*, float*, float*, GridF, SweepKF);
-  void (*sweep_y)(const float*, const float*, float*, float*, GridF, SweepKF, int);
-  void (*sweep_z)(const float*, const float*, float*, float*, GridF, SweepKF, int);
+  TileFnF yz[2][3];                    // y and z tiles by TX
+  ColFnF col[2];                       // y, z column walkers
 };
 
-#define AWFL_VARIANT_F(O, N) \
-  VariantF { O, N, k_sweep_x_f32<O, N>, k_sweep_col_f32<O, N, 1>, k_sweep_col_f32<O, N, 2> }
+#define AWFL_VARIANT_F(O, N)                                                                              \
+  VariantF {                                                                                              \
+    O, N, k_sweep_x_f32<O, N>,                                                                            \
+        {{k_sweep_tile_f32<O, N, 1, 4>, k_sweep_tile_f32<O, N, 1, 8>, k_sweep_tile_f32<O, N, 1, 16>},     \
+         {k_sweep_tile_f32<O, N, 2, 4>, k_sweep_tile_f32<O, N, 2, 8>, k_sweep_tile_f32<O, N, 2, 16>}},    \
+        {k_sweep_col_f32<O, N, 1>, k_sweep_col_f32<O, N, 2>}                                              \
+  }
 
 const VariantF kVariantsF[] = {AWFL_VARIANT_F(3, 2), AWFL_VARIANT_F(5, 3)};
 
@@ -406,33 +475,40 @@ SweepKF sweep_constants_f(const awfl_ctx* c, double dt, int dir) {
   return K;
 }
 
+// Rates of the FP32 kernels for the cuts.  Fitted to: tiles 8 us at 64x64x32 (y
+// and z; the walkers 46 and 43), 25 at 120x100x60 (51 and 56), 33 at 128x128x64
+// (48), 108 and 112-128 at 192x192x96 (103 and 104), 234 and 260 at 256x256x128
+// (230 and 218), 1947 and 1999 at 512x512x256 (1545 and 1609).
+constexpr awfl_tile::Rates RATES_F32{1.75, 1.2, {1.15, 1.18, 1.12, 1.07}, 1.4, 1.0, 2.7};
+
 int launch_sweep_f32(awfl_ctx* c, const float* s, const float* cs, float* so, float* co, double dt, int dir) {
   GridF F = grid_f(c);
   SweepKF K = sweep_constants_f(c, dt, dir);
   const VariantF* v = find_variant_f(c->cfg.ord, c->cfg.ngll);
   if (dir == 0) {
-    int nx = c->cfg.nx;
-    int threads = line_threads(nx);
-    size_t lds = sizeof(float) * (size_t)(5 * (nx + 2 * c->hs) + 10 * nx);
+    const int nx = c->cfg.nx;
+    const size_t lds = sizeof(float) * (size_t)(5 * (nx + 2 * c->hs) + 10 * nx);
     if (lds > 64 * 1024)
       HIP_TRY(c, hipFuncSetAttribute((const void*)v->sweep_x, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    v->sweep_x<<<c->cfg.ny * c->cfg.nz, threads, lds, c->stream>>>(s, cs, so, co, F, K);
+    v->sweep_x<<<c->cfg.ny * c->cfg.nz, line_threads(nx), lds, c->stream>>>(s, cs, so, co, F, K);
     LAUNCH_CHECK(c);
     return AWFL_OK;
   }
-  int n = dir == 1 ? c->cfg.ny : c->cfg.nz;
-  int other = dir == 1 ? c->cfg.nz : c->cfg.ny;
-  int bx = (c->cfg.nx + 63) / 64;
-  // segments as in the FP64 sweeps: at most 32 cells, down to 16 for ~4
-  // waves per SIMD
-  int64_t layer = (int64_t)bx * other;
-  int nseg = (int)std::max<int64_t>(1, std::min<int64_t>(std::max<int64_t>((4096 + layer - 1) / layer, (n + 31) / 32),
-                                                           std::max(1, n / 16)));
-  int seglen = (n + nseg - 1) / nseg;
-  nseg = (n + seglen - 1) / seglen;
-  dim3 grid(bx, other, nseg);
-  auto kern = dir == 1 ? v->sweep_y : v->sweep_z;
-  kern<<<grid, 64, 0, c->stream>>>(s, cs, so, co, F, K, seglen);
+  // y and z: tiles, or the column walker where its modelled time is the smaller
+  const int n = dir == 1 ? c->cfg.ny : c->cfg.nz;
+  const int other = dir == 1 ? c->cfg.nz : c->cfg.ny;
+  const int bc = dir == 1 ? c->cfg.bc_y : c->cfg.bc_z;
+  const awfl_tile::TileCut cut = awfl_tile::tile_cut(dir, n, c->cfg.nx, other, bc == AWFL_BC_PERIODIC, RATES_F32);
+  const awfl_tile::WalkCut walk = awfl_tile::walk_cut(n, c->cfg.nx, other, RATES_F32);
+  if (walk.us < cut.us) {
+    v->col[dir - 1]<<<dim3(walk.bx, other, walk.nseg), 64, 0, c->stream>>>(s, cs, so, co, F, K, walk.seglen);
+    LAUNCH_CHECK(c);
+    return AWFL_OK;
+  }
+  const TileFnF k = v->yz[dir - 1][cut.tx];
+  const size_t lds = sizeof(float) * awfl_tile::lds_elems(cut.p, c->hs);
+  k<<<dim3((c->cfg.nx + cut.p.cols - 1) / cut.p.cols, other, cut.p.nseg), cut.threads, lds, c->stream>>>(s, cs, so, co,
+                                                                                                         F, K, cut.p);
   LAUNCH_CHECK(c);
   return AWFL_OK;
 }
