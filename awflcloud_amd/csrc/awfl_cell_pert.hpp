@@ -54,146 +54,132 @@ struct CellBgP {
   bool wall_bot, wall_top; // z: solid wall and k == 0 / k == nz-1
 };
 
-// Launch constants in FP32
-// Launch constants in FP32.  dn[kt][s][ii] = D[s][ii] * ndt[kt]: the GLL
-// derivative matrix with the transform factor -1/(d (kt+1)) folded in
-// (ngll <= 3 here).
-constexpr int PK_NA = 3, PK_NG = 3;
+// Launch constants in FP32.
 struct SweepKF {
   float dt, rd;
   float ndt[KMAX];
   float tav[KMAX];
-  float dn[PK_NA - 1][PK_NG][PK_NG];
 };
 
+// n times the GLL derivative of point values (two or three points), and that
+// added to the two edge values: gll_deriv / gll_deriv_edges of awfl_cell.hpp
+template <int NGLL>
+__device__ __forceinline__ void gll_deriv_f(const float (&F)[NGLL], float n, float (&d)[NGLL]) {
+  static_assert(NGLL == 2 || NGLL == 3, "FP32 sweeps have two or three points");
+  if constexpr (NGLL == 2) {
+    d[0] = d[1] = (F[1] - F[0]) * n;
+  } else {
+    const float a = (F[2] - F[0]) * n, c = fmaf(-2.0f, F[1], F[0] + F[2]), h = 2.0f * n;
+    d[0] = fmaf(-h, c, a);
+    d[1] = a;
+    d[2] = fmaf(h, c, a);
+  }
+}
+template <int NGLL>
+__device__ __forceinline__ void gll_deriv_edges_f(const float (&F)[NGLL], float n, float& eL, float& eR) {
+  if constexpr (NGLL == 2) {
+    const float t = (F[1] - F[0]) * n;
+    eL += t;
+    eR += t;
+  } else {
+    const float a = F[2] - F[0], c = fmaf(-2.0f, F[1], F[0] + F[2]), h = 2.0f * n;
+    eL = fmaf(-h, c, fmaf(n, a, eL));
+    eR = fmaf(h, c, fmaf(n, a, eR));
+  }
+}
+
 // One cell of a DIR sweep in perturbation form: deviation stencils -> deviation
-// edge states (time averaged) and the z gravity source.
+// edge states (time averaged) and the z gravity source.  The transform's
+// organisation is cell_edges_of's (awfl_cell.hpp): the normal velocity's Taylor
+// coefficients u_k carry every flux (u_k sums in place of the reference's
+// quotients), the last level goes straight into the edge states, and the z
+// source's cell average comes from the end points.
 template <int ORD, int NGLL, int DIR>
 __device__ __forceinline__ void cell_edges_pert(const float (&st)[5][ORD], const CellBgP<NGLL>& bg, bool weno_s,
                                                 bool weno_w, const SweepKF& K, float (&eL)[5], float (&eR)[5],
                                                 float& src_avg) {
-  constexpr int NA = NGLL;
   constexpr int NM = 1 + DIR;
-  static_assert(NA <= PK_NA && NGLL <= PK_NG, "FP32 launch constants sized for ngll <= 3");
-  float q[5][NA][NGLL];    // level 0: deviations for rho and rho*theta; other levels deviations throughout
-  float fr0[NGLL], frt0[NGLL];   // full rho and rho*theta at level 0
-  float f[4][NA][NGLL];
-  float g[NA][NGLL];       // (rho theta)^gamma: level 0 full, higher levels (doubled) deviations
-  float pp[NGLL];          // p' at level 0
-  float src[NA][NGLL];
-  float rr[NGLL], rrt[NGLL];
-
-  sfor<5>([&](auto l) {
-    float gv[NGLL];
-    reconstruct<ORD, NGLL>(st[l], (l == idR || l == idT) ? weno_s : weno_w, gv);
-    sfor<NGLL>([&](auto ii) { q[l][0][ii] = gv[ii]; });
-  });
+  static_assert(NGLL <= 3, "one or two transform levels");
+  float q[5][NGLL];              // level 0: deviations (full rho in r0, rho*theta in t0)
+  float r0[NGLL], t0[NGLL], rr[NGLL], u0[NGLL], pp[NGLL];
+  sfor<5>([&](auto l) { reconstruct<ORD, NGLL>(st[l], (l == idR || l == idT) ? weno_s : weno_w, q[l]); });
+  const float sv = DIR == 2 ? -GRAVF * q[idR][NGLL - 1] : 0.0f;   // S:1439: the last point's, everywhere
   if constexpr (DIR == 2) {
-    if (bg.wall_top) q[idW][0][NGLL - 1] = 0.0f;
-    if (bg.wall_bot) q[idW][0][0] = 0.0f;
+    if (bg.wall_top) q[idW][NGLL - 1] = 0.0f;
+    if (bg.wall_bot) q[idW][0] = 0.0f;
   }
-  float sv = 0.0f;
   sfor<NGLL>([&](auto ii) {
     const PointBg& b = bg.pt[ii];
-    fr0[ii] = b.r + q[idR][0][ii];
-    frt0[ii] = b.rt + q[idT][0][ii];
-    rr[ii] = __builtin_amdgcn_rcpf(fr0[ii]);
-    const float un = q[NM][0][ii] * rr[ii];   // r * (q_nm / r) * (q_l / r) = (q_nm / r) * q_l
-    f[0][0][ii] = un * q[1][0][ii];
-    f[1][0][ii] = un * q[2][0][ii];
-    f[2][0][ii] = un * q[3][0][ii];
-    f[3][0][ii] = un * frt0[ii];
-    float s = powm1_gamma(q[idT][0][ii] * b.rrt);
-    pp[ii] = b.p * s;
-    g[0][ii] = (b.p + pp[ii]) * (1.0f / C0F);
-    rrt[ii] = __builtin_amdgcn_rcpf(frt0[ii]);
-    if constexpr (DIR == 2) sv = -q[idR][0][ii] * GRAVF;
+    r0[ii] = b.r + q[idR][ii];
+    t0[ii] = b.rt + q[idT][ii];
+    rr[ii] = __builtin_amdgcn_rcpf(r0[ii]);
+    u0[ii] = q[NM][ii] * rr[ii];
+    // p' at level 0; the constant-in-the-sweep background pressure has zero
+    // derivative (x/y), z subtracts hyPressureGLL (S:2042): both leave p'
+    pp[ii] = b.p * powm1_gamma(q[idT][ii] * b.rrt);
   });
-  if constexpr (DIR == 2) {
-    sfor<NA>([&](auto kt) { sfor<NGLL>([&](auto ii) { src[kt][ii] = sv; }); });   // S:1439
-  }
-
-  sfor<NA - 1>([&](auto kt) {
-    constexpr float rkt1 = 1.0f / (kt + 1.0f);
-    sfor<NGLL>([&](auto ii) {
-      float d[5];
-      sfor<5>([&](auto l) { d[l] = -0.0f; });
-      sfor<NGLL>([&](auto s) {
-        if constexpr (Deriv<NGLL>::m[s][ii] == 0.0) return;
-        const float D = K.dn[kt][s][ii];
-        d[0] += D * q[NM][kt][s];
-        sfor<4>([&](auto m) {
-          constexpr int l = m + 1;
-          if constexpr (l == NM) {
-            // the constant-in-the-sweep background pressure has zero derivative
-            // (x/y); z subtracts hyPressureGLL (S:2042): both leave p'
-            if constexpr (kt == 0) d[l] += D * (f[m][kt][s] + pp[s]);
-            else d[l] += D * (f[m][kt][s] + (0.5f * C0F) * g[kt][s]);
-          } else {
-            d[l] += D * f[m][kt][s];
-          }
-        });
-      });
-      sfor<5>([&](auto l) {
-        if constexpr (DIR == 2 && l == idW) q[l][kt + 1][ii] = d[l] + src[kt][ii] * rkt1;
-        else q[l][kt + 1][ii] = d[l];
-      });
-      if constexpr (DIR == 2) {
-        if (bg.wall_top) q[idW][kt + 1][NGLL - 1] = 0.0f;
-        if (bg.wall_bot) q[idW][kt + 1][0] = 0.0f;
-        src[kt + 1][ii] = -q[idR][kt + 1][ii] * GRAVF;
-      }
+  sfor<5>([&](auto l) {
+    eL[l] = q[l][0];
+    eR[l] = q[l][NGLL - 1];
+  });
+  float sa = sv;
+  if constexpr (DIR == 2) sa = fmaf(-GRAVF * (K.tav[1] * K.ndt[0]), q[NM][NGLL - 1] - q[NM][0], sa);
+  // level 1
+  float d[5][NGLL];
+  sfor<5>([&](auto l) {
+    float F[NGLL];
+    sfor<NGLL>([&](auto s) {
+      if constexpr (l == idR) F[s] = q[NM][s];
+      else if constexpr (l == NM) F[s] = fmaf(u0[s], q[NM][s], pp[s]);
+      else F[s] = u0[s] * (l == idT ? t0[s] : q[l][s]);
     });
-    if constexpr (kt + 2 < NA) {
-      sfor<NGLL>([&](auto ii) {
-        auto full = [&](int l, int lev) -> float {
-          if (lev == 0 && l == idR) return fr0[ii];
-          if (lev == 0 && l == idT) return frt0[ii];
-          return q[l][lev][ii];
-        };
-        sfor<4>([&](auto m) {
-          constexpr int l = m + 1;
-          float tot = 0.0f;
-          sfor<kt + 2>([&](auto ir) {
-            if constexpr (ir == 0) tot += q[NM][ir][ii] * q[l][kt + 1 - ir][ii];
-            else tot += q[NM][ir][ii] * full(l, kt + 1 - ir) - full(idR, ir) * f[m][kt + 1 - ir][ii];
-          });
-          f[m][kt + 1][ii] = tot * rr[ii];
-        });
-        float tg = 0.0f;
-        sfor<kt + 1>([&](auto ir) {
-          constexpr float wgt = kt + 1.0f - ir;
-          if constexpr (ir == 0)
-            tg += wgt * (GAMMAF * g[ir][ii] * q[idT][kt + 1 - ir][ii]);
-          else
-            tg += wgt * (GAMMAF * g[ir][ii] * q[idT][kt + 1 - ir][ii] - full(idT, ir) * g[kt + 1 - ir][ii]);
-        });
-        g[kt + 1][ii] = (GAMMAF * g[0][ii] * q[idT][kt + 1][ii] + tg * rkt1) * rrt[ii];
-      });
+    if constexpr (NGLL == 2) {
+      gll_deriv_edges_f<NGLL>(F, K.ndt[0] * K.tav[1], eL[l], eR[l]);
+      if constexpr (DIR == 2 && l == idW) {
+        eL[l] = fmaf(K.tav[1], sv, eL[l]);
+        eR[l] = fmaf(K.tav[1], sv, eR[l]);
+      }
+    } else {
+      gll_deriv_f<NGLL>(F, K.ndt[0], d[l]);
+      if constexpr (DIR == 2 && l == idW) {       // S:2049-2055
+        sfor<NGLL>([&](auto ii) { d[l][ii] += sv; });
+        if (bg.wall_top) d[l][NGLL - 1] = 0.0f;
+        if (bg.wall_bot) d[l][0] = 0.0f;
+      }
+      eL[l] = fmaf(d[l][0], K.tav[1], eL[l]);
+      eR[l] = fmaf(d[l][NGLL - 1], K.tav[1], eR[l]);
     }
   });
-
-  sfor<5>([&](auto l) {
-    float a0 = q[l][0][0], a1 = q[l][0][NGLL - 1];
-    sfor<NA - 1>([&](auto km) {
-      constexpr int kt = km + 1;
-      a0 += q[l][kt][0] * K.tav[kt];
-      a1 += q[l][kt][NGLL - 1] * K.tav[kt];
+  // level 2
+  if constexpr (NGLL == 3) {
+    float u1[NGLL], p1[NGLL];
+    sfor<NGLL>([&](auto ii) {
+      u1[ii] = fmaf(-d[idR][ii], u0[ii], d[NM][ii]) * rr[ii];
+      p1[ii] = ((bg.pt[ii].p + pp[ii]) * __builtin_amdgcn_rcpf(t0[ii])) * (GAMMAF * d[idT][ii]);
     });
-    eL[l] = a0;
-    eR[l] = a1;
-  });
-  if constexpr (DIR == 2) {
-    sfor<NA - 1>([&](auto km) {
-      constexpr int kt = km + 1;
-      sfor<NGLL>([&](auto ii) { src[0][ii] += src[kt][ii] * K.tav[kt]; });
+    if constexpr (DIR == 2) sa = fmaf(-GRAVF * (K.tav[2] * K.ndt[1]), d[NM][2] - d[NM][0], sa);
+    sfor<5>([&](auto l) {
+      float F[NGLL];
+      sfor<NGLL>([&](auto s) {
+        if constexpr (l == idR) F[s] = d[NM][s];
+        else {
+          F[s] = u0[s] * d[l][s];
+          F[s] = fmaf(u1[s], l == idT ? t0[s] : q[l][s], F[s]);
+          if constexpr (l == NM) F[s] += p1[s];
+        }
+      });
+      gll_deriv_edges_f<NGLL>(F, K.ndt[1] * K.tav[2], eL[l], eR[l]);
+      if constexpr (DIR == 2 && l == idW) {
+        eL[l] = fmaf(-0.5f * GRAVF * K.tav[2], d[idR][0], eL[l]);
+        eR[l] = fmaf(-0.5f * GRAVF * K.tav[2], d[idR][NGLL - 1], eR[l]);
+      }
     });
-    float sa = 0.0f;
-    sfor<NGLL>([&](auto ii) { sa += src[0][ii] * (float)Gll<NGLL>::wts[ii]; });
-    src_avg = sa;
-  } else {
-    src_avg = 0.0f;
   }
+  if constexpr (DIR == 2) {
+    if (bg.wall_top) eR[idW] = 0.0f;
+    if (bg.wall_bot) eL[idW] = 0.0f;
+  }
+  src_avg = sa;
 }
 
 // background seen by one face
@@ -234,35 +220,25 @@ __device__ __forceinline__ void riemann_pert(const float (&L)[5], const float (&
   // sound speed and its reciprocal from one hardware reciprocal square root
   const float c2 = GAMMAF * p * __builtin_amdgcn_rcpf(r);
   const float rc = __builtin_amdgcn_rsqf(c2);
-  float cs = c2 * rc;
-  float it = __builtin_amdgcn_rcpf(t);
-  float i2c = 0.5f * rc;
-  // characteristic amplitudes of the deviation vector
-  float w1, w2, w3;
-  if (un > 0) {
-    float a = L[4] * it;
-    w1 = L[0] - a;
-    w2 = L[T1] - ut1 * a;
-    w3 = L[T2] - ut2 * a;
-  } else {
-    float a = R[4] * it;
-    w1 = R[0] - a;
-    w2 = R[T1] - ut1 * a;
-    w3 = R[T2] - ut2 * a;
-  }
-  float w5 = (un * R[0] - R[NM]) * i2c + 0.5f * R[4] * it;
-  float w6 = (L[NM] - un * L[0]) * i2c + 0.5f * L[4] * it;
-  float q1 = w1 + w5 + w6;                          // deviations of the recomposed state
-  float qn = un * w1 + (un - cs) * w5 + (un + cs) * w6;
-  float qt1 = w2 + ut1 * w5 + ut1 * w6;
-  float qt2 = w3 + ut2 * w5 + ut2 * w6;
-  float q5 = t * w5 + t * w6;
-  float iq1 = __builtin_amdgcn_rcpf(fb.r + q1);
+  const float cs = c2 * rc;
+  const float i2c = 0.5f * rc;
+  // the waves and the recomposed deviations in differences of the two sides
+  // (riemann in awfl_cell.hpp): v the deviation that the acoustic waves and the
+  // upwind side add to U
+  const bool up = un > 0;
+  const float u0 = up ? L[0] : R[0], u1 = up ? L[T1] : R[T1], u2 = up ? L[T2] : R[T2];
+  const float D = fmaf(un, R[0] - L[0], L[NM] - R[NM]) * i2c;
+  const float d = (R[4] - L[4]) * (0.5f * __builtin_amdgcn_rcpf(t));
+  const float v = D + (up ? d : -d);
+  const float q1 = u0 + v;                          // deviations of the recomposed state
+  const float qn = fmaf(-cs, d, fmaf(un, q1 - 0.5f * (L[0] + R[0]), 0.5f * (L[NM] + R[NM])));
+  const float q5 = fmaf(t, D, 0.5f * (L[4] + R[4]));
+  const float un1 = qn * __builtin_amdgcn_rcpf(fb.r + q1);
   F[0] = qn;
-  F[NM] = qn * qn * iq1 + fb.p * powm1_gamma(q5 * fb.rrt);
-  F[T1] = qn * qt1 * iq1;
-  F[T2] = qn * qt2 * iq1;
-  F[4] = qn * (fb.rt + q5) * iq1;
+  F[NM] = fmaf(qn, un1, fb.p * powm1_gamma(q5 * fb.rrt));
+  F[T1] = un1 * fmaf(ut1, v, u1);
+  F[T2] = un1 * fmaf(ut2, v, u2);
+  F[4] = un1 * (fb.rt + q5);
 }
 
 }  // namespace pert

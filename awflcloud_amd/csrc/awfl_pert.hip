@@ -465,13 +465,6 @@ SweepKF sweep_constants_f(const awfl_ctx* c, double dt, int dir) {
       dtmult *= dt;
     }
   }
-  const int ng = c->cfg.ngll;
-  for (int kt = 0; kt + 1 < ng && kt < PK_NA - 1; kt++)
-    for (int s = 0; s < ng; s++)
-      for (int ii = 0; ii < ng; ii++) {
-        double D = ng == 2 ? awfl_deriv_2[s][ii] : awfl_deriv_3[s][ii];
-        K.dn[kt][s][ii] = (float)(D * (-1.0 / (dsw * (kt + 1.0))));
-      }
   return K;
 }
 
