@@ -189,12 +189,15 @@ __global__ __launch_bounds__(64) void k_edges(const double* __restrict__ st, con
   if constexpr (std::is_same<T, double>::value) load_stencil<ORD, DIR>(st, G, p, w);
   else load_stencil<ORD, DIR>(st, dst, G, p, w);
   const CellBg<NGLL> bg = cell_bg<NGLL, DIR>(G, p.k);
-  adj::Tape<NGLL, T> tp;
   T q0[5][NGLL], eL[5], eR[5], sa;
   adj::cell_recon<ORD, NGLL>(w, G.weno_s, G.weno_w, q0);
-  if constexpr (std::is_same<T, double>::value)
+  if constexpr (std::is_same<T, double>::value) {
     sfor<5>([&](auto l) { sfor<NGLL>([&](auto ii) { Q0[(l * NGLL + ii) * nc + t] = q0[l][ii]; }); });
-  adj::cell_dt<NGLL, DIR>(q0, bg, K, tp, eL, eR, sa);
+    cell_transform<NGLL, DIR>(q0, bg, K, eL, eR, sa, [](const auto&, const auto&) {});
+  } else {
+    adj::Tape<NGLL, T> tp;
+    adj::cell_dt<NGLL, DIR>(q0, bg, K, tp, eL, eR, sa);
+  }
   sfor<5>([&](auto l) {
     E[l * nc + t] = adj::val(eL[l]);
     E[(5 + l) * nc + t] = adj::val(eR[l]);
@@ -512,8 +515,7 @@ __global__ __launch_bounds__(256) void k_adj_line(const double* __restrict__ in,
     }
     double q0[5][NGLL], eL[5], eR[5], sa;
     sfor<5>([&](auto l) { sfor<NGLL>([&](auto ii) { q0[l][ii] = s_q[(l * NGLL + ii) * n + c]; }); });
-    adj::Tape<NGLL, double> tp;
-    adj::cell_dt<NGLL, DIR>(q0, bg_of(c), K, tp, eL, eR, sa);
+    cell_transform<NGLL, DIR>(q0, bg_of(c), K, eL, eR, sa, [](const auto&, const auto&) {});
     sfor<5>([&](auto l) {
       s_e[l * n + c] = eL[l];
       s_e[(5 + l) * n + c] = eR[l];

@@ -540,8 +540,8 @@ template <int ORD, int NGLL, class T>
 __host__ __device__ __forceinline__ void reconstruct(const T (&u)[ORD], bool doweno, T (&g)[NGLL]) {
   using P = Proj<ORD, NGLL>;
   // the difference forms serve the sweeps' scalars (double and float); the
-  // tangent-linear scalar keeps the general form its hand-written reverse
-  // follows, and the bridge parity build the reference's three statements
+  // tangent-linear scalar keeps the general form, and the bridge parity build
+  // the reference's three statements
   constexpr bool diff = (std::is_same<T, double>::value || std::is_same<T, float>::value) &&
                         !(AWFL_PARITY & AWFL_PAR_BRIDGE);
   if (doweno) {
@@ -678,16 +678,13 @@ __host__ __device__ __forceinline__ void gll_deriv_edges(const double (&F)[NGLL]
 // 256x256x128 from 1.148 to 1.000 ms; the errors against 64-bit torch did not
 // grow (7.6e-15 -> 7.4e-15 of the state).
 // ---------------------------------------------------------------------------
-// load_bg() returns the cell's background; it is called after the
-// reconstructions, so that a background that differs between lanes is not
-// held in registers through them.
 // levels(r0, u) receives the density at the GLL points (background added) and
 // the normal velocity's Taylor coefficients u[level][point], levels 0 ..
 // NGLL-2, which the tracer sweeps' transform takes (S:757-758).
-template <int ORD, int NGLL, int DIR, class LoadBg, class Levels>
-__host__ __device__ __forceinline__ void cell_edges_of(const double (&st)[5][ORD], LoadBg&& load_bg, bool weno_s,
-                                              bool weno_w, const SweepK& K, double (&eL)[5], double (&eR)[5],
-                                              double& src_avg, Levels&& levels) {
+template <int NGLL, int DIR, class Levels>
+__host__ __device__ __forceinline__ void cell_transform(const double (&q0)[5][NGLL], const CellBg<NGLL>& bg,
+                                               const SweepK& K, double (&eL)[5], double (&eR)[5], double& src_avg,
+                                               Levels&& levels) {
   AWFL_NO_CONTRACT
   constexpr int NA = NGLL;             // nAder = ngll (Temporal_ader.h:8)
   constexpr int NM = 1 + DIR;          // momentum normal to the sweep
@@ -697,13 +694,8 @@ __host__ __device__ __forceinline__ void cell_edges_of(const double (&st)[5][ORD
   double g[NA][NGLL];                  // (r t)^gamma, levels >= 1 carried doubled (S:1904-1915)
   double rr[NGLL], rrt[NGLL];          // 1/r and 1/(r t) at level 0
 
-  // level 0: reconstruction + background
-  sfor<5>([&](auto l) {
-    double gv[NGLL];
-    reconstruct<ORD, NGLL>(st[l], (l == idR || l == idT) ? weno_s : weno_w, gv);
-    sfor<NGLL>([&](auto ii) { q[l][0][ii] = gv[ii]; });
-  });
-  const CellBg<NGLL> bg = load_bg();
+  // level 0: the reconstruction, and the background
+  sfor<5>([&](auto l) { sfor<NGLL>([&](auto ii) { q[l][0][ii] = q0[l][ii]; }); });
   // S:1439 assigns a scalar to the whole SArray: every entry of the source's
   // level 0 holds the value of the last GLL point
   const double sv = DIR == 2 ? -GRAV * q[idR][0][NGLL - 1] : 0.0;
@@ -825,6 +817,18 @@ __host__ __device__ __forceinline__ void cell_edges_of(const double (&st)[5][ORD
   src_avg = DIR == 2 ? sa : 0.0;       // S:1462, 1489-1492
 }
 
+// Reconstruction and transform of a cell.  load_bg() returns the cell's
+// background; it is called after the reconstructions, so that a background
+// that differs between lanes is not held in registers through them.
+template <int ORD, int NGLL, int DIR, class LoadBg, class Levels>
+__host__ __device__ __forceinline__ void cell_edges_of(const double (&st)[5][ORD], LoadBg&& load_bg, bool weno_s,
+                                              bool weno_w, const SweepK& K, double (&eL)[5], double (&eR)[5],
+                                              double& src_avg, Levels&& levels) {
+  double q0[5][NGLL];
+  sfor<5>([&](auto l) { reconstruct<ORD, NGLL>(st[l], (l == idR || l == idT) ? weno_s : weno_w, q0[l]); });
+  const CellBg<NGLL> bg = load_bg();
+  cell_transform<NGLL, DIR>(q0, bg, K, eL, eR, src_avg, levels);
+}
 template <int ORD, int NGLL, int DIR, class Levels>
 __host__ __device__ __forceinline__ void cell_edges(const double (&st)[5][ORD], const CellBg<NGLL>& bg, bool weno_s,
                                            bool weno_w, const SweepK& K, double (&eL)[5], double (&eR)[5],
