@@ -4,11 +4,10 @@
 // awfl_forward_ckpt / awfl_adjoint_ckpt in include/awfl_dycore.h).
 //
 // One split sweep is out = in + dt * T(in) (awfl_sweep).  Its adjoint
-// adj_in = adj_out + J^T (dt adj_out) runs as one fused kernel per line
-// along the sweep direction (k_adj_line: forward, face adjoints, transform
-// and WENO reverses and the gather, all in LDS).  Lines too long for LDS
-// (more than about 580 cells at WENO5) run as five kernels over per-cell
-// scratch in HBM:
+// adj_in = adj_out + J^T (dt adj_out) runs as one fused kernel over whole lines
+// along the sweep direction (k_adj_tile: forward, face adjoints, transform
+// and WENO reverses and the gather in registers and LDS).  Lines of more than
+// ADJ_MAX cells run as five kernels over per-cell scratch in HBM:
 //   k_edges      cell forward, one thread per cell: WENO values at the GLL
 //                points [5 ngll/cell], then time-averaged edge states and
 //                z source                                                [11/cell]
@@ -342,356 +341,239 @@ __global__ __launch_bounds__(64) void k_weno_adj(const double* __restrict__ st, 
 }
 
 // ---------------------------------------------------------------------------
-// Sweep adjoint fused into one kernel: one work-group per line along DIR
-// with the line and every intermediate in LDS (nothing per cell crosses
-// HBM).  x lines are contiguous; y and z lines are strided, and the
-// XCD-aware line order keeps neighbouring lines (which share every cache
-// line they touch) on one XCD at about the same time.  LDS (doubles): the
-// state line [5][n+2hs], a region [5 NGLL][n] for the WENO values of each
-// cell and then, in place, their adjoints q0b, and a region [10][n] for the
-// edge states, replaced in place by the edge-state adjoints (every slot is
-// read and written by the one face thread that owns it); the two regions
-// then hold the stencil adjoints of all five variables (adj_row); then the
-// line's constants and adj_out along the line [5][n], staged once.
+// Sweep adjoint fused into one kernel: a work-group takes whole lines along
+// DIR, one lane per cell, and nothing per cell crosses HBM but the state and
+// the two adjoints.  A cell's reconstruction (and, after the transform's
+// reverse, its adjoint) stays in the registers of its lane through all phases;
+// LDS holds what neighbours exchange, 20 doubles per cell: the state [5],
+// adj_out [5], and ten slots that hold the edge states, then in place their
+// adjoints (every slot is read and written by the one face lane that owns
+// it), then the stencil adjoints of adj_pv variables at a time.
+//
+// Bound by FP64 issue and its latencies: about 2,400 of 3,000 instructions per
+// cell are FP64 and the VALU is busy two thirds of the time.  20 doubles of LDS
+// and 168 registers allow 12 waves per CU; the form before (the GLL values and
+// all stencil adjoints in LDS, 35 doubles per cell and 8 waves, one line per
+// work-group) took 155 us for x and y and 168 us for z at 128x128x64 against
+// 123, 128 and 131 us, and left the lanes past a line's end idle: z at 100x90x75
+// 205 us with the older reverses, 96 us now.
 // ---------------------------------------------------------------------------
-// WENO reverses per thread side by side in the line kernel
+// WENO reverses per lane side by side: what the ten slots hold
 template <int ORD>
 constexpr int adj_pv() {
-  return 2 * ORD <= 10 ? 2 : 1;
+  return 10 / ORD;
 }
-// row of the stencil adjoint of variable l, slot s, in the line kernel's row
-// region [s_q | s_e] of 5 NGLL + 10 rows: variable after variable from the
-// first edge row on, wrapping to row 0
-template <int ORD, int NGLL>
-__host__ __device__ constexpr int adj_row(int l, int s) {
-  return (5 * NGLL + l * ORD + s) % (5 * NGLL + 10);
-}
-// every stencil adjoint has a row of its own, and none lands on the q0b rows
-// (l NGLL .. l NGLL + NGLL - 1) of a variable whose WENO reverse runs in a
-// later group of PV
-template <int ORD, int NGLL, int PV>
-constexpr bool adj_rows_ok() {
-  if (5 * ORD > 5 * NGLL + 10) return false;
-  for (int l = 0; l < 5; ++l) {
-    const int next = (l / PV + 1) * PV < 5 ? (l / PV + 1) * PV : 5;
-    for (int s = 0; s < ORD; ++s) {
-      const int r = adj_row<ORD, NGLL>(l, s);
-      if (r >= next * NGLL && r < 5 * NGLL) return false;
-    }
-  }
-  return true;
-}
-template <int ORD, int NGLL>
-constexpr int adj_line_rows() {
-  return 5 * NGLL + 10;
-}
-constexpr int LINE_K = 10;
+constexpr int ADJ_SLOTS = 20;
+constexpr int ADJ_MAX = 640;    // cells of a line, lanes of a work-group
 
 template <int ORD, int NGLL, int DIR>
-__global__ __launch_bounds__(256) void k_adj_line(const double* __restrict__ in, const double* __restrict__ adj_out,
-                                                  double* __restrict__ adj_in, Grid G, SweepK K) {
-  static_assert(ORD <= 10, "stencil adjoints of one variable fit the edge region");
+__global__ __launch_bounds__(ADJ_MAX) __attribute__((amdgpu_waves_per_eu(3))) void k_adj_tile(
+    const double* __restrict__ in, const double* __restrict__ adj_out, double* __restrict__ adj_in, Grid G, SweepK K,
+    int cols) {
+  static_assert(ORD <= 10, "stencil adjoints of one variable fit the ten slots");
   constexpr int hs = (ORD - 1) / 2;
   constexpr int NM = 1 + DIR;
+  constexpr int PV = adj_pv<ORD>();
   extern __shared__ double sm[];
   const int n = axis_len<DIR>(G);
-  const int W = n + 2 * hs;
-  const int bd = line_threads(n);     // blockDim.x of the launch
-  // line -> its first interior cell, the stride along DIR and the level k of
-  // an x or y line
-  const unsigned line = tile_index();
-  int64_t base, stride;
-  int kl = 0;
-  if constexpr (DIR == 0) {
-    const int j = line % G.ny;
-    kl = line / G.ny;
-    base = (int64_t)(hs + kl) * G.sz + (int64_t)(hs + j) * G.sy + hs;
-    stride = 1;
-  } else if constexpr (DIR == 1) {
-    const int i = line % G.nx;
-    kl = line / G.nx;
-    base = (int64_t)(hs + kl) * G.sz + (int64_t)hs * G.sy + hs + i;
-    stride = G.sy;
-  } else {
-    const int i = line % G.nx;
-    const int j = line / G.nx;
-    base = (int64_t)hs * G.sz + (int64_t)(hs + j) * G.sy + hs + i;
-    stride = G.sz;
-  }
-  double* s_st = sm;                 // [5][W]
-  double* s_q = s_st + 5 * W;        // [5 NGLL][n]: q0, then q0b
-  double* s_e = s_q + 5 * NGLL * n;  // [10][n]: eL|eR, then eLb|eRb, then stencil adjoints
-  double* s_k = s_e + 10 * n;        // [LINE_K]: background and power references of an x or y line
-  double* s_ao = s_k + LINE_K;       // [5][n]: adj_out along the line
+  const int lanes = cols * n;
+  // [lanes][5] each: a cell's five values at constant offsets from one address
+  double* s_st = sm;
+  double* s_ao = s_st + 5 * lanes;
+  double* s_e = s_ao + 5 * lanes;      // slots 0 .. 4
+  double* s_f = s_e + 5 * lanes;       // slots 5 .. 9
+  auto slot = [&](auto k, int cell5) -> double& {
+    if constexpr (k < 5) return s_e[cell5 + k];
+    else return s_f[cell5 + (k - 5)];
+  };
+  // lane -> line and cell c; the cells of a line are st5 doubles apart
+  const int t = threadIdx.x, t5 = 5 * t;
+  const int col = DIR == 0 ? t / n : t % cols;
+  const int c = DIR == 0 ? t - col * n : t / cols;
+  const int st5 = DIR == 0 ? 5 : 5 * cols;
+  const int nlines = (int)(ncell(G) / n);
+  const int line = (int)tile_index() * cols + col;
+  const bool on = t < lanes && line < nlines;
   const bool per = G.bc[DIR] == AWFL_BC_PERIODIC;
-  // background of cell c: the line's level for x and y (read from LDS, so
-  // that these per-line values live in vector registers only where they are
-  // used), the cell's own for z
-  auto bg_of = [&](int c) {
-    if constexpr (DIR == 2) {
-      return cell_bg<NGLL, DIR>(G, c);
-    } else {
-      CellBg<NGLL> bg{};
-      bg.r = s_k[0];
-      bg.rt = s_k[1];
-      bg.pt = PowRef{s_k[2], s_k[3], s_k[4], s_k[5]};
-      bg.wall_bot = bg.wall_top = false;
-      return bg;
-    }
-  };
-  auto fref_of = [&](int f) {
-    if constexpr (DIR == 2) {
-      return face_ref<DIR>(G, kl, f);
-    } else {
-      FaceRef fr;
-      fr.q5 = PowRef{s_k[2], s_k[3], s_k[4], s_k[5]};
-      fr.rt = DIR == 0 ? fr.q5 : PowRef{s_k[6], s_k[7], s_k[8], s_k[9]};
-      return fr;
-    }
-  };
-  // 1. stage the line (boundary rule at load), adj_out along it and an x or
-  // y line's constants.  Every global load of a thread is issued before its
-  // first LDS store, so the stage waits for memory once (each thread holds
-  // at most one halo cell, and one cell of the line when n <= bd).
-  {
-    const int t = threadIdx.x;
-    const bool halo = t < 2 * hs;
-    const int hc = t < hs ? t : n + t;  // padded slot of halo cell t
-    double hv[5];
-    if (halo) {
-      bool zn;
-      const int src = map_axis(hc - hs, n, per, zn);
-      sfor<5>([&](auto l) { hv[l] = (zn && l == NM) ? 0.0 : in[l * G.sl + base + src * stride]; });
-    }
-    double kv[LINE_K];
-    if constexpr (DIR != 2) {
-      if (t == 0) {
-        const CellBg<NGLL> bg = cell_bg<NGLL, DIR>(G, kl);
-        const FaceRef fr = face_ref<DIR>(G, kl, 0);
-        kv[0] = bg.r;
-        kv[1] = bg.rt;
-        kv[2] = bg.pt.h, kv[3] = bg.pt.l, kv[4] = bg.pt.rb, kv[5] = bg.pt.b;
-        kv[6] = fr.rt.h, kv[7] = fr.rt.l, kv[8] = fr.rt.rb, kv[9] = fr.rt.b;
-      }
-    }
-    for (int c = t; c < n; c += bd) {
-      double v[5], a[5];
-      sfor<5>([&](auto l) {
-        v[l] = in[l * G.sl + base + c * stride];
-        a[l] = adj_out[l * G.sl + base + c * stride];
-      });
-      sfor<5>([&](auto l) {
-        s_st[l * W + hs + c] = v[l];
-        s_ao[l * n + c] = a[l];
-      });
-    }
-    if (halo) sfor<5>([&](auto l) { s_st[l * W + hc] = hv[l]; });
-    if constexpr (DIR != 2) {
-      if (t == 0) sfor<LINE_K>([&](auto k) { s_k[k] = kv[k]; });
-    }
+  Pos p{0, 0, 0};
+  if (on) {
+    if constexpr (DIR == 0) p = Pos{c, line % G.ny, line / G.ny};
+    else if constexpr (DIR == 1) p = Pos{line % G.nx, c, line / G.nx};
+    else p = Pos{line % G.nx, line / G.nx, c};
   }
-  __syncthreads();
-  // 2. cell forward: WENO values (independent chains the scheduler
-  // interleaves: two variables at a time in x, all five in y and z, as
-  // measured fastest) and edge states
-  auto dow = [&](int l) { return (l == idR || l == idT) ? G.weno_s : G.weno_w; };
-  auto recon = [&](int c, int l0, auto nv) {
-    constexpr int NV = decltype(nv)::value;
-    double w[NV][ORD], g[NV][NGLL];
-    sfor<NV>([&](auto v) { sfor<ORD>([&](auto s) { w[v][s] = s_st[(l0 + v) * W + c + s]; }); });
-    bool all = true;
-    sfor<NV>([&](auto v) { all = all && dow(l0 + v); });
-    if (all) sfor<NV>([&](auto v) { reconstruct<ORD, NGLL>(w[v], true, g[v]); });
-    else sfor<NV>([&](auto v) { reconstruct<ORD, NGLL>(w[v], dow(l0 + v), g[v]); });
-    sfor<NV>([&](auto v) { sfor<NGLL>([&](auto ii) { s_q[((l0 + v) * NGLL + ii) * n + c] = g[v][ii]; }); });
-  };
-  for (int c = threadIdx.x; c < n; c += bd) {
-    if constexpr (DIR == 0) {
-#pragma unroll 1
-      for (int l0 = 0; l0 < 4; l0 += 2) recon(c, l0, std::integral_constant<int, 2>{});
-      recon(c, 4, std::integral_constant<int, 1>{});
-    } else {
-      recon(c, 0, std::integral_constant<int, 5>{});
-    }
-    double q0[5][NGLL], eL[5], eR[5], sa;
-    sfor<5>([&](auto l) { sfor<NGLL>([&](auto ii) { q0[l][ii] = s_q[(l * NGLL + ii) * n + c]; }); });
-    cell_transform<NGLL, DIR>(q0, bg_of(c), K, eL, eR, sa, [](const auto&, const auto&) {});
+  const int64_t o = sidx(G, 0, p);
+  if (on) {
+    double v[5], a[5];
     sfor<5>([&](auto l) {
-      s_e[l * n + c] = eL[l];
-      s_e[(5 + l) * n + c] = eR[l];
+      v[l] = in[l * G.sl + o];
+      a[l] = adj_out[l * G.sl + o];
+    });
+    sfor<5>([&](auto l) {
+      s_st[t5 + l] = v[l];
+      s_ao[t5 + l] = a[l];
+    });
+  }
+  // the stencil's cells: LDS offset of slot s, and the slots past a wall
+  int at[ORD];
+  unsigned clamped = 0;
+  sfor<ORD>([&](auto s) {
+    bool zn;
+    at[s] = on ? t5 + __mul24(st5, map_axis(c - hs + s, n, per, zn) - c) : 0;
+    if (on && zn) clamped |= 1u << s;
+  });
+  auto stencil = [&](int l, double (&u)[ORD]) {
+    sfor<ORD>([&](auto s) {
+      const double v = s_st[at[s] + l];
+      u[s] = l == NM && (clamped >> s & 1u) ? 0.0 : v;
+    });
+  };
+  auto dow = [&](int l) { return (l == idR || l == idT) ? G.weno_s : G.weno_w; };
+  __syncthreads();
+  // reconstruction, transform, edge states
+  double q[5][NGLL];
+  if (on) {
+    sfor<5>([&](auto l) {
+      double u[ORD];
+      stencil(l, u);
+      reconstruct<ORD, NGLL>(u, dow(l), q[l]);
+    });
+    double eL[5], eR[5], sa;
+    cell_transform<NGLL, DIR>(q, cell_bg<NGLL, DIR>(G, p.k), K, eL, eR, sa, [](const auto&, const auto&) {});
+    sfor<5>([&](auto l) {
+      s_e[t5 + l] = eL[l];
+      s_f[t5 + l] = eR[l];
     });
   }
   __syncthreads();
-  // 3. faces: flux adjoint -> edge-state adjoints, over the edge states.  A
-  // z line with walls has n + 1 faces for n threads: thread 0 takes both wall
-  // faces through the short wall form (riemann_adj_zwall), the others one
-  // interior face each, all in one pass.
+  // faces: flux adjoint -> edge-state adjoints, over the edge states.  A lane
+  // takes the face at its cell's low side; between walls the first takes both
+  // wall faces, whose reverse is short.
   const double cdr = K.dt * K.rd;
-  const bool zwall = DIR == 2 && !per;
-  const int nfaces = (per || zwall) ? n : n + 1;
-  for (int f = threadIdx.x; f < nfaces; f += bd) {
-    if (zwall && f == 0) {
+  if (on) {
+    if (!per && c == 0) {
       sfor<2>([&](auto side) {         // face 0, then face n
-        const int sl = side == 0 ? 0 : 5 * n + n - 1;            // the boundary cell's edge slot
-        const int ca = side == 0 ? 0 : n - 1;
+        const int e = side == 0 ? t5 : t5 + st5 * (n - 1);
+        double* es = side == 0 ? s_e : s_f;
         double L[5], Fb[5], Lb[5];
         sfor<5>([&](auto l) {
-          L[l] = s_e[sl + l * n];
-          const double v = side == 0 ? s_ao[l * n + ca] : -s_ao[l * n + ca];
-          Fb[l] = (G.sim2d && l == idV) ? 0.0 : cdr * v;
+          L[l] = es[e + l];
+          const double v = s_ao[e + l];
+          Fb[l] = (G.sim2d && l == idV) ? 0.0 : (side == 0 ? cdr : -cdr) * v;
           Lb[l] = 0.0;
         });
-        adj::riemann_adj_zwall(L, fref_of(side == 0 ? 0 : n), Fb, Lb);
-        sfor<5>([&](auto l) { s_e[sl + l * n] = Lb[l]; });
+        adj::wall_adj<DIR>(L, face_ref<DIR>(G, p.k, side == 0 ? 0 : n), Fb, Lb);
+        sfor<5>([&](auto l) { es[e + l] = Lb[l]; });
       });
-      continue;
-    }
-    const bool wl = !per && f == 0, wr = !per && f == n;
-    const int a = wl ? 0 : (f == 0 ? n - 1 : f - 1);      // cell on the low side
-    const int b = wr ? n - 1 : (f == n ? 0 : f);          // cell on the high side
-    // slots this face owns: the low cell's high edge and the high cell's
-    // low edge (at a wall, the one edge of the boundary cell)
-    const int sL = wl ? 0 : (5 * n + a);                  // + l * n
-    const int sR = wr ? (5 * n + n - 1) : b;
-    double L[5], R[5], Fb[5], Lb[5], Rb[5];
-    sfor<5>([&](auto l) {
-      L[l] = s_e[sL + l * n];
-      R[l] = s_e[sR + l * n];
-      double v = 0.0;
-      if (!wr) v += s_ao[l * n + b];
-      if (!wl) v -= s_ao[l * n + a];
-      Fb[l] = (G.sim2d && l == idV) ? 0.0 : cdr * v;
-      Lb[l] = Rb[l] = 0.0;
-    });
-    adj::riemann_adj<DIR>(L, R, fref_of(f), Fb, Lb, Rb);
-    if (wl || wr) {
-      sfor<5>([&](auto l) { s_e[sL + l * n] = Lb[l] + Rb[l]; });
     } else {
+      const int lo = t5 + (c == 0 ? st5 * (n - 1) : -st5);
+      double L[5], R[5], Fb[5], Lb[5], Rb[5];
       sfor<5>([&](auto l) {
-        s_e[sL + l * n] = Lb[l];
-        s_e[sR + l * n] = Rb[l];
+        L[l] = s_f[lo + l];
+        R[l] = s_e[t5 + l];
+        const double v = s_ao[t5 + l] - s_ao[lo + l];
+        Fb[l] = (G.sim2d && l == idV) ? 0.0 : cdr * v;
+        Lb[l] = Rb[l] = 0.0;
+      });
+      adj::riemann_adj<DIR>(L, R, face_ref<DIR>(G, p.k, c), Fb, Lb, Rb);
+      sfor<5>([&](auto l) {
+        s_f[lo + l] = Lb[l];
+        s_e[t5 + l] = Rb[l];
       });
     }
   }
   __syncthreads();
-  // 4a. transform reverse: q0b over q0 (each cell's own column); in z the
-  // source enters rho*w as out += dt * src
-  for (int c = threadIdx.x; c < n; c += bd) {
-    double q0[5][NGLL], q0b[5][NGLL], eLb[5], eRb[5];
+  // transform reverse; in z the source enters rho*w as out += dt * src
+  double qb[5][NGLL];
+  if (on) {
+    double eLb[5], eRb[5];
     sfor<5>([&](auto l) {
-      sfor<NGLL>([&](auto ii) { q0[l][ii] = s_q[(l * NGLL + ii) * n + c]; });
-      eLb[l] = s_e[l * n + c];
-      eRb[l] = s_e[(5 + l) * n + c];
+      eLb[l] = s_e[t5 + l];
+      eRb[l] = s_f[t5 + l];
     });
-    const double srcb = DIR == 2 ? K.dt * s_ao[idW * n + c] : 0.0;
-    adj::cell_dt_adj<NGLL, DIR>(q0, bg_of(c), K, eLb, eRb, srcb, q0b);
-    sfor<5>([&](auto l) { sfor<NGLL>([&](auto ii) { s_q[(l * NGLL + ii) * n + c] = q0b[l][ii]; }); });
+    const double srcb = DIR == 2 ? K.dt * s_ao[t5 + idW] : 0.0;
+    adj::cell_dt_adj<NGLL, DIR>(q, cell_bg<NGLL, DIR>(G, p.k), K, eLb, eRb, srcb, qb);
   }
-  // 4b. WENO reverse in each cell's own column, PV variables at a time side
-  // by side (independent chains the scheduler interleaves).  The stencil
-  // adjoints of every variable go to the row region [s_q | s_e] (5 NGLL + 10
-  // rows; adj_row), in rows that hold no q0b of a later group, so one
-  // barrier and one gather of the stencil adjoints that point at each cell
-  // finish the sweep.
-  static_assert(adj_rows_ok<ORD, NGLL, adj_pv<ORD>()>(), "stencil adjoints fit the row region");
-  constexpr int PV = adj_pv<ORD>();
-  double* s_r = s_q;
-  auto weno_rev = [&](auto l0c, auto nv) {
-    constexpr int l0 = decltype(l0c)::value;
-    constexpr int NV = decltype(nv)::value;
-    bool all = true;
-    sfor<NV>([&](auto v) { all = all && dow(l0 + v); });
-    for (int c = threadIdx.x; c < n; c += bd) {
-      double u[NV][ORD], ub[NV][ORD], gb[NV][NGLL];
+  // WENO reverse, PV variables at a time: stencil adjoints to the slots, then
+  // each cell gathers those that point at it.  Cell c - hs + s' holds it in
+  // slot ORD - 1 - s'; a wall drops what lies past it, and the cell at the wall
+  // collects the clamped slots (not of the normal momentum, zero there).
+  sfor<(5 + PV - 1) / PV>([&](auto g) {
+    constexpr int v0 = g * PV;
+    constexpr int NV = v0 + PV <= 5 ? PV : 5 - v0;
+    if constexpr (v0 > 0) __syncthreads();
+    if (on) {
+      double u[NV][ORD], ub[NV][ORD];
+      bool all = true;
       sfor<NV>([&](auto v) {
-        sfor<ORD>([&](auto s) {
-          u[v][s] = s_st[(l0 + v) * W + c + s];
-          ub[v][s] = 0.0;
-        });
-        sfor<NGLL>([&](auto ii) { gb[v][ii] = s_q[((l0 + v) * NGLL + ii) * n + c]; });
+        stencil(v0 + v, u[v]);
+        sfor<ORD>([&](auto s) { ub[v][s] = 0.0; });
+        all = all && dow(v0 + v);
       });
-      if (all) {
-        sfor<NV>([&](auto v) { adj::reconstruct_adj<ORD, NGLL>(u[v], true, gb[v], ub[v]); });
-      } else {
-        sfor<NV>([&](auto v) { adj::reconstruct_adj<ORD, NGLL>(u[v], dow(l0 + v), gb[v], ub[v]); });
-      }
-      sfor<NV>([&](auto v) {
-        sfor<ORD>([&](auto s) { s_r[adj_row<ORD, NGLL>(l0 + v, s) * n + c] = ub[v][s]; });
-      });
+      if (all) sfor<NV>([&](auto v) { adj::reconstruct_adj<ORD, NGLL>(u[v], true, qb[v0 + v], ub[v]); });
+      else sfor<NV>([&](auto v) { adj::reconstruct_adj<ORD, NGLL>(u[v], dow(v0 + v), qb[v0 + v], ub[v]); });
+      sfor<NV>([&](auto v) { sfor<ORD>([&](auto s) { slot(std::integral_constant<int, v * ORD + s>{}, t5) = ub[v][s]; }); });
     }
-  };
-  sfor<5 / PV>([&](auto g) { weno_rev(std::integral_constant<int, g * PV>{}, std::integral_constant<int, PV>{}); });
-  if constexpr (5 % PV != 0)
-    weno_rev(std::integral_constant<int, 5 - 5 % PV>{}, std::integral_constant<int, 5 % PV>{});
-  __syncthreads();
-  // src = c + hs - s is the cell whose stencil slot s is c: a periodic line
-  // wraps it (by one period when n >= hs, else by the remainder), a wall
-  // drops it when it falls outside the line.  At a wall the stencil slots
-  // past the end read the clamped end cell; the normal momentum there is
-  // zero, so it passes nothing back.
-  // MODE 0: periodic with n < hs (wrap by the remainder), 1: periodic with
-  // n >= hs (one period at most, every slot in the line), 2: walls
-  auto gather = [&](int l0, auto nv, auto mode) {
-    constexpr int NV = decltype(nv)::value;
-    constexpr int MODE = decltype(mode)::value;
-    for (int c = threadIdx.x; c < n; c += bd) {
+    __syncthreads();
+    if (on) {
       sfor<NV>([&](auto v) {
-        const int l = l0 + v;
-        double acc = s_ao[l * n + c];
-        sfor<ORD>([&](auto s) {
-          if constexpr (s == hs) {
-            acc += s_r[adj_row<ORD, NGLL>(l, s) * n + c];
-          } else {
-            int src = c + hs - s;
-            if constexpr (MODE == 0) {
-              src %= n;
-              src += src < 0 ? n : 0;
-            } else if constexpr (MODE == 1) {
-              src += src < 0 ? n : 0;
-              src -= src >= n ? n : 0;
-            }
-            if constexpr (MODE != 2) {
-              acc += s_r[adj_row<ORD, NGLL>(l, s) * n + src];
-            } else {
-              const bool ok = src >= 0 && src < n;
-              const double val = s_r[adj_row<ORD, NGLL>(l, s) * n + (ok ? src : c)];
-              acc += ok ? val : 0.0;
-            }
-          }
+        constexpr int l = v0 + v;
+        double acc = s_ao[t5 + l];
+        sfor<ORD>([&](auto sp) {
+          const double x = slot(std::integral_constant<int, v * ORD + ORD - 1 - sp>{}, at[sp]);
+          acc += (clamped >> sp & 1u) ? 0.0 : x;
         });
-        if (MODE == 2 && l != NM) {
-          if (c == 0)                    // slot s of cell cc reads index cc - hs + s < 0
+        if (l != NM && !per) {
+          if (c == 0)                  // slot s of cell cc reads index cc - hs + s < 0
             sfor<hs>([&](auto cc) {
               sfor<ORD>([&](auto s) {
                 if constexpr (cc - hs + s < 0) {
-                  if (cc < n) acc += s_r[adj_row<ORD, NGLL>(l, s) * n + cc];
+                  if (cc < n) acc += slot(std::integral_constant<int, v * ORD + s>{}, t5 + st5 * cc);
                 }
               });
             });
-          if (c == n - 1)                // slot s of cell n-1-m reads index >= n
+          if (c == n - 1)              // slot s of cell n-1-m reads index >= n
             sfor<hs>([&](auto m) {
-              const int cc = n - 1 - m;
               sfor<ORD>([&](auto s) {
                 if constexpr (s >= hs + 1 + m) {
-                  if (cc >= 0) acc += s_r[adj_row<ORD, NGLL>(l, s) * n + cc];
+                  if (n - 1 - m >= 0) acc += slot(std::integral_constant<int, v * ORD + s>{}, t5 - st5 * m);
                 }
               });
             });
         }
-        adj_in[l * G.sl + base + c * stride] = acc;
+        adj_in[l * G.sl + o] = acc;
       });
     }
-  };
-  if (!per) gather(0, std::integral_constant<int, 5>{}, std::integral_constant<int, 2>{});
-  else if (n < hs) gather(0, std::integral_constant<int, 5>{}, std::integral_constant<int, 0>{});
-  else gather(0, std::integral_constant<int, 5>{}, std::integral_constant<int, 1>{});
+  });
   // the halo cells of an x line (y and z halos: k_zero_halo)
   if constexpr (DIR == 0) {
-    for (int c = threadIdx.x; c < 2 * hs; c += bd) {
-      const int64_t o = c < hs ? base - hs + c : base + n + (c - hs);
-      sfor<5>([&](auto l) { adj_in[l * G.sl + o] = 0.0; });
+    if (on)
+      for (int h = c; h < 2 * hs; h += n) {
+        const int64_t oh = o - c + (h < hs ? h - hs : n + h - hs);
+        sfor<5>([&](auto l) { adj_in[l * G.sl + oh] = 0.0; });
+      }
+  }
+}
+
+// Lines per work-group, of at most four waves, one per SIMD (longer lines
+// alone): few idle lanes first, then whole groups of four, of which three fit a
+// CU and load its SIMDs alike; never so many that CUs stay without a group.
+// Against four waves, one, two and three took 1.10, 1.06 and 1.05 times as
+// long (128x128x64, z 143.8, 137.6 and 138.1 against 131.1 us; x and y by one
+// line of two waves 127.9 and 139.8, by two 123.1 and 127.6), five to eight
+// 1.09 to 1.4 times (100x90x75, x in 500 lanes 106 against 97 us).
+inline int adj_cols(int n, int64_t lines) {
+  constexpr double slack[5] = {0, 1.10, 1.06, 1.05, 1.0};
+  int best = 1;
+  double cost = 1e300;
+  for (int m = 1; m * n <= 256 && (m == 1 || (lines + m - 1) / m >= 256); m++) {
+    const int waves = (m * n + 63) / 64;
+    const double e = slack[waves] * waves / m;
+    if (e < cost) {
+      cost = e;
+      best = m;
     }
   }
+  return best;
 }
 
 // zero the halo of a padded array, one thread per halo cell: the 2hs z
@@ -855,8 +737,7 @@ struct VariantA {
   void (*weno[3])(const double*, const double*, Grid, double*);
   void (*gather[3])(const double*, const double*, Grid, double*);
   void (*tlm[3])(const double*, const double*, const double*, const double*, Grid, SweepK, double*, double*);
-  void (*line[3])(const double*, const double*, double*, Grid, SweepK);
-  int line_rows;
+  void (*tile[3])(const double*, const double*, double*, Grid, SweepK, int);
 };
 
 #define AWFL_VARIANT_A(O, N)                                                                        \
@@ -868,7 +749,7 @@ struct VariantA {
         {k_weno_adj<O, N, 0>, k_weno_adj<O, N, 1>, k_weno_adj<O, N, 2>},                            \
         {k_gather<O, 0>, k_gather<O, 1>, k_gather<O, 2>},                                           \
         {k_tlm_update<N, 0>, k_tlm_update<N, 1>, k_tlm_update<N, 2>},                               \
-        {k_adj_line<O, N, 0>, k_adj_line<O, N, 1>, k_adj_line<O, N, 2>}, adj_line_rows<O, N>(),       \
+        {k_adj_tile<O, N, 0>, k_adj_tile<O, N, 1>, k_adj_tile<O, N, 2>},                              \
   }
 
 const VariantA kVariantsA[] = {AWFL_VARIANT_A(3, 2), AWFL_VARIANT_A(5, 3)};
@@ -885,8 +766,8 @@ int check_variant(awfl_ctx* c) {
   return AWFL_OK;
 }
 
-// per-cell scratch of the multi-kernel sweeps (tangent; adjoint lines too
-// long for LDS)
+// per-cell scratch of the multi-kernel sweeps (tangent; adjoint lines of more
+// than ADJ_MAX cells)
 int ensure_cell_scratch(awfl_ctx* c) {
   int rc = check_variant(c);
   if (rc != AWFL_OK) return rc;
@@ -902,14 +783,6 @@ int ensure_tmp(awfl_ctx* c) {
   if (rc != AWFL_OK) return rc;
   if (!c->a_tmp) HIP_TRY(c, hipMalloc(&c->a_tmp, sizeof(double) * c->state_elems()));
   return AWFL_OK;
-}
-
-// LDS bytes of the fused line kernel along dir (0 if it does not fit)
-size_t line_lds(const awfl_ctx* c, const VariantA* v, int dir) {
-  const int n = dir == 0 ? c->cfg.nx : dir == 1 ? c->cfg.ny : c->cfg.nz;
-  // state line, row regions, line constants, adj_out along the line
-  const size_t b = sizeof(double) * (size_t)(5 * (n + 2 * c->hs) + v->line_rows * n + LINE_K + 5 * n);
-  return b <= 160 * 1024 ? b : 0;
 }
 
 // launch shapes: cells (ceil(nx/64), ny, nz), (cell, variable) pairs
@@ -938,13 +811,14 @@ int sweep_adjoint(awfl_ctx* c, const double* in, const double* adj_out, double* 
   const SweepK K = sweep_constants(c, dt, dir);
   const int64_t nc = (int64_t)c->cfg.nx * c->cfg.ny * c->cfg.nz;
   const int ng = c->cfg.ngll;
-  if (const size_t lds = line_lds(c, v, dir)) {
-    const int n = dir == 0 ? c->cfg.nx : dir == 1 ? c->cfg.ny : c->cfg.nz;
-    const unsigned lines = (unsigned)(nc / n);
+  if (const int n = dir == 0 ? c->cfg.nx : dir == 1 ? c->cfg.ny : c->cfg.nz; n <= ADJ_MAX) {
+    const int64_t lines = nc / n;
+    const int cols = adj_cols(n, lines);
+    const size_t lds = sizeof(double) * ADJ_SLOTS * cols * n;
     if (lds > 64 * 1024)
-      HIP_TRY(c, hipFuncSetAttribute((const void*)v->line[dir], hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    const int threads = line_threads(n);
-    v->line[dir]<<<lines, threads, lds, c->stream>>>(in, adj_out, adj_in, G, K);
+      HIP_TRY(c, hipFuncSetAttribute((const void*)v->tile[dir], hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    v->tile[dir]<<<(unsigned)((lines + cols - 1) / cols), (cols * n + 63) / 64 * 64, lds, c->stream>>>(
+        in, adj_out, adj_in, G, K, cols);
     LAUNCH_CHECK(c);
     if (zero_halo) {
       const int64_t nh = halo_cells(G, dir != 0);

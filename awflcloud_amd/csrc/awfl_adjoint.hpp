@@ -362,18 +362,24 @@ AWFL_HD void riemann_adj(const double (&L)[5], const double (&R)[5], const FaceR
   }
 }
 
-// Lb += (dF(L, L) / dL)^T Fb at a solid z wall, whose face takes both sides
-// from the boundary cell's edge state L (S:1577-1578) and where the wall rows
-// of the transform make the normal momentum L[idW] zero.  A consistent flux
-// of two equal states is the physical flux (rho w, rho u w, rho v w,
-// rho w^2 + p, rho theta w) / rho of L, whose derivative at rho w = 0 is
-// nonzero only in d(rho w) and in dp/d(rho theta) = gamma p / (rho theta):
-// the same derivative riemann_adj forms term by term, in a few operations.
-AWFL_HD void riemann_adj_zwall(const double (&L)[5], const FaceRef& fr, const double (&Fb)[5], double (&Lb)[5]) {
-  const double iL = rcp(L[0]);
+// Lb += (dF(L, L) / dL)^T Fb at a wall, whose face takes both sides from the
+// boundary cell's edge state L (S:822-823, 1577-1578).  A consistent flux of
+// two equal states is the physical flux of L (wall_flux), whose derivative
+// riemann_adj forms term by term; here it takes a few operations.
+template <int DIR>
+AWFL_HD void wall_adj(const double (&L)[5], const FaceRef& fr, const double (&Fb)[5], double (&Lb)[5]) {
+  constexpr int NM = 1 + DIR;
+  constexpr int T1 = DIR == 0 ? 2 : 1;
+  constexpr int T2 = DIR == 2 ? 2 : 3;
+  const double z = rcp(L[0] * L[4]), iL = z * L[4];
+  const double un = L[NM] * iL;
   const double p5 = C0 * pow_at(L[4], fr.q5);
-  Lb[idW] += Fb[0] + (Fb[idU] * L[idU] + Fb[idV] * L[idV] + Fb[idT] * L[idT]) * iL;
-  Lb[idT] += Fb[idW] * GAMMA * p5 * rcp(L[4]);
+  const double xb = fma(Fb[NM], L[NM], fma(Fb[T1], L[T1], fma(Fb[T2], L[T2], Fb[4] * L[4])));   // un's adjoint
+  Lb[0] -= xb * un * iL;
+  Lb[NM] += Fb[0] + fma(Fb[NM], un, xb * iL);
+  Lb[T1] += Fb[T1] * un;
+  Lb[T2] += Fb[T2] * un;
+  Lb[4] += fma(Fb[4], un, Fb[NM] * GAMMA * p5 * (z * L[0]));
 }
 
 // tvb * d tv_eval<N>(a) / da, accumulated into ab
@@ -694,7 +700,10 @@ AWFL_HD void gll_deriv_t(const double (&d)[NGLL], double (&Fb)[NGLL]) {
 // transform stage with the statements and names of cell_transform
 // (awfl_cell.hpp), whose levels it recomputes from the GLL values q0.  The last
 // level is linear in the fluxes of the level before and is never formed, and
-// 1/r and 1/(r t) pass their adjoints on where they are used.
+// 1/r and 1/(r t) pass their adjoints on where they are used.  The two
+// transverse momenta are carried by the velocity and act on nothing else, so
+// each is transformed and reversed by itself, ahead of the others: its levels
+// and those of the other variables' adjoints are never held together.
 template <int NGLL, int DIR>
 AWFL_HD void cell_dt_adj(const double (&q0)[5][NGLL], const CellBg<NGLL>& bg, const SweepK& K,
                          const double (&eLb)[5], const double (&eRb)[5], double srcb, double (&q0b)[5][NGLL]) {
@@ -702,6 +711,8 @@ AWFL_HD void cell_dt_adj(const double (&q0)[5][NGLL], const CellBg<NGLL>& bg, co
   constexpr int NM = 1 + DIR;
   constexpr int NL = NA - 1;           // levels formed
   constexpr int E = NGLL - 1;          // the high edge
+  constexpr int T1 = DIR == 0 ? 2 : 1;
+  constexpr int T2 = DIR == 2 ? 2 : 3;
   double q[5][NL][NGLL], u[NL][NGLL], g[NL][NGLL], rr[NGLL], rrt[NGLL];
   // levels 0 .. NA-2
   sfor<5>([&](auto l) { sfor<NGLL>([&](auto ii) { q[l][0][ii] = q0[l][ii]; }); });
@@ -723,32 +734,37 @@ AWFL_HD void cell_dt_adj(const double (&q0)[5][NGLL], const CellBg<NGLL>& bg, co
     rrt[ii] = r * z;
     u[0][ii] = q[NM][0][ii] * rr[ii];
   });
+  // q[l][kt + 1] from the levels up to kt
+  auto next_level = [&](auto l, auto kt) {
+    constexpr double rkt1 = 1.0 / (kt + 1.0);
+    double F[NGLL], d[NGLL];
+    sfor<NGLL>([&](auto s) {
+      if constexpr (l == idR) {
+        F[s] = q[NM][kt][s];
+      } else {
+        double t = 0.0;
+        if constexpr (l == NM) {
+          if constexpr (kt == 0) t = DIR == 2 ? fma(C0, g[kt][s], -bg.pG[s]) : C0 * g[kt][s];
+          else t = (0.5 * C0) * g[kt][s];
+          t = fma(u[0][s], q[l][kt][s], t);
+        } else {
+          t = u[0][s] * q[l][kt][s];
+        }
+        sfor<kt>([&](auto j) { t = fma(u[j + 1][s], q[l][kt - 1 - j][s], t); });
+        F[s] = t;
+      }
+    });
+    gll_deriv<NGLL>(F, K.ndt[kt], d);
+    sfor<NGLL>([&](auto ii) {
+      if constexpr (DIR == 2 && l == idW) d[ii] = kt == 0 ? d[ii] + sv : fma(-GRAV * rkt1, q[idR][kt][ii], d[ii]);
+      q[l][kt + 1][ii] = d[ii];
+    });
+  };
   sfor<NL - 1>([&](auto kt) {
     constexpr double rkt1 = 1.0 / (kt + 1.0);
-    sfor<5>([&](auto l) {
-      double F[NGLL], d[NGLL];
-      sfor<NGLL>([&](auto s) {
-        if constexpr (l == idR) {
-          F[s] = q[NM][kt][s];
-        } else {
-          double t = 0.0;
-          if constexpr (l == NM) {
-            if constexpr (kt == 0) t = DIR == 2 ? fma(C0, g[kt][s], -bg.pG[s]) : C0 * g[kt][s];
-            else t = (0.5 * C0) * g[kt][s];
-            t = fma(u[0][s], q[l][kt][s], t);
-          } else {
-            t = u[0][s] * q[l][kt][s];
-          }
-          sfor<kt>([&](auto j) { t = fma(u[j + 1][s], q[l][kt - 1 - j][s], t); });
-          F[s] = t;
-        }
-      });
-      gll_deriv<NGLL>(F, K.ndt[kt], d);
-      sfor<NGLL>([&](auto ii) {
-        if constexpr (DIR == 2 && l == idW) d[ii] = kt == 0 ? d[ii] + sv : fma(-GRAV * rkt1, q[idR][kt][ii], d[ii]);
-        q[l][kt + 1][ii] = d[ii];
-      });
-    });
+    next_level(std::integral_constant<int, idR>{}, kt);
+    next_level(std::integral_constant<int, NM>{}, kt);
+    next_level(std::integral_constant<int, idT>{}, kt);
     if constexpr (DIR == 2) {
       if (bg.wall_top) q[idW][kt + 1][E] = 0.0;
       if (bg.wall_bot) q[idW][kt + 1][0] = 0.0;
@@ -771,7 +787,7 @@ AWFL_HD void cell_dt_adj(const double (&q0)[5][NGLL], const CellBg<NGLL>& bg, co
   // wall every level of the normal momentum is zero there)
   double qb[5][NL][NGLL], ub[NL][NGLL], gb[NL][NGLL];
   double lb[5], hb[5], svb = 0.0;      // low- and high-edge adjoints
-  sfor<5>([&](auto l) {
+  auto averages = [&](auto l) {
     lb[l] = eLb[l];
     hb[l] = eRb[l];
     if constexpr (DIR == 2 && l == idW) {
@@ -784,8 +800,43 @@ AWFL_HD void cell_dt_adj(const double (&q0)[5][NGLL], const CellBg<NGLL>& bg, co
       qb[l][k][0] = w * lb[l];
       qb[l][k][E] = w * hb[l];
     });
-  });
+  };
+  // the reverse of the fluxes at level kt behind q[l][kt + 1]
+  auto flux_rev = [&](auto l, auto kt) {
+    constexpr bool last = kt + 2 == NA;
+    double d[NGLL], Fb[NGLL];
+    if constexpr (last) {
+      const double w = K.ndt[kt] * K.tav[kt + 1];
+      sfor<NGLL>([&](auto ii) { d[ii] = 0.0; });
+      d[0] = w * lb[l];
+      d[E] = w * hb[l];
+    } else {
+      sfor<NGLL>([&](auto ii) { d[ii] = K.ndt[kt] * qb[l][kt + 1][ii]; });
+    }
+    gll_deriv_t<NGLL>(d, Fb);
+    sfor<NGLL>([&](auto s) {
+      if constexpr (l == idR) {
+        qb[NM][kt][s] += Fb[s];
+      } else {
+        sfor<kt + 1>([&](auto j) {
+          ub[j][s] = fma(Fb[s], q[l][kt - j][s], ub[j][s]);
+          qb[l][kt - j][s] = fma(Fb[s], u[j][s], qb[l][kt - j][s]);
+        });
+        if constexpr (l == NM) gb[kt][s] = fma(Fb[s], kt == 0 ? C0 : 0.5 * C0, gb[kt][s]);
+      }
+    });
+  };
   sfor<NL>([&](auto k) { sfor<NGLL>([&](auto ii) { ub[k][ii] = gb[k][ii] = 0.0; }); });
+  auto transverse = [&](auto l) {
+    averages(l);
+    sfor<NL - 1>([&](auto kt) { next_level(l, kt); });
+    sfor<NA - 1>([&](auto km) { flux_rev(l, std::integral_constant<int, NA - 2 - km>{}); });
+  };
+  transverse(std::integral_constant<int, T1>{});
+  transverse(std::integral_constant<int, T2>{});
+  averages(std::integral_constant<int, idR>{});
+  averages(std::integral_constant<int, NM>{});
+  averages(std::integral_constant<int, idT>{});
   if constexpr (DIR == 2) svb = srcb;
   sfor<NA - 1>([&](auto km) {
     constexpr int kt = NA - 2 - km;
@@ -834,28 +885,10 @@ AWFL_HD void cell_dt_adj(const double (&q0)[5][NGLL], const CellBg<NGLL>& bg, co
       qb[NM][kt][E] += s;
       qb[NM][kt][0] -= s;
     }
-    sfor<5>([&](auto l) {
-      double d[NGLL], Fb[NGLL];
-      if constexpr (last) {
-        sfor<NGLL>([&](auto ii) { d[ii] = 0.0; });
-        d[0] = (ndt * tav) * lb[l];
-        d[E] = (ndt * tav) * hb[l];
-      } else {
-        sfor<NGLL>([&](auto ii) { d[ii] = ndt * qb[l][kt + 1][ii]; });
-      }
-      gll_deriv_t<NGLL>(d, Fb);
-      sfor<NGLL>([&](auto s) {
-        if constexpr (l == idR) {
-          qb[NM][kt][s] += Fb[s];
-        } else {
-          sfor<kt + 1>([&](auto j) {
-            ub[j][s] = fma(Fb[s], q[l][kt - j][s], ub[j][s]);
-            qb[l][kt - j][s] = fma(Fb[s], u[j][s], qb[l][kt - j][s]);
-          });
-          if constexpr (l == NM) gb[kt][s] = fma(Fb[s], kt == 0 ? C0 : 0.5 * C0, gb[kt][s]);
-        }
-      });
-    });
+    const std::integral_constant<int, kt> k{};
+    flux_rev(std::integral_constant<int, idR>{}, k);
+    flux_rev(std::integral_constant<int, NM>{}, k);
+    flux_rev(std::integral_constant<int, idT>{}, k);
   });
   // level 0
   if constexpr (DIR == 2) qb[idR][0][E] -= svb * GRAV;

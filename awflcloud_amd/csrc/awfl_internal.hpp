@@ -53,12 +53,8 @@ using awfl_detail::Grid;
 // ---------------------------------------------------------------------------
 constexpr unsigned AWFL_NUM_XCD = 8;
 
-// Threads of a line work-group: the line rounded up to whole waves, at most
-// 256.  The adjoint line kernel also uses it in place of blockDim.x, which
-// reaches a kernel through a memory load that the work-group's first loop
-// would wait for (measured 1-2% faster there; no gain in the forward line
-// kernels).
-__host__ __device__ constexpr int line_threads(int n) { return n < 256 ? (n + 63) / 64 * 64 : 256; }
+// Threads of a line work-group: the line rounded up to whole waves, at most 256.
+constexpr int line_threads(int n) { return n < 256 ? (n + 63) / 64 * 64 : 256; }
 
 __device__ __forceinline__ unsigned tile_index() {
   const unsigned n = gridDim.x * gridDim.y * gridDim.z;
