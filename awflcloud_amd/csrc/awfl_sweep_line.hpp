@@ -13,13 +13,13 @@
 //      a. WENO, one lane per (cell, variable): the ORD-cell stencil -> NGLL
 //         GLL values (WenoLimiter.h:93-172, S:1800-1833) into LDS;
 //      b. the differential transform, one lane per (cell, GLL point): each
-//         lane carries its point's levels of the 5 variables and the 4
-//         fluxes, the derivative across the cell's points (S:1863-1882 and
-//         analogues) reads the NGLL lanes' flux values from LDS, the
-//         products (S:1885-1915) and the z source (S:2049-2055) are
-//         pointwise; the edge lanes form the time-averaged edge states
-//         (S:2142-2177), the z source is averaged at every point and summed
-//         with the GLL weights (S:1489-1497);
+//         lane carries its point's levels of the 5 variables and the normal
+//         velocity's Taylor coefficients, the derivative across the cell's
+//         points (S:1863-1882 and analogues) reads the NGLL lanes' flux values
+//         from LDS, the products (S:1885-1915) and the z source (S:2049-2055)
+//         are pointwise; the edge lanes form the time-averaged edge states
+//         (S:2142-2177), the first one also the z source's average
+//         (S:1489-1497);
 //      the NGLL lanes of a cell sit in one wave (12 cells per wave, 4 lanes
 //      idle), so their exchanges need no work-group barrier;
 //   3. one lane per face: the Riemann flux (S:842-887, 1202-1245, 1583-1629)
@@ -28,8 +28,11 @@
 //   4. one lane per cell: the flux difference and the update (S:940-956,
 //      1298-1310, 1680-1696; T:63-65), or the tendency alone.
 // The arithmetic is the production kernels' (reconstruct, riemann and the
-// transform's statements in their order), so results agree with them to
-// rounding.
+// transform's statements), so results agree with them to rounding.
+//
+// Bound by FP64 issue.  At 192x192x96 the x, y and z sweeps took 788, 833 and
+// 958 us with three-way LDS bank conflicts in the exchange and every flux
+// product carried through the levels, 669, 698 and 944 us with neither.
 #pragma once
 #include "awfl_cell.hpp"
 #include "awfl_internal.hpp"
@@ -58,11 +61,12 @@ __device__ __forceinline__ void wave_lds_sync() {
 }
 
 // LDS of one line of n cells: staged line (reused for the face fluxes), GLL
-// values / flux exchange of a chunk, the source value of each chunk cell's
-// last GLL point, edge states, z source averages (and, in place, the face
-// fluxes apart from the line)
+// values / flux exchange of a chunk (a variable's points of a cell side by side,
+// so that a wave's 60 lanes touch 60 consecutive doubles: rows of points cost
+// three-way bank conflicts), edge states, z source averages (and, in place, the
+// face fluxes apart from the line)
 inline size_t line_lds_doubles(int n, int hs, int ngll, bool inplace = false) {
-  return (size_t)5 * (n + 2 * hs) + (size_t)5 * ngll * LS_CHUNK + LS_CHUNK + (size_t)10 * n + n +
+  return (size_t)5 * (n + 2 * hs) + (size_t)5 * ngll * LS_CHUNK + (size_t)10 * n + n +
          (inplace ? (size_t)5 * (n + 1) : 0);
 }
 
@@ -72,9 +76,11 @@ inline size_t line_lds_doubles(int n, int hs, int ngll, bool inplace = false) {
 template <int ORD, int NGLL, int DIR, bool TEND, bool INPLACE = false>
 __global__ __launch_bounds__(LS_THREADS) __attribute__((amdgpu_waves_per_eu(AWFL_LS_WAVES))) void k_sweep_line(const double* __restrict__ in, double* __restrict__ out,
                                                            Grid G, SweepK K) {
+  AWFL_NO_CONTRACT
   constexpr int hs = (ORD - 1) / 2;
   constexpr int NA = NGLL;
   constexpr int NM = 1 + DIR;
+  constexpr int XR = NGLL * LS_CHUNK;                  // exchange rows of one variable
   static_assert(NGLL * LS_CELLS_PER_WAVE <= 64, "a cell's GLL lanes must share a wave");
   extern __shared__ double sm[];
   const int n = DIR == 0 ? G.nx : DIR == 1 ? G.ny : G.nz;
@@ -100,9 +106,8 @@ __global__ __launch_bounds__(LS_THREADS) __attribute__((amdgpu_waves_per_eu(AWFL
     stride = G.sz;
   }
   double* s_st = sm;                                   // [5][W]; then face fluxes [5][n+1]
-  double* s_x = s_st + 5 * W;                          // [5 NGLL][CHUNK]: GLL values, then flux exchange
-  double* s_sv = s_x + 5 * NGLL * LS_CHUNK;            // [CHUNK]
-  double* s_e = s_sv + LS_CHUNK;                       // [10][n]: eL | eR
+  double* s_x = s_st + 5 * W;                          // [5][CHUNK][NGLL]: GLL values, then flux exchange
+  double* s_e = s_x + 5 * XR;                          // [10][n]: eL | eR
   double* s_src = s_e + 10 * n;                        // [n]: z source averages
   double* s_F = INPLACE ? s_src + n : sm;               // [5][n+1]
   const bool per = G.bc[DIR] == AWFL_BC_PERIODIC;
@@ -147,7 +152,7 @@ __global__ __launch_bounds__(LS_THREADS) __attribute__((amdgpu_waves_per_eu(AWFL
         sfor<ORD>([&](auto s) { u[s] = s_st[v * W + c0 + cl + s]; });
         const bool dw = (v == idR || v == idT) ? G.weno_s : G.weno_w;
         reconstruct<ORD, NGLL>(u, dw, gv);
-        sfor<NGLL>([&](auto p) { s_x[(v * NGLL + p) * LS_CHUNK + cl] = gv[p]; });
+        sfor<NGLL>([&](auto p) { s_x[v * XR + cl * NGLL + p] = gv[p]; });
       }
     }
     __syncthreads();
@@ -155,28 +160,27 @@ __global__ __launch_bounds__(LS_THREADS) __attribute__((amdgpu_waves_per_eu(AWFL
     const int cl = cl_t;
     const int c = c0 + cl;
     const bool act = lane_ok && cl < cnt;
-    // LDS slot of this lane's cell: an idle lane reads the last cell's
+    // LDS slots of this lane's cell: an idle lane reads the last cell's
     // values and stores nothing
-    const int clr = min(cl, LS_CHUNK - 1);
+    const double* xc = s_x + min(cl, LS_CHUNK - 1) * NGLL;
+    double* xw = s_x + min(cl, LS_CHUNK - 1) * NGLL + ii;
     const int kc = DIR == 2 ? min(c, n - 1) : kl;       // level of the cell's background
-    double q[5][NA], f[4][NA], g[NA];
-    double src0 = 0.0;                                  // z: the source at level 0 (Q2 broadcast)
-    // z gravity source at level kt: the level-0 value, then -rho_kt g (S:2055),
-    // formed where it is used rather than kept
-    auto src = [&](auto kt) -> double {
-      if constexpr (kt == 0) return src0;
-      else return -q[idR][kt] * GRAV;
-    };
-    double rr = 1.0, rrt = 1.0;
+    // levels 0 .. NA-2, the normal velocity's Taylor coefficients u (the flux of
+    // l is sum_j u_j q_l,k-j; cell_transform in awfl_cell.hpp) and (r t)^gamma
+    double q[5][NA], u[NA], g[NA], e[5];
+    double sv = 0.0, sa = 0.0, rr, rrt;
     {
       double q0[5];
-      sfor<5>([&](auto l) { q0[l] = s_x[(l * NGLL + ii) * LS_CHUNK + clr]; });
+      sfor<5>([&](auto l) { q0[l] = xw[l * XR]; });
       double brho, brt;
       PowRef pr;
       if constexpr (DIR == 2) {
         brho = G.hyDensGLL[kc * NGLL + ii];
         brt = G.hyDensThetaGLL[kc * NGLL + ii];
         pr = G.prG[kc * NGLL + ii];
+        // S:1439 assigns a scalar to the whole SArray: every entry of the
+        // source holds the value of the last GLL point
+        sa = sv = -GRAV * xc[idR * XR + NGLL - 1];
       } else {
         brho = G.hyDensCells[hs + kl];
         brt = G.hyDensThetaCells[hs + kl];
@@ -195,100 +199,69 @@ __global__ __launch_bounds__(LS_THREADS) __attribute__((amdgpu_waves_per_eu(AWFL
         q[idR][0] = 1.0;
         q[idT][0] = 300.0;
       }
-      const double r = q[idR][0];
-      rr = rcp(r);
-      double vel[5];
-      sfor<4>([&](auto m) { vel[m + 1] = q[m + 1][0] * rr; });
-      sfor<4>([&](auto m) { f[m][0] = r * vel[NM] * vel[m + 1]; });
+      const double z = rcp(q[idR][0] * q[idT][0]);
+      rr = q[idT][0] * z;
+      rrt = q[idR][0] * z;
+      u[0] = q[NM][0] * rr;
       g[0] = act ? pow_gamma_near(q[idT][0], et, pr.h, pr.l) : 1.0;
-      rrt = rcp(q[idT][0]);
-      if constexpr (DIR == 2) {
-        // S:1439 assigns a scalar to the whole SArray: every entry of the
-        // source holds the value of the last GLL point
-        const double sv = -(q[idR][0] - brho) * GRAV;
-        if (act && ii == NGLL - 1) s_sv[cl] = sv;
-        wave_lds_sync();
-        const double svl = s_sv[clr];
-        src0 = svl;
-      }
     }
+    sfor<5>([&](auto l) { e[l] = q[l][0]; });
     sfor<NA - 1>([&](auto kt) {
       constexpr double rkt1 = 1.0 / (kt + 1.0);
+      const double ndt = K.ndt[kt], tav = K.tav[kt + 1];
       // this point's five flux values at level kt into the exchange rows
       double Fl[5];
-      Fl[0] = q[NM][kt];
+      Fl[idR] = q[NM][kt];
       sfor<4>([&](auto m) {
         constexpr int l = m + 1;
+        double t;
         if constexpr (l == NM) {
-          if constexpr (kt == 0) {
-            if constexpr (DIR == 2) Fl[l] = f[m][kt] + C0 * g[kt] - G.hyPressureGLL[kc * NGLL + ii];
-            else Fl[l] = f[m][kt] + C0 * g[kt];
-          } else {
-            Fl[l] = f[m][kt] + (0.5 * C0) * g[kt];
-          }
+          if constexpr (kt == 0) t = DIR == 2 ? fm(C0, g[kt], -G.hyPressureGLL[kc * NGLL + ii]) : C0 * g[kt];
+          else t = (0.5 * C0) * g[kt];
+          t = fm(u[0], q[l][kt], t);
         } else {
-          Fl[l] = f[m][kt];
+          t = u[0] * q[l][kt];
         }
+        sfor<kt>([&](auto j) { t = fm(u[j + 1], q[l][kt - 1 - j], t); });
+        Fl[l] = t;
       });
       wave_lds_sync();                                  // the cell's lanes are done with the previous rows
-      if (act) sfor<5>([&](auto l) { s_x[(l * NGLL + ii) * LS_CHUNK + cl] = Fl[l]; });
+      if (act) sfor<5>([&](auto l) { xw[l * XR] = Fl[l]; });
       wave_lds_sync();
-      double d[5];
       sfor<5>([&](auto l) {
-        double t = -0.0;
-        sfor<NGLL>([&](auto s) { t += Dc[s] * s_x[(l * NGLL + s) * LS_CHUNK + clr]; });
-        d[l] = t;
-      });
-      const double ndt = K.ndt[kt];
-      sfor<5>([&](auto l) {
-        if constexpr (DIR == 2 && l == idW) q[l][kt + 1] = d[l] * ndt + src(kt) * rkt1;
-        else q[l][kt + 1] = d[l] * ndt;
+        double x[NGLL];
+        sfor<NGLL>([&](auto s) { x[s] = xc[l * XR + s]; });
+        double t = Dc[0] * x[0];
+        sfor<NGLL - 1>([&](auto s) { t = fm(Dc[s + 1], x[s + 1], t); });
+        double v = t * ndt;
+        if constexpr (DIR == 2 && l == idW) v = kt == 0 ? v + sv : fm(-GRAV * rkt1, q[idR][kt], v);
+        q[l][kt + 1] = v;
+        // the source average takes the exact integral of d(rho)/dt (S:1462, 1489-1492)
+        if constexpr (DIR == 2 && l == idR) sa = fm(-GRAV * (tav * ndt), x[NGLL - 1] - x[0], sa);
       });
       if constexpr (DIR == 2) {                         // S:2051-2055
         if (!per && c == n - 1 && ii == NGLL - 1) q[idW][kt + 1] = 0.0;
         if (!per && c == 0 && ii == 0) q[idW][kt + 1] = 0.0;
       }
-      if constexpr (kt + 2 < NA) {                      // products at level kt+1
-        sfor<4>([&](auto m) {
-          constexpr int l = m + 1;
-          double tot = 0.0;
-          sfor<kt + 2>([&](auto ir) {
-            if constexpr (ir == 0) tot += q[NM][ir] * q[l][kt + 1 - ir];
-            else tot += q[NM][ir] * q[l][kt + 1 - ir] - q[idR][ir] * f[m][kt + 1 - ir];
-          });
-          f[m][kt + 1] = tot * rr;
-        });
+      sfor<5>([&](auto l) { e[l] = fm(q[l][kt + 1], tav, e[l]); });   // time averages (S:2142-2177)
+      if constexpr (kt + 2 < NA) {
+        double t = q[NM][kt + 1];
+        sfor<kt + 1>([&](auto j) { t = fm(-q[idR][j + 1], u[kt - j], t); });
+        u[kt + 1] = t * rr;
         double tg = 0.0;
         sfor<kt + 1>([&](auto ir) {
           constexpr double wgt = kt + 1.0 - ir;
-          if constexpr (ir == 0)
-            tg += wgt * (GAMMA * g[ir] * q[idT][kt + 1 - ir]);
-          else
-            tg += wgt * (GAMMA * g[ir] * q[idT][kt + 1 - ir] - q[idT][ir] * g[kt + 1 - ir]);
+          double p = (GAMMA * g[ir]) * q[idT][kt + 1 - ir];
+          if constexpr (ir > 0) p = fm(-q[idT][ir], g[kt + 1 - ir], p);
+          tg = fm(wgt, p, tg);
         });
-        g[kt + 1] = (GAMMA * g[0] * q[idT][kt + 1] + tg * rkt1) * rrt;
+        g[kt + 1] = fm(GAMMA * g[0], q[idT][kt + 1], tg * rkt1) * rrt;
       }
     });
-    // time-averaged edge states from the edge points (S:2142-2177)
-    if (act && (ii == 0 || ii == NGLL - 1)) {
+    if (act && (ii == 0 || ii == NGLL - 1)) {           // edge states, z source average
       const int row = ii == 0 ? 0 : 5;
-      sfor<5>([&](auto l) {
-        double a = q[l][0];
-        sfor<NA - 1>([&](auto km) { a += q[l][km + 1] * K.tav[km + 1]; });
-        s_e[(row + l) * n + c] = a;
-      });
-    }
-    if constexpr (DIR == 2) {                           // S:1462, 1489-1492
-      double s0 = src(std::integral_constant<int, 0>{});
-      sfor<NA - 1>([&](auto km) { s0 += src(std::integral_constant<int, km + 1>{}) * K.tav[km + 1]; });
-      wave_lds_sync();
-      if (act) s_x[ii * LS_CHUNK + cl] = s0 * Gll<NGLL>::wts[ii];
-      wave_lds_sync();
-      if (act && ii == 0) {
-        double sa = 0.0;
-        sfor<NGLL>([&](auto p) { sa += s_x[p * LS_CHUNK + cl]; });
-        s_src[c] = sa;
-      }
+      sfor<5>([&](auto l) { s_e[(row + l) * n + c] = e[l]; });
+      if (DIR == 2 && ii == 0) s_src[c] = sa;
     }
     __syncthreads();                                    // the next chunk rewrites s_x
   }
