@@ -15,8 +15,15 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # -fno-signed-zeros lets the compiler drop the addition of a zero-initialised
 # accumulator's first term (x + 0.0 is not x only for x = -0.0); no result
 # changes except the sign of an exact zero, which nothing here depends on.
+# -disable-machine-licm keeps the FP64 constants of a loop body as scalar moves
+# next to their use (the scalar unit issues them beside the vector unit) instead
+# of hoisting them out of the loop, which runs out of scalar registers, parks
+# them in vector registers and reads them back lane by lane: the WENO of the
+# WENO9 line kernels held 70 such vector instructions in 460.  Registers go from
+# 142 to 119 there, from 159 to 124 in the tracers' y walker and from 203 to 190
+# in the FP64 one.
 HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-signed-zeros",
-             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+             "-mllvm", "-disable-machine-licm", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 # translation units of libawfl_dycore.so: FP64 sweeps + ABI, FP32 perturbation form, adjoint,
 # alternative time integrators, tracers
 HIP_UNITS = ["awfl_dycore.hip", "awfl_pert.hip", "awfl_adjoint.hip", "awfl_splitting.hip", "awfl_tracers.hip"]
