@@ -20,12 +20,13 @@
 //   a positivity flux limiter for positive tracers (S:904-935);
 //   the flux-difference tendency, and the tracer masses multiplied back
 //   (S:948-955).
-// Here the x sweep runs one line per work-group with the line in LDS, state
-// and tracers together (k_sweep_tr), and the y and z sweeps run the walker
+// Here a sweep runs as a tile of whole lines, one lane per cell, state and
+// tracers together (k_tile_tr); y and z lines that suit it less run the walker
 // (k_walk_tr: four x-adjacent lines per work-group walked in 64-cell steps);
-// both run the production sweep's statements (cell_edges / riemann) for the
-// state, so the state they return is awfl_sweep's up to the compiler's
-// contraction choices in these kernels.
+// WENO9/ADER5, and x lines past a tile, run one line per work-group with the
+// line in LDS (k_sweep_tr).  All run the production sweep's statements
+// (cell_edges / riemann) for the state, so the state they return is
+// awfl_sweep's up to the compiler's contraction choices in these kernels.
 // Departures from the source text, where it cannot run as written:
 //   T1 the limiter forms every cell's reduction factor from the unlimited
 //      fluxes and then applies it to the faces it is upwind of; the
@@ -420,11 +421,312 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
 }
 
 // ---------------------------------------------------------------------------
+// The tracer tile: a work-group takes `cols` whole lines, one lane per cell.
+// A lane keeps its cell's low edge state and low face's flux in registers; LDS
+// holds what neighbours exchange, [row][5] for the state and [row][ts] for the
+// tracers (ts: their number made odd, against bank conflicts):
+//   s_st, s_tq   the cells with hs cells beyond either end: state, and mixing
+//                ratios (then the limiter's cell factors)
+//   s_e, s_te    one slot per face: the high edge of the cell below it, then
+//                in place its flux (its one lane reads and writes it)
+//   s_tl         the tracers' low edges
+// A periodic line's face 0 takes its left edge from the last slot and leaves
+// its flux in both.  The arithmetic is the line kernel's.
+//
+// Bound by FP64 issue.  107-124 registers allow 16 waves per CU and 19 doubles
+// of LDS per cell (3 tracers) leave room for them; the line kernel (25 doubles
+// and all of a cell's values through LDS) holds 12 and the walker, with its ring,
+// head, tail and carries, 12: x at 256x256x128 with 3 tracers 546 us against the
+// line kernel's 612, y and z 662 and 670 against the walker's 704 and 779; at
+// 128x128x64 with 5 tracers 86, 95 and 95 against 128, 148 and 177; at 64x64x32
+// 15 against 16, 22 and 35.
+// ---------------------------------------------------------------------------
+constexpr int TT_MAX = 1024;    // lanes of a work-group
+
+inline int tt_stride(int ntr) { return ntr | 1; }
+inline size_t tt_lds(int n, int cols, int hs, int ntr) {
+  const size_t ts = tt_stride(ntr);
+  return sizeof(double) * cols * ((5 + ts) * (n + 2 * hs) + (5 + 2 * ts) * (n + 1));
+}
+
+template <int ORD, int NGLL, int DIR, bool TEND>
+__global__ __launch_bounds__(TT_MAX) __attribute__((amdgpu_waves_per_eu(4))) void k_tile_tr(
+    const double* __restrict__ in, const double* __restrict__ tr_in, double* __restrict__ out,
+    double* __restrict__ tr_out, Grid G, SweepK K, int ntr, unsigned pos, int cols) {
+  constexpr int hs = (ORD - 1) / 2;
+  constexpr int NM = 1 + DIR;
+  constexpr int NA = NGLL;
+  extern __shared__ double sm[];
+  const int n = axis_n(G, DIR);
+  const int ts = ntr | 1;
+  const bool per = G.bc[DIR] == AWFL_BC_PERIODIC;
+  const int t = threadIdx.x;
+  const int col = DIR == 0 ? t / n : t % cols;
+  const int c = DIR == 0 ? t - col * n : t / cols;
+  const int nlines = DIR == 0 ? G.ny * G.nz : DIR == 1 ? G.nx * G.nz : G.nx * G.ny;
+  const int line0 = (int)tile_index() * cols;
+  const bool on = t < cols * n && line0 + col < nlines;
+  // first interior cell and level (x, y) of a line, stride along DIR
+  const int64_t stride = DIR == 0 ? 1 : DIR == 1 ? G.sy : G.sz;
+  auto line_at = [&](int line, int& k) -> int64_t {
+    if constexpr (DIR == 0) {
+      k = line / G.ny;
+      return (int64_t)(hs + k) * G.sz + (int64_t)(hs + line - k * G.ny) * G.sy + hs;
+    } else if constexpr (DIR == 1) {
+      k = line / G.nx;
+      return (int64_t)(hs + k) * G.sz + (int64_t)hs * G.sy + hs + (line - k * G.nx);
+    } else {
+      const int j = line / G.nx;
+      k = 0;
+      return (int64_t)hs * G.sz + (int64_t)(hs + j) * G.sy + hs + (line - j * G.nx);
+    }
+  };
+  // LDS rows: padded cell p (from -hs), and face or cell p, of column cc
+  auto row_w = [&](int cc, int p) { return DIR == 0 ? cc * (n + 2 * hs) + p + hs : (p + hs) * cols + cc; };
+  auto row_f = [&](int cc, int p) { return DIR == 0 ? cc * (n + 1) + p : p * cols + cc; };
+  double* s_st = sm;
+  double* s_e = s_st + 5 * cols * (n + 2 * hs);
+  double* s_tq = s_e + 5 * cols * (n + 1);
+  double* s_te = s_tq + ts * cols * (n + 2 * hs);
+  double* s_tl = s_te + ts * cols * (n + 1);
+
+  // 1. stage: the state (normal momentum zero in wall ghosts) and the mixing
+  // ratios (ghosts copy the end cell at a wall) by the full density (S:624-626)
+  auto stage = [&](int cc, int pr, int src, bool zn) {
+    int k;
+    const int64_t o = line_at(line0 + cc, k) + src * stride;
+    double v[5];
+    sfor<5>([&](auto l) { v[l] = in[l * G.sl + o]; });
+    const double rr = rcp(v[idR] + G.hyDensCells[hs + (DIR == 2 ? src : k)]);
+    const int r = row_w(cc, pr);
+    sfor<5>([&](auto l) { s_st[5 * r + l] = (zn && l == NM) ? 0.0 : v[l]; });
+    for (int q = 0; q < ntr; q++) s_tq[ts * r + q] = tr_in[q * G.sl + o] * rr;
+  };
+  if (on) stage(col, c, c, false);
+  for (int h = t; h < 2 * hs * cols; h += blockDim.x) {
+    const int hc = DIR == 0 ? h / (2 * hs) : h % cols, hp = DIR == 0 ? h % (2 * hs) : h / cols;
+    if (line0 + hc < nlines) {
+      const int pr = hp < hs ? hp - hs : n + hp - hs;
+      bool zn;
+      const int src = wrap_axis(pr, n, per, zn);
+      stage(hc, pr, src, zn);
+    }
+  }
+  __syncthreads();
+
+  // 2. cells: edges of the state, then of each tracer from the density and the
+  // velocity coefficients of the state's transform
+  int kl = 0;
+  int64_t o = 0;
+  const int rw = row_w(col, c), rf = row_f(col, c), up_row = DIR == 0 ? 1 : cols;
+  double eL[5], src = 0.0;
+  if (on) {
+    o = line_at(line0 + col, kl) + c * stride;
+    CellBg<NGLL> bg{};
+    double st[5][ORD], eR[5];
+    double rl[NGLL], ul[NA - 1][NGLL];
+    sfor<5>([&](auto l) { sfor<ORD>([&](auto s) { st[l][s] = s_st[5 * (rw + (s - hs) * up_row) + l]; }); });
+    cell_edges_of<ORD, NGLL, DIR>(
+        st,
+        [&]() {
+          if constexpr (DIR == 2) {
+            sfor<NGLL>([&](auto ii) {
+              bg.rG[ii] = G.hyDensGLL[c * NGLL + ii];
+              bg.rtG[ii] = G.hyDensThetaGLL[c * NGLL + ii];
+              bg.pG[ii] = G.hyPressureGLL[c * NGLL + ii];
+              bg.ptG[ii] = G.prG[c * NGLL + ii];
+            });
+            bg.wall_bot = !per && c == 0;
+            bg.wall_top = !per && c == n - 1;
+          } else {
+            bg.r = G.hyDensCells[hs + kl];
+            bg.rt = G.hyDensThetaCells[hs + kl];
+            bg.pt = G.prT[kl];
+            bg.wall_bot = bg.wall_top = false;
+          }
+          return bg;
+        },
+        G.weno_s, G.weno_w, K, eL, eR, src, [&](const auto& r0, const auto& u) {
+          sfor<NGLL>([&](auto ii) {
+            rl[ii] = r0[ii];
+            sfor<NA - 1>([&](auto kt) { ul[kt][ii] = u[kt][ii]; });
+          });
+        });
+    sfor<5>([&](auto l) { s_e[5 * (rf + up_row) + l] = eR[l]; });
+    for (int q = 0; q < ntr; q++) {
+      double u[ORD], g[NGLL], a0, a1;
+      sfor<ORD>([&](auto s) { u[s] = s_tq[ts * (rw + (s - hs) * up_row) + q]; });
+      reconstruct<ORD, NGLL>(u, G.weno_s, g);
+      tracer_edges<NGLL>(g, rl, ul, (pos >> q) & 1u, K, a0, a1);
+      s_tl[ts * rf + q] = a0;
+      s_te[ts * (rf + up_row) + q] = a1;
+    }
+  }
+  __syncthreads();
+
+  // 3. faces: state flux, tracer fluxes upwinded with the state's normal
+  // velocity, and the limiter's direction (the normal momentum average, S:907).
+  // A lane takes its cell's low face; the last cell of a walled line also face
+  // n, the first of a periodic z line also face n, whose background differs
+  // from face 0's (S:1628-1629).
+  auto face_ref = [&](int f) {
+    FaceRef fr;
+    if constexpr (DIR == 0) {
+      fr.rt = fr.q5 = G.prT[kl];
+    } else if constexpr (DIR == 1) {
+      fr.rt = G.prRT[kl];
+      fr.q5 = G.prT[kl];
+    } else {
+      fr.rt = fr.q5 = G.prF[f];
+    }
+    return fr;
+  };
+  auto subtract_p = [&](int f, double(&F)[5]) {
+    if constexpr (DIR == 2)
+      F[idW] -= f < n ? G.hyPressureGLL[f * NGLL] : G.hyPressureGLL[(n - 1) * NGLL + NGLL - 1];
+  };
+  const bool wrap = per && c == 0;
+  const int rn = row_f(col, n);
+  double F[5], un, dlo = 0.0, dn = 0.0;     // limiter directions of the low face and of face n
+  if (on) {
+    if (!per && c == 0) {
+      wall_flux<DIR>(eL, face_ref(0), F);
+      dlo = eL[NM];
+      const double up = F[0] * rcp(eL[0]);
+      for (int q = 0; q < ntr; q++) s_te[ts * rf + q] = s_tl[ts * rf + q] * up;
+      subtract_p(0, F);
+    } else {
+      const int rs = wrap ? rn : rf;        // slot of the left edge
+      double L[5];
+      sfor<5>([&](auto l) { L[l] = s_e[5 * rs + l]; });
+      riemann<DIR>(L, eL, face_ref(c), F, un);
+      dlo = dn = L[NM] + eL[NM];
+      const bool left = un > 0;
+      const double up = F[0] * rcp(left ? L[0] : eL[0]);
+      if (DIR == 2 && wrap) {
+        double Fn[5];
+        riemann<DIR>(L, eL, face_ref(n), Fn, un);
+        const double upn = Fn[0] * rcp(left ? L[0] : eL[0]);
+        for (int q = 0; q < ntr; q++) {
+          const double e = left ? s_te[ts * rn + q] : s_tl[ts * rf + q];
+          s_te[ts * rf + q] = e * up;
+          s_te[ts * rn + q] = e * upn;
+        }
+        subtract_p(n, Fn);
+        sfor<5>([&](auto l) { s_e[5 * rn + l] = Fn[l]; });
+      } else {
+        for (int q = 0; q < ntr; q++) {
+          const double e = (left ? s_te[ts * rs + q] : s_tl[ts * rf + q]) * up;
+          s_te[ts * rf + q] = e;
+          if (wrap) s_te[ts * rn + q] = e;
+        }
+      }
+      subtract_p(c, F);
+      if (!(DIR == 2 && wrap)) sfor<5>([&](auto l) { s_e[5 * rs + l] = F[l]; });
+    }
+    if (!per && c == n - 1) {
+      double e[5], Fn[5];
+      sfor<5>([&](auto l) { e[l] = s_e[5 * rn + l]; });
+      wall_flux<DIR>(e, face_ref(n), Fn);
+      dn = e[NM];
+      const double up = Fn[0] * rcp(e[0]);
+      for (int q = 0; q < ntr; q++) s_te[ts * rn + q] *= up;
+      subtract_p(n, Fn);
+      sfor<5>([&](auto l) { s_e[5 * rn + l] = Fn[l]; });
+    }
+  }
+  __syncthreads();
+
+  // 4. positivity limiter (T1): cell factors from the unlimited fluxes, then
+  // each face takes its upwind cell's factor
+  if (pos) {
+    if (on) {
+      const double dens = s_st[5 * rw + idR] + G.hyDensCells[hs + (DIR == 2 ? c : kl)];
+      for (int q = 0; q < ntr; q++)
+        if ((pos >> q) & 1u) {
+          const double f1 = fmin(s_te[ts * rf + q], 0.0);
+          const double f2 = fmax(s_te[ts * (rf + up_row) + q], 0.0);
+          const double fluxOut = K.dt * (f2 - f1) * K.rd;
+          s_tq[ts * rw + q] = fmin(1.0, s_tq[ts * rw + q] * dens * rcp(fluxOut + TRACER_EPS));
+        }
+    }
+    __syncthreads();
+    if (on) {
+      auto limit = [&](int f, int slot, double dir) {
+        if (!(dir > 0) && !(dir < 0)) return;
+        const int a = dir > 0 ? (f == 0 ? n - 1 : f - 1) : (f == n ? 0 : f);
+        const int ra = row_w(col, a);
+        for (int q = 0; q < ntr; q++)
+          if ((pos >> q) & 1u) s_te[ts * slot + q] *= s_tq[ts * ra + q];
+      };
+      limit(c, rf, dlo);
+      if (wrap || (!per && c == n - 1)) limit(wrap && DIR != 2 ? 0 : n, rn, dn);
+    }
+    __syncthreads();
+  }
+
+  // 5. tendencies: the state as the production sweep forms them, the tracers
+  // as -(flux difference) / d (S:950) by the same reciprocal
+  if (on) {
+    int64_t ot = 0, nc = 0;
+    if constexpr (TEND) {
+      const int line = line0 + col;
+      nc = (int64_t)G.nx * G.ny * G.nz;
+      ot = DIR == 0   ? (int64_t)line * G.nx + c
+           : DIR == 1 ? ((int64_t)kl * G.ny + c) * G.nx + (line - kl * G.nx)
+                      : (int64_t)c * G.ny * G.nx + line;
+    }
+    sfor<5>([&](auto l) {
+      double td = -(s_e[5 * (rf + up_row) + l] - F[l]) * K.rd;
+      if (DIR == 2 && l == idW) td = src + td;
+      if (G.sim2d && l == idV) td = 0.0;
+      if constexpr (TEND) out[l * nc + ot] = td;
+      else out[l * G.sl + o] = s_st[5 * rw + l] + K.dt * td;
+    });
+    for (int q = 0; q < ntr; q++) {
+      const double td = -(s_te[ts * (rf + up_row) + q] - s_te[ts * rf + q]) * K.rd;
+      if constexpr (TEND) tr_out[q * nc + ot] = td;
+      else tr_out[q * G.sl + o] = tr_in[q * G.sl + o] + K.dt * td;
+    }
+  }
+}
+
+// Lines per work-group of a tile, and its modelled cost per cell in waves of
+// full lanes: the idle lanes of the waves, the waves a CU holds (16, by the
+// registers; work-groups of 5 to 8 waves fit twice, larger ones and those that
+// fill the LDS once, and a lone group idles at its barriers), and in y and z the
+// runs of `cols` neighbouring lines that a load covers.  Measured, y at
+// 256x256x128 with 3 tracers: 1 line 791 us, 2 (8 waves) 662, 3 (12 waves) 953, 4
+// (16 waves) 856; z: 1 line 1110, 2 747, 3 (6 waves) 974, 4 (8 waves) 670, 5 (10
+// waves) 1065, 6 (12 waves) 915, 8 (16 waves) 835.
+struct TtCut {
+  int cols;
+  double cost;
+};
+inline TtCut tt_cut(int dir, int n, int64_t lines, int hs, int ntr) {
+  TtCut best{0, 1e300};
+  for (int m = 1; m * n <= TT_MAX && (m == 1 || (lines + m - 1) / m >= 256); m++) {
+    const int waves = (m * n + 63) / 64;
+    const size_t lds = tt_lds(n, m, hs, ntr);
+    if (lds > 160 * 1024) break;
+    const int groups = (int)std::min<size_t>(waves <= 4 ? 16 / waves : waves <= 8 ? 2 : 1, 160 * 1024 / lds);
+    const double runs = dir == 0 || m >= 4 ? 1.0 : m == 3 ? 1.05 : m == 2 ? 1.11 : 1.33;
+    // a small grid needs fewer waves than a CU holds, but whole rounds of groups
+    const double need = std::min(16.0, (double)lines * n / 64 / 256);
+    const double held = std::max(1.0, need / (groups * waves)) * (groups == 1 ? 1.4 : 1.0);
+    const int64_t wgs = (lines + m - 1) / m;
+    const double rounds = wgs <= 1024 && wgs >= 256 ? (wgs + 255) / 256 * 256.0 / wgs : 1.0;
+    const double cost = 64.0 * waves / (m * n) * held * rounds * runs * (waves == 1 ? 1.06 : waves == 2 ? 1.03 : 1.0);
+    if (cost < best.cost * 0.999) best = TtCut{m, cost};
+  }
+  return best;
+}
+
+// ---------------------------------------------------------------------------
 // y and z sweeps: the tracer walker.
 //
-// A y or z line is strided in memory (each cell on its own cache line), so
-// the line kernel above, one line per work-group, issues one cache line per
-// lane for every load and store.  Here a work-group of four waves takes
+// For y and z lines whose length leaves a tile's waves idle, or too few of them
+// on a CU.  A work-group of four waves takes
 // WK_WX = 4 lines that are neighbours in x, wave w on line w, and walks them
 // in steps of WK_SEG = 64 cells, lane c on cell X = c0 + c of the step.
 // - Loads are issued with the lanes across x (the four lines' values of one
@@ -1057,27 +1359,31 @@ __global__ void k_fill_tr(double* __restrict__ p, int64_t n, double v) {
 using KernelTr = void (*)(const double*, const double*, double*, double*, Grid, SweepK, int, unsigned);
 using KernelWk = void (*)(WalkArgs);
 
+using KernelTt = void (*)(const double*, const double*, double*, double*, Grid, SweepK, int, unsigned, int);
 struct VariantTr {
   int ord, ngll;
-  KernelTr upd[3], tend[3];
-  KernelWk wupd[2], wtend[2];   // y and z walkers (null: the line kernels run y and z)
+  KernelTr upd[3], tend[3];     // line kernels (null: the tiles and walkers take every y and z line)
+  KernelWk wupd[2], wtend[2];   // y and z walkers (null: none)
+  KernelTt tile[2][3];          // tiles (null: none), update and tendency
   void (*init)(double*, Grid, int, double, double);
 };
 
-#define AWFL_VARIANT_TR(O, N, WU, WT)                                                          \
+#define AWFL_TILE_TR(O, N)                                                                     \
+  {{k_tile_tr<O, N, 0, false>, k_tile_tr<O, N, 1, false>, k_tile_tr<O, N, 2, false>},          \
+   {k_tile_tr<O, N, 0, true>, k_tile_tr<O, N, 1, true>, k_tile_tr<O, N, 2, true>}}
+#define AWFL_VARIANT_TR(O, N)                                                                  \
   VariantTr {                                                                                  \
-    O, N, {k_sweep_tr<O, N, 0, false>, k_sweep_tr<O, N, 1, false>, k_sweep_tr_z<O, N, false>}, \
-        {k_sweep_tr<O, N, 0, true>, k_sweep_tr<O, N, 1, true>, k_sweep_tr_z<O, N, true>}, WU, WT, \
-        k_init_tr<O>,                                                                          \
+    O, N, {k_sweep_tr<O, N, 0, false>}, {k_sweep_tr<O, N, 0, true>}, AWFL_WALK_TR(O, N, false), \
+        AWFL_WALK_TR(O, N, true), AWFL_TILE_TR(O, N), k_init_tr<O>,                            \
   }
 #define AWFL_WALK_TR(O, N, T) {k_walk_tr<O, N, 1, T>, k_walk_tr<O, N, 2, T>}
 
-// (9, 5) keeps the line kernels in y and z: its cell is too large for a
-// work-group of four lines
+// (9, 5) keeps the line kernels: its cell is too large for the registers of a
+// tile or for a walker's work-group of four lines
 const VariantTr kVariantsTr[] = {
-    AWFL_VARIANT_TR(3, 2, AWFL_WALK_TR(3, 2, false), AWFL_WALK_TR(3, 2, true)),
-    AWFL_VARIANT_TR(5, 3, AWFL_WALK_TR(5, 3, false), AWFL_WALK_TR(5, 3, true)),
-    AWFL_VARIANT_TR(9, 5, {}, {})};
+    AWFL_VARIANT_TR(3, 2), AWFL_VARIANT_TR(5, 3),
+    VariantTr{9, 5, {k_sweep_tr<9, 5, 0, false>, k_sweep_tr<9, 5, 1, false>, k_sweep_tr_z<9, 5, false>},
+              {k_sweep_tr<9, 5, 0, true>, k_sweep_tr<9, 5, 1, true>, k_sweep_tr_z<9, 5, true>}, {}, {}, {}, k_init_tr<9>}};
 
 const VariantTr* find_variant_tr(int ord, int ngll) {
   for (const VariantTr& v : kVariantsTr)
@@ -1097,22 +1403,43 @@ int launch_sweep_tr(awfl_ctx* c, const double* in, const double* tr_in, double* 
   const int n = dir == 0 ? c->cfg.nx : dir == 1 ? c->cfg.ny : c->cfg.nz;
   const int W = n + 2 * c->hs, ntr = c->ntr;
   const int64_t nc = (int64_t)c->cfg.nx * c->cfg.ny * c->cfg.nz;
-  if (dir > 0 && n >= 8 && v->wupd[dir - 1]) {
+  const bool walks = dir > 0 && n >= 8 && v->wupd[dir - 1];
+  const size_t lds = sizeof(double) * (size_t)(5 * W + ntr * W + 10 * n + 2 * ntr * n + (dir == 2 ? 2 : 1) * n);
+  if (!walks && lds > 160 * 1024) return fail(c, AWFL_E_UNSUPPORTED, "tracers: line too long for the tracer sweep's LDS");
+  // Tile or walker: the walker's waves take steps of 64 cells of a line, the tile
+  // pays for idle lanes and short runs but not for the walker's head, tail and
+  // carries.  Around the line: y at n = 256 (cost 1.11 of the walker's) 662
+  // against 704 us, 210 (1.33) 225 and 240, 150 (1.42) 486 and 552, 400 (1.5)
+  // 78 and 71, 300 (1.6) 607 and 422; z at 128 (1.0) 670 and 777, 150 (1.42) 577
+  // and 566, 180 (1.42) 238 and 230.
+  if (KernelTt k = v->tile[tend][dir]) {
+    const int64_t lines = nc / n;
+    const TtCut cut = tt_cut(dir, n, lines, c->hs, ntr);
+    const double walker = (n + 63) / 64 * 64.0 / n;
+    if (cut.cols && (!walks || cut.cost < (dir == 1 ? 1.45 : 1.3) * walker)) {
+      const size_t tlds = tt_lds(n, cut.cols, c->hs, ntr);
+      if (tlds > 64 * 1024)
+        HIP_TRY(c, hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)tlds));
+      k<<<(unsigned)((lines + cut.cols - 1) / cut.cols), (cut.cols * n + 63) / 64 * 64, tlds, c->stream>>>(
+          in, tr_in, out, tr_out, c->grid(), sweep_constants(c, dt, dir), ntr, c->tpos, cut.cols);
+      LAUNCH_CHECK(c);
+      return AWFL_OK;
+    }
+  }
+  if (walks) {
     // the walker: tiles of WK_WX x-adjacent lines
     const int hs = c->hs, HB = hs > 2 ? hs : 2;
     const WalkLds L = walk_lds(ntr, WK_SEG + HB + hs, dir == 2);
-    const size_t lds = sizeof(double) * (size_t)L.size * WK_WX;
+    const size_t wlds = sizeof(double) * (size_t)L.size * WK_WX;
     KernelWk k = tend ? v->wtend[dir - 1] : v->wupd[dir - 1];
-    if (lds > 64 * 1024)
-      HIP_TRY(c, hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    if (wlds > 64 * 1024)
+      HIP_TRY(c, hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)wlds));
     const unsigned tiles = (unsigned)((c->cfg.nx + WK_WX - 1) / WK_WX) * (unsigned)(dir == 1 ? c->cfg.nz : c->cfg.ny);
     const WalkArgs a{in, tr_in, out, tr_out, c->grid(), sweep_constants(c, dt, dir), ntr, c->tpos};
-    k<<<tiles, 64 * WK_WX, lds, c->stream>>>(a);
+    k<<<tiles, 64 * WK_WX, wlds, c->stream>>>(a);
     LAUNCH_CHECK(c);
     return AWFL_OK;
   }
-  const size_t lds = sizeof(double) * (size_t)(5 * W + ntr * W + 10 * n + 2 * ntr * n + (dir == 2 ? 2 : 1) * n);
-  if (lds > 160 * 1024) return fail(c, AWFL_E_UNSUPPORTED, "tracers: line too long for the tracer sweep's LDS");
   KernelTr k = tend ? v->tend[dir] : v->upd[dir];
   if (lds > 64 * 1024)
     HIP_TRY(c, hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
