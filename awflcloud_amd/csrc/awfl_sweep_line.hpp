@@ -32,16 +32,19 @@
 //
 // Bound by FP64 issue.  At 192x192x96 the x, y and z sweeps took 788, 833 and
 // 958 us with three-way LDS bank conflicts in the exchange and every flux
-// product carried through the levels, 669, 698 and 944 us with neither.
+// product carried through the levels, 669, 698 and 944 us with neither, and 497,
+// 533 and 583 us with the constants left beside their use, four waves per SIMD
+// and no division in the stage.  Packing a short last chunk's lanes into fewer
+// waves and skipping the rest cost 5% on full chunks and is not done.
 #pragma once
 #include "awfl_cell.hpp"
 #include "awfl_internal.hpp"
 
-// Waves per SIMD the line kernels are compiled for.  Bounded to three, the
-// (9, 5) kernels take 150 (x, y) and 158 (z) VGPRs and no scratch; bounded
-// to four they spill 208-240 bytes per lane and run 1.6x slower.
+// Waves per SIMD the line kernels are compiled for: 119 registers in x and y,
+// 127 in z (two of them parked; bounded to three it takes 129 and z at
+// 192x192x96 629 us against 583).
 #ifndef AWFL_LS_WAVES
-#define AWFL_LS_WAVES 3
+#define AWFL_LS_WAVES 4
 #endif
 
 namespace awfl_line {
@@ -117,8 +120,9 @@ __global__ __launch_bounds__(LS_THREADS) __attribute__((amdgpu_waves_per_eu(AWFL
     int a = c - hs, src;
     bool zn = false;
     if (per) {
-      src = a % n;
-      if (src < 0) src += n;
+      src = a;                                          // at most hs cells past the line
+      while (src < 0) src += n;
+      while (src >= n) src -= n;
     } else if (a < 0) {
       src = 0; zn = true;
     } else if (a >= n) {
