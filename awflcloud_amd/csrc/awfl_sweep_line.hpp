@@ -41,8 +41,9 @@
 #include "awfl_internal.hpp"
 
 // Waves per SIMD the line kernels are compiled for: 119 registers in x and y,
-// 127 in z (two of them parked; bounded to three it takes 129 and z at
-// 192x192x96 629 us against 583).
+// 128 in z, where the source average accumulates in LDS (bounded to three, z at
+// 192x192x96 took 629 us against 583).  No scratch: the allocation-free step
+// runs these kernels, and a spilling one would make the runtime allocate.
 #ifndef AWFL_LS_WAVES
 #define AWFL_LS_WAVES 4
 #endif
@@ -172,7 +173,7 @@ __global__ __launch_bounds__(LS_THREADS) __attribute__((amdgpu_waves_per_eu(AWFL
     // levels 0 .. NA-2, the normal velocity's Taylor coefficients u (the flux of
     // l is sum_j u_j q_l,k-j; cell_transform in awfl_cell.hpp) and (r t)^gamma
     double q[5][NA], u[NA], g[NA], e[5];
-    double sv = 0.0, sa = 0.0, rr, rrt;
+    double sv = 0.0, rr, rrt;
     {
       double q0[5];
       sfor<5>([&](auto l) { q0[l] = xw[l * XR]; });
@@ -184,7 +185,8 @@ __global__ __launch_bounds__(LS_THREADS) __attribute__((amdgpu_waves_per_eu(AWFL
         pr = G.prG[kc * NGLL + ii];
         // S:1439 assigns a scalar to the whole SArray: every entry of the
         // source holds the value of the last GLL point
-        sa = sv = -GRAV * xc[idR * XR + NGLL - 1];
+        sv = -GRAV * xc[idR * XR + NGLL - 1];
+        if (act && ii == 0) s_src[c] = sv;
       } else {
         brho = G.hyDensCells[hs + kl];
         brt = G.hyDensThetaCells[hs + kl];
@@ -241,7 +243,8 @@ __global__ __launch_bounds__(LS_THREADS) __attribute__((amdgpu_waves_per_eu(AWFL
         if constexpr (DIR == 2 && l == idW) v = kt == 0 ? v + sv : fm(-GRAV * rkt1, q[idR][kt], v);
         q[l][kt + 1] = v;
         // the source average takes the exact integral of d(rho)/dt (S:1462, 1489-1492)
-        if constexpr (DIR == 2 && l == idR) sa = fm(-GRAV * (tav * ndt), x[NGLL - 1] - x[0], sa);
+        if constexpr (DIR == 2 && l == idR)
+          if (act && ii == 0) s_src[c] = fm(-GRAV * (tav * ndt), x[NGLL - 1] - x[0], s_src[c]);
       });
       if constexpr (DIR == 2) {                         // S:2051-2055
         if (!per && c == n - 1 && ii == NGLL - 1) q[idW][kt + 1] = 0.0;
@@ -262,10 +265,9 @@ __global__ __launch_bounds__(LS_THREADS) __attribute__((amdgpu_waves_per_eu(AWFL
         g[kt + 1] = fm(GAMMA * g[0], q[idT][kt + 1], tg * rkt1) * rrt;
       }
     });
-    if (act && (ii == 0 || ii == NGLL - 1)) {           // edge states, z source average
+    if (act && (ii == 0 || ii == NGLL - 1)) {           // edge states
       const int row = ii == 0 ? 0 : 5;
       sfor<5>([&](auto l) { s_e[(row + l) * n + c] = e[l]; });
-      if (DIR == 2 && ii == 0) s_src[c] = sa;
     }
     __syncthreads();                                    // the next chunk rewrites s_x
   }
