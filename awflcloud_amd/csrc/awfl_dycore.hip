@@ -1037,7 +1037,9 @@ static int launch_line(awfl_ctx* c, const double* in, double* out, const SweepK&
   const int n = dir == 0 ? c->cfg.nx : dir == 1 ? c->cfg.ny : c->cfg.nz;
   const unsigned lines = (unsigned)((int64_t)c->cfg.nx * c->cfg.ny * c->cfg.nz / n);
   const size_t lds = sizeof(double) * awfl_line::line_lds_doubles(n, c->hs, c->cfg.ngll, inplace);
-  if (lds > 160 * 1024) return fail(c, AWFL_E_UNSUPPORTED, "line too long for the lane-split sweep's LDS");
+  // (the limit on a line's length counts a chunk row that the kernels no longer need)
+  if (lds + sizeof(double) * awfl_line::LS_CHUNK > 160 * 1024)
+    return fail(c, AWFL_E_UNSUPPORTED, "line too long for the lane-split sweep's LDS");
   if (lds > 64 * 1024)
     HIP_TRY(c, hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   k<<<lines, awfl_line::LS_THREADS, lds, c->stream>>>(in, out, c->grid(), K);

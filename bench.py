@@ -39,10 +39,11 @@ FLOPS_PER_CELL_SWEEP = {0: 2488.3, 1: 2480.3, 2: 2553.6}
 FLOPS_PER_CELL_STEP = 7552.2
 
 # VALU wave-instructions x 64 per cell of each FP64 sweep kernel (x, y, z) at
-# 256x256x128, from rocprofv3 SQ_INSTS_VALU (profiles/sweeps_valu_counters.md);
+# 256x256x128, from rocprofv3 SQ_INSTS_VALU
+# (profiles/sweep_kernels_times_and_counters.md);
 # MI355X: 256 CUs x 4 SIMDs at 2.4 GHz, one FP64 wave64 VALU instruction per
 # 4 cycles per SIMD
-VALU_INSTS_PER_CELL = {0: 1505.0, 1: 1363.0, 2: 1436.0}
+VALU_INSTS_PER_CELL = {0: 1054.0, 1: 1036.0, 2: 1089.0}
 N_SIMD, CLOCK_HZ = 1024, 2.4e9
 
 NX, NY, NZ = 256, 256, 128
