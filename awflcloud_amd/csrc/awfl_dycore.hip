@@ -66,7 +66,8 @@ __device__ __forceinline__ int64_t tend_index(const Grid& G, int l, int k, int j
 // K.br; 2 takes the branch from K.br instead of the sign test (frozen-branch
 // forward for difference checks of the adjoint).  Branch bytes: x face f of
 // line (k, j) at (k ny + j)(nx+1) + f; y face f of (k, i) at (k (ny+1) + f) nx
-// + i; z face f of (j, i) at (f ny + j) nx + i.
+// + i; z face f of (j, i) at (f ny + j) nx + i.  All faces, but the last of
+// a periodic x line, which is its first.
 template <int DIR, int BR>
 __device__ __forceinline__ void face_flux(const double (&qL)[5], const double (&qR)[5], const FaceRef& fr,
                                           double (&F)[5], unsigned char* bp) {
@@ -139,9 +140,11 @@ struct Sweep64 {
     }
     return fr;
   }
+  // (a periodic x line's last face is its first: one byte, the first's)
   __device__ unsigned char* branch(int o, int line, int f) const {
     if constexpr (BR == 0) return nullptr;
-    else if constexpr (DIR == 0) return K.br + ((int64_t)o * g.ny + line) * (g.nx + 1) + f;
+    else if constexpr (DIR == 0)
+      return K.br + ((int64_t)o * g.ny + line) * (g.nx + 1) + (g.bc[0] == AWFL_BC_PERIODIC && f == g.nx ? 0 : f);
     else if constexpr (DIR == 1) return K.br + ((int64_t)o * (g.ny + 1) + f) * g.nx + line;
     else return K.br + ((int64_t)f * g.ny + o) * g.nx + line;
   }
@@ -153,6 +156,8 @@ struct Sweep64 {
   __device__ __forceinline__ void face(int o, int line, int f, const double (&qL)[5], const double (&qR)[5],
                                        double (&F)[5]) const {
     face_flux<DIR, BR>(qL, qR, face_ref(o, f), F, branch(o, line, f));
+    if constexpr (BR == 1 && DIR == 1)               // a whole periodic line forms its last face with its first
+      if (f == 0 && g.bc[1] == AWFL_BC_PERIODIC) *branch(o, line, g.ny) = *branch(o, line, 0);
     subtract_p(f, F);
   }
   __device__ __forceinline__ void wall(int o, int line, int f, const double (&q)[5], double (&F)[5]) const {
