@@ -364,7 +364,12 @@ constexpr int adj_pv() {
   return 10 / ORD;
 }
 constexpr int ADJ_SLOTS = 20;
-constexpr int ADJ_MAX = 640;    // cells of a line, lanes of a work-group
+// Cells of a line, lanes of a work-group: the twelve waves that a CU holds.  The
+// five kernels for longer lines, with 56 doubles (3, 2) or 76 (5, 3) of HBM per
+// cell, took 1.1 to 1.2 ms for a sweep along a line of 700 cells, 160 x 40 of them,
+// at (3, 2) and 1.6 ms at (5, 3); this kernel takes 0.37 (x), 0.58 (y), 0.62 (z) and
+// 0.53, 0.72, 0.73 ms.
+constexpr int ADJ_MAX = 768;
 
 template <int ORD, int NGLL, int DIR>
 __global__ __launch_bounds__(ADJ_MAX) __attribute__((amdgpu_waves_per_eu(3))) void k_adj_tile(
