@@ -7,7 +7,7 @@
 // adj_in = adj_out + J^T (dt adj_out) runs as one fused kernel over whole lines
 // along the sweep direction (k_adj_tile: forward, face adjoints, transform
 // and WENO reverses and the gather in registers and LDS).  Lines of more than
-// ADJ_MAX cells run as five kernels over per-cell scratch in HBM:
+// awfl_cut::ADJ_MAX cells run as five kernels over per-cell scratch in HBM:
 //   k_edges      cell forward, one thread per cell: WENO values at the GLL
 //                points [5 ngll/cell], then time-averaged edge states and
 //                z source                                                [11/cell]
@@ -31,6 +31,7 @@
 #include <vector>
 
 #include "awfl_adjoint.hpp"
+#include "awfl_cut.hpp"
 #include "awfl_internal.hpp"
 
 using namespace awfl;
@@ -364,15 +365,9 @@ constexpr int adj_pv() {
   return 10 / ORD;
 }
 constexpr int ADJ_SLOTS = 20;
-// Cells of a line, lanes of a work-group: the twelve waves that a CU holds.  The
-// five kernels for longer lines, with 56 doubles (3, 2) or 76 (5, 3) of HBM per
-// cell, took 1.1 to 1.2 ms for a sweep along a line of 700 cells, 160 x 40 of them,
-// at (3, 2) and 1.6 ms at (5, 3); this kernel takes 0.37 (x), 0.58 (y), 0.62 (z) and
-// 0.53, 0.72, 0.73 ms.
-constexpr int ADJ_MAX = 768;
 
 template <int ORD, int NGLL, int DIR>
-__global__ __launch_bounds__(ADJ_MAX) __attribute__((amdgpu_waves_per_eu(3))) void k_adj_tile(
+__global__ __launch_bounds__(awfl_cut::ADJ_MAX) __attribute__((amdgpu_waves_per_eu(3))) void k_adj_tile(
     const double* __restrict__ in, const double* __restrict__ adj_out, double* __restrict__ adj_in, Grid G, SweepK K,
     int cols) {
   static_assert(ORD <= 10, "stencil adjoints of one variable fit the ten slots");
@@ -557,28 +552,6 @@ __global__ __launch_bounds__(ADJ_MAX) __attribute__((amdgpu_waves_per_eu(3))) vo
         sfor<5>([&](auto l) { adj_in[l * G.sl + oh] = 0.0; });
       }
   }
-}
-
-// Lines per work-group, of at most four waves, one per SIMD (longer lines
-// alone): few idle lanes first, then whole groups of four, of which three fit a
-// CU and load its SIMDs alike; never so many that CUs stay without a group.
-// Against four waves, one, two and three took 1.10, 1.06 and 1.05 times as
-// long (128x128x64, z 143.8, 137.6 and 138.1 against 131.1 us; x and y by one
-// line of two waves 127.9 and 139.8, by two 123.1 and 127.6), five to eight
-// 1.09 to 1.4 times (100x90x75, x in 500 lanes 106 against 97 us).
-inline int adj_cols(int n, int64_t lines) {
-  constexpr double slack[5] = {0, 1.10, 1.06, 1.05, 1.0};
-  int best = 1;
-  double cost = 1e300;
-  for (int m = 1; m * n <= 256 && (m == 1 || (lines + m - 1) / m >= 256); m++) {
-    const int waves = (m * n + 63) / 64;
-    const double e = slack[waves] * waves / m;
-    if (e < cost) {
-      cost = e;
-      best = m;
-    }
-  }
-  return best;
 }
 
 // zero the halo of a padded array, one thread per halo cell: the 2hs z
@@ -772,7 +745,7 @@ int check_variant(awfl_ctx* c) {
 }
 
 // per-cell scratch of the multi-kernel sweeps (tangent; adjoint lines of more
-// than ADJ_MAX cells)
+// than awfl_cut::ADJ_MAX cells)
 int ensure_cell_scratch(awfl_ctx* c) {
   int rc = check_variant(c);
   if (rc != AWFL_OK) return rc;
@@ -816,9 +789,9 @@ int sweep_adjoint(awfl_ctx* c, const double* in, const double* adj_out, double* 
   const SweepK K = sweep_constants(c, dt, dir);
   const int64_t nc = (int64_t)c->cfg.nx * c->cfg.ny * c->cfg.nz;
   const int ng = c->cfg.ngll;
-  if (const int n = dir == 0 ? c->cfg.nx : dir == 1 ? c->cfg.ny : c->cfg.nz; n <= ADJ_MAX) {
+  if (const int n = dir == 0 ? c->cfg.nx : dir == 1 ? c->cfg.ny : c->cfg.nz; n <= awfl_cut::ADJ_MAX) {
     const int64_t lines = nc / n;
-    const int cols = adj_cols(n, lines);
+    const int cols = awfl_cut::adj_cols(n, lines);
     const size_t lds = sizeof(double) * ADJ_SLOTS * cols * n;
     if (lds > 64 * 1024)
       HIP_TRY(c, hipFuncSetAttribute((const void*)v->tile[dir], hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));

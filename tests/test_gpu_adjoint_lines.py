@@ -1,5 +1,6 @@
-"""The fused sweep adjoint on long lines: it takes lines of up to 768 cells and
-no scratch per cell; longer ones run as five kernels.  Tolerances as in
+"""The fused sweep adjoint on long lines: two lines of up to 384 cells share a
+work-group; it takes lines of up to 768 cells and no scratch per cell; longer ones
+run as five kernels.  Tolerances as in
 test_gpu_adjoint_tiles.py, whose test this is at other boxes."""
 import pytest
 import torch
@@ -17,6 +18,11 @@ pytestmark = pytest.mark.gpu
     (768, 2, 3, (1, 0, 1), 5, 3),
     (2, 768, 3, (0, 0, 1), 5, 3),
     (2, 3, 768, (0, 0, 1), 3, 2),
+    (257, 3, 87, (0, 0, 1), 5, 3),        # two lines to a group, the last group with one
+    (20, 300, 13, (0, 1, 1), 3, 2),
+    (9, 29, 384, (1, 0, 1), 5, 3),
+    (7, 37, 321, (0, 0, 0), 3, 2),
+    (384, 20, 13, (1, 1, 1), 3, 2),
     (769, 2, 3, (0, 0, 1), 3, 2),
     (2, 769, 3, (0, 1, 1), 5, 3),
     (2, 3, 769, (0, 0, 0), 3, 2),
