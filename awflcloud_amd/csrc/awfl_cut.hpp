@@ -1,9 +1,122 @@
 // awfl_cut.hpp -- how the sweeps are cut into work-groups: rules on sizes, host
 // code alone, with the timings that they rest on.
 #pragma once
+#include <algorithm>
+#include <cstddef>
 #include <cstdint>
 
 namespace awfl_cut {
+
+// ---------------------------------------------------------------------------
+// tile sweeps (awfl_tile.hpp) and column walkers
+// ---------------------------------------------------------------------------
+// How a sweep is cut: lines per work-group, rows (lanes along a line),
+// segments per line and their length.
+struct TilePlan {
+  int cols, rows, nseg, seglen;
+};
+
+constexpr int MAX_THREADS = 1024;
+
+// LDS elements of a work-group: staged cells and face slots
+inline size_t lds_elems(const TilePlan& p, int hs) { return (size_t)5 * p.cols * (2 * p.rows + 2 * hs + 1); }
+
+// TX choices of y and z tiles
+constexpr int TX_OF[3] = {4, 8, 16};
+
+// Rates of a sweep's kernels for the models below, in microseconds: a tile's
+// wave (one cell a lane), the factor of 4-line tiles (short runs of memory),
+// the factors of work-groups of 5 to 8 waves (how they pack on a CU), and the
+// column walker's step with x waves on a SIMD, max(walk_least, walk x + walk_0).
+struct Rates {
+  double tile, narrow, pack[4];
+  double walk, walk_0, walk_least;
+};
+
+// Rates of the (5, 3) kernels, which the cuts of the other orders share (a
+// ratio of the two kernels' times is all that they decide).  Fitted to sweeps
+// of 64x64x32 to 512x512x256 cells, every cut timed: best tiles 9 us at 64x64x32
+// (y and z; the walkers 55), 43 and 45 at 128x128x64 (57 and 62), 84 and 92 at
+// 160x160x80 (124 and 131), 147 and 161 at 192x192x96 (160 and 167), 228 and 271
+// at 96x300x200 (319 and 364), 340 and 393 at 256x256x128 (330 and 340).  The z
+// kernel has 112 registers, four waves per SIMD, which work-groups of five to
+// eight waves fill badly.
+inline const Rates& rates_f64(int dir) {
+  static constexpr Rates xy{2.55, 1.03, {1.15, 1.18, 1.12, 1.07}, 2.3, 0.8, 3.2};
+  static constexpr Rates z{2.6, 1.03, {1.4, 1.33, 1.2, 1.15}, 2.35, 0.9, 3.4};
+  return dir == 2 ? z : xy;
+}
+
+// Rates of the FP32 kernels for the cuts.  Fitted to: tiles 8 us at 64x64x32 (y
+// and z; the walkers 46 and 43), 25 at 120x100x60 (51 and 56), 33 at 128x128x64
+// (48), 108 and 112-128 at 192x192x96 (103 and 104), 234 and 260 at 256x256x128
+// (230 and 218), 1947 and 1999 at 512x512x256 (1545 and 1609).
+constexpr Rates RATES_F32{1.75, 1.2, {1.15, 1.18, 1.12, 1.07}, 1.4, 1.0, 2.7};
+
+struct TileCut {
+  int tx;                     // index into TX_OF (y, z)
+  TilePlan p;
+  int threads;
+  double us;                  // modelled time
+};
+
+// Cut of a sweep of n-cell lines, nline of them side by side in each of `other`
+// rows: the one of least modelled time, a tile's latency (some 5 us from its
+// loads to its stores) plus the issue time of the waves that a SIMD gets (256
+// CUs of four SIMDs; small grids in whole rounds).  An idle lane costs three
+// quarters of a busy one.  `whole`: x lines that are updated in place, which a
+// work-group must hold whole.  Other x lines of more than 512 cells run in
+// segments: a group of 9 to 16 waves leaves a CU's places empty and its barriers
+// uncovered (160 x 64 lines at (5, 3), whole against the best segments: 513 cells
+// 336 and 219 us, 640 356 and 273, 800 435 and 328, 1024 456 and 427; at (3, 2) 249
+// and 158, 269 and 194, 328 and 234, 345 and 311).
+inline TileCut tile_cut(int dir, int n, int nline, int other, bool per, const Rates& rate, bool whole = false) {
+  TileCut best{};
+  best.us = 1e300;
+  auto consider = [&](int tx, int cols, int nseg, int limit) {
+    const int seglen = (n + nseg - 1) / nseg;
+    if ((n + seglen - 1) / seglen != nseg) return;
+    const int rows = nseg == 1 ? n : !per && nseg == 2 ? seglen + 1 : seglen + 2;
+    if (rows * cols > limit) return;
+    const int waves = (rows * cols + 63) / 64;
+    const double wgs = (double)nseg * ((nline + cols - 1) / cols) * other;
+    const double rounds = wgs <= 1024 ? (double)(((int64_t)wgs + 255) / 256) : wgs / 256;
+    const double eq = (0.75 * waves + 0.25 * rows * cols / 64.0) * (waves > 4 ? rate.pack[std::min(waves, 8) - 5] : 1.0) *
+                      (dir > 0 && cols == 4 ? rate.narrow : 1.0);
+    const double us = 5.0 + rate.tile * std::max(rounds * eq / 4, (double)((waves + 3) / 4));
+    if (us < best.us) best = TileCut{tx, TilePlan{cols, rows, nseg, seglen}, waves * 64, us};
+  };
+  if (dir == 0) {
+    if (whole || n <= 512)
+      for (int cols = 1; cols <= std::max(1, std::min(nline, 512 / n)); cols++) consider(0, cols, 1, MAX_THREADS);
+    else
+      for (int nseg = 2; nseg <= n / 64; nseg++) consider(0, 1, nseg, 512);
+  } else {
+    for (int x = 0; x < 3; x++)
+      for (int nseg = 1; nseg <= std::max(1, n / 14); nseg++) consider(x, TX_OF[x], nseg, 512);
+  }
+  return best;
+}
+
+// Cut of a column-walker sweep (a lane walks a segment of its column; y and z):
+// segments of at most 32 cells, and shorter (down to 16) where that is needed
+// for ~4 waves per SIMD.  Modelled time: every wave reconstructs two cells more
+// than its segment has.
+struct WalkCut {
+  int bx, nseg, seglen;
+  double us;
+};
+inline WalkCut walk_cut(int n, int nx, int other, const Rates& rate) {
+  WalkCut w{};
+  w.bx = (nx + 63) / 64;
+  const int64_t layer = (int64_t)w.bx * other;
+  const int nseg = (int)std::max<int64_t>(1, std::min<int64_t>(std::max<int64_t>((4096 + layer - 1) / layer, (n + 31) / 32),
+                                                               std::max(1, n / 16)));
+  w.seglen = (n + nseg - 1) / nseg;
+  w.nseg = (n + w.seglen - 1) / w.seglen;
+  w.us = (w.seglen + 2) * std::max(rate.walk * (double)(layer * w.nseg) / 1024.0 + rate.walk_0, rate.walk_least);
+  return w;
+}
 
 // ---------------------------------------------------------------------------
 // sweep adjoint (k_adj_tile in awfl_adjoint.hip)

@@ -184,8 +184,8 @@ struct Sweep64 {
 };
 
 template <int ORD, int NGLL, int DIR, int TX, bool TEND, int BR = 0>
-__global__ __launch_bounds__(awfl_tile::MAX_THREADS) void k_sweep_tile(const double* in, double* out, Grid G,
-                                                                       SweepK K, awfl_tile::TilePlan T) {
+__global__ __launch_bounds__(awfl_cut::MAX_THREADS) void k_sweep_tile(const double* in, double* out, Grid G,
+                                                                       SweepK K, awfl_cut::TilePlan T) {
   awfl_tile::sweep(Sweep64<ORD, NGLL, DIR, TX, TEND, BR>{in, out, G, K}, T);
 }
 
@@ -583,7 +583,7 @@ __global__ void k_init(double* __restrict__ st, Grid G, InitDev S) {
 // kernel of awfl_time_step_noalloc
 using LineFn = void (*)(const double*, double*, Grid, SweepK);
 // the tile kernels: x, then y and z with 4, 8 and 16 lines a tile
-using TileFn = void (*)(const double*, double*, Grid, SweepK, awfl_tile::TilePlan);
+using TileFn = void (*)(const double*, double*, Grid, SweepK, awfl_cut::TilePlan);
 struct TileFns {
   TileFn x, yz[2][3];
 };
@@ -985,31 +985,18 @@ int awfl_state_sums(awfl_ctx* c, const double* d_state, double* h_out) {
 }  // extern "C"
 
 
-// Rates of the (5, 3) kernels, which the cuts of the other orders share (a
-// ratio of the two kernels' times is all that they decide).  Fitted to sweeps
-// of 64x64x32 to 512x512x256 cells, every cut timed: best tiles 9 us at 64x64x32
-// (y and z; the walkers 55), 43 and 45 at 128x128x64 (57 and 62), 84 and 92 at
-// 160x160x80 (124 and 131), 147 and 161 at 192x192x96 (160 and 167), 228 and 271
-// at 96x300x200 (319 and 364), 340 and 393 at 256x256x128 (330 and 340).  The z
-// kernel has 112 registers, four waves per SIMD, which work-groups of five to
-// eight waves fill badly.
-static const awfl_tile::Rates& rates_of(int dir) {
-  static const awfl_tile::Rates xy{2.55, 1.03, {1.15, 1.18, 1.12, 1.07}, 2.3, 0.8, 3.2};
-  static const awfl_tile::Rates z{2.6, 1.03, {1.4, 1.33, 1.2, 1.15}, 2.35, 0.9, 3.4};
-  return dir == 2 ? z : xy;
-}
-
-// launch one tile sweep with the given kernels
+// launch one tile sweep with the given kernels (x: in == out updates in place)
 static int launch_tile(awfl_ctx* c, const double* in, double* out, const SweepK& K, int dir, const TileFns& f,
-                       const awfl_tile::TileCut* known = nullptr) {
+                       const awfl_cut::TileCut* known = nullptr) {
   const int n = dir == 0 ? c->cfg.nx : dir == 1 ? c->cfg.ny : c->cfg.nz;
   const int nline = dir == 0 ? c->cfg.ny : c->cfg.nx;
   const int other = dir == 2 ? c->cfg.ny : c->cfg.nz;
   const int bc = dir == 0 ? c->cfg.bc_x : dir == 1 ? c->cfg.bc_y : c->cfg.bc_z;
-  const awfl_tile::TileCut cut =
-      known ? *known : awfl_tile::tile_cut(dir, n, nline, other, bc == AWFL_BC_PERIODIC, rates_of(dir));
+  const awfl_cut::TileCut cut = known ? *known
+                                      : awfl_cut::tile_cut(dir, n, nline, other, bc == AWFL_BC_PERIODIC,
+                                                           awfl_cut::rates_f64(dir), in == out);
   const TileFn k = dir == 0 ? f.x : f.yz[dir - 1][cut.tx];
-  const size_t lds = sizeof(double) * awfl_tile::lds_elems(cut.p, c->hs);
+  const size_t lds = sizeof(double) * awfl_cut::lds_elems(cut.p, c->hs);
   if (lds > 64 * 1024)
     HIP_TRY(c, hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   const dim3 grid((nline + cut.p.cols - 1) / cut.p.cols, other, cut.p.nseg);
@@ -1027,9 +1014,9 @@ static int launch_cells(awfl_ctx* c, const double* in, double* out, const SweepK
   const int n = dir == 1 ? c->cfg.ny : c->cfg.nz;
   const int other = dir == 1 ? c->cfg.nz : c->cfg.ny;
   const int bc = dir == 1 ? c->cfg.bc_y : c->cfg.bc_z;
-  const awfl_tile::Rates& rate = rates_of(dir);
-  const awfl_tile::TileCut cut = awfl_tile::tile_cut(dir, n, c->cfg.nx, other, bc == AWFL_BC_PERIODIC, rate);
-  const awfl_tile::WalkCut walk = awfl_tile::walk_cut(n, c->cfg.nx, other, rate);
+  const awfl_cut::Rates& rate = awfl_cut::rates_f64(dir);
+  const awfl_cut::TileCut cut = awfl_cut::tile_cut(dir, n, c->cfg.nx, other, bc == AWFL_BC_PERIODIC, rate);
+  const awfl_cut::WalkCut walk = awfl_cut::walk_cut(n, c->cfg.nx, other, rate);
   if (cut.us <= walk.us) return launch_tile(c, in, out, K, dir, v->tile[tend], &cut);
   v->col[dir - 1][tend]<<<dim3(walk.bx, other, walk.nseg), 64, 0, c->stream>>>(in, out, c->grid(), K, walk.seglen);
   LAUNCH_CHECK(c);
@@ -1196,7 +1183,7 @@ int awfl_time_step_noalloc(awfl_ctx* c, double* d_state, double dt) {
       rc = (d == 0 && src == dst) ? launch_line(c, src, dst, K, 0, v->line_x_inplace, true)
                                   : launch_line(c, src, dst, K, d, v->sweep_line[d][0]);
     else
-      rc = launch_cells(c, src, dst, K, d, v, false);   // (x lines are whole up to the limit above: in place)
+      rc = launch_cells(c, src, dst, K, d, v, false);   // (in place: whole x lines, up to the limit above)
     if (rc != AWFL_OK) return rc;
   }
   c->dimSwitch = !c->dimSwitch;

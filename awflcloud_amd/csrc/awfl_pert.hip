@@ -191,9 +191,9 @@ struct Sweep32 {
 };
 
 template <int ORD, int NGLL, int DIR, int TX>
-__global__ __launch_bounds__(awfl_tile::MAX_THREADS) void k_sweep_tile_f32(const float* s, const float* c, float* so,
+__global__ __launch_bounds__(awfl_cut::MAX_THREADS) void k_sweep_tile_f32(const float* s, const float* c, float* so,
                                                                            float* co, GridF G, SweepKF K,
-                                                                           awfl_tile::TilePlan T) {
+                                                                           awfl_cut::TilePlan T) {
   awfl_tile::sweep(Sweep32<ORD, NGLL, DIR, TX>{s, c, so, co, G, K}, T);
 }
 
@@ -356,7 +356,7 @@ __global__ void k_from_f32(const float* __restrict__ s, const float* __restrict_
     d[t] = (double)s[t] - (double)c[t];
 }
 
-using TileFnF = void (*)(const float*, const float*, float*, float*, GridF, SweepKF, awfl_tile::TilePlan);
+using TileFnF = void (*)(const float*, const float*, float*, float*, GridF, SweepKF, awfl_cut::TilePlan);
 using ColFnF = void (*)(const float*, const float*, float*, float*, GridF, SweepKF, int);
 struct VariantF {
   int ord, ngll;
@@ -468,12 +468,6 @@ SweepKF sweep_constants_f(const awfl_ctx* c, double dt, int dir) {
   return K;
 }
 
-// Rates of the FP32 kernels for the cuts.  Fitted to: tiles 8 us at 64x64x32 (y
-// and z; the walkers 46 and 43), 25 at 120x100x60 (51 and 56), 33 at 128x128x64
-// (48), 108 and 112-128 at 192x192x96 (103 and 104), 234 and 260 at 256x256x128
-// (230 and 218), 1947 and 1999 at 512x512x256 (1545 and 1609).
-constexpr awfl_tile::Rates RATES_F32{1.75, 1.2, {1.15, 1.18, 1.12, 1.07}, 1.4, 1.0, 2.7};
-
 int launch_sweep_f32(awfl_ctx* c, const float* s, const float* cs, float* so, float* co, double dt, int dir) {
   GridF F = grid_f(c);
   SweepKF K = sweep_constants_f(c, dt, dir);
@@ -491,15 +485,15 @@ int launch_sweep_f32(awfl_ctx* c, const float* s, const float* cs, float* so, fl
   const int n = dir == 1 ? c->cfg.ny : c->cfg.nz;
   const int other = dir == 1 ? c->cfg.nz : c->cfg.ny;
   const int bc = dir == 1 ? c->cfg.bc_y : c->cfg.bc_z;
-  const awfl_tile::TileCut cut = awfl_tile::tile_cut(dir, n, c->cfg.nx, other, bc == AWFL_BC_PERIODIC, RATES_F32);
-  const awfl_tile::WalkCut walk = awfl_tile::walk_cut(n, c->cfg.nx, other, RATES_F32);
+  const awfl_cut::TileCut cut = awfl_cut::tile_cut(dir, n, c->cfg.nx, other, bc == AWFL_BC_PERIODIC, awfl_cut::RATES_F32);
+  const awfl_cut::WalkCut walk = awfl_cut::walk_cut(n, c->cfg.nx, other, awfl_cut::RATES_F32);
   if (walk.us < cut.us) {
     v->col[dir - 1]<<<dim3(walk.bx, other, walk.nseg), 64, 0, c->stream>>>(s, cs, so, co, F, K, walk.seglen);
     LAUNCH_CHECK(c);
     return AWFL_OK;
   }
   const TileFnF k = v->yz[dir - 1][cut.tx];
-  const size_t lds = sizeof(float) * awfl_tile::lds_elems(cut.p, c->hs);
+  const size_t lds = sizeof(float) * awfl_cut::lds_elems(cut.p, c->hs);
   k<<<dim3((c->cfg.nx + cut.p.cols - 1) / cut.p.cols, other, cut.p.nseg), cut.threads, lds, c->stream>>>(s, cs, so, co,
                                                                                                          F, K, cut.p);
   LAUNCH_CHECK(c);

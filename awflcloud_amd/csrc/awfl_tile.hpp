@@ -29,9 +29,7 @@
 // second reconstructions, but its loop takes the FP64 kernel to 144-168
 // registers (spills at 128).
 #pragma once
-#include <algorithm>
-#include <cstdint>
-
+#include "awfl_cut.hpp"
 #include "awfl_internal.hpp"
 #include "awfl_tables.hpp"
 
@@ -39,16 +37,7 @@ namespace awfl_tile {
 
 using awfl::sfor;
 
-// How a sweep is cut: lines per work-group, rows (lanes along a line),
-// segments per line and their length.
-struct TilePlan {
-  int cols, rows, nseg, seglen;
-};
-
-constexpr int MAX_THREADS = 1024;
-
-// LDS elements of a work-group: staged cells and face slots
-inline size_t lds_elems(const TilePlan& p, int hs) { return (size_t)5 * p.cols * (2 * p.rows + 2 * hs + 1); }
+using awfl_cut::TilePlan;
 
 // P supplies the scalar (P::real), ORD, DIR, TX (lines of a y or z tile, x
 // fastest; x tiles take p.cols lines along y), and over its arguments A:
@@ -196,80 +185,6 @@ __device__ __forceinline__ void sweep(const P& A, const TilePlan& T) {
     });
     A.put(o, line, a, line_base(line) + a * sa, cell, F, F1, src);
   }
-}
-
-// ---------------------------------------------------------------------------
-// the cut
-// ---------------------------------------------------------------------------
-// TX choices of y and z tiles
-constexpr int TX_OF[3] = {4, 8, 16};
-
-// Rates of a sweep's kernels for the models below, in microseconds: a tile's
-// wave (one cell a lane), the factor of 4-line tiles (short runs of memory),
-// the factors of work-groups of 5 to 8 waves (how they pack on a CU), and the
-// column walker's step with x waves on a SIMD, max(walk_least, walk x + walk_0).
-struct Rates {
-  double tile, narrow, pack[4];
-  double walk, walk_0, walk_least;
-};
-
-struct TileCut {
-  int tx;                     // index into TX_OF (y, z)
-  TilePlan p;
-  int threads;
-  double us;                  // modelled time
-};
-
-// Cut of a sweep of n-cell lines, nline of them side by side in each of `other`
-// rows: the one of least modelled time, a tile's latency (some 5 us from its
-// loads to its stores) plus the issue time of the waves that a SIMD gets (256
-// CUs of four SIMDs; small grids in whole rounds).  An idle lane costs three
-// quarters of a busy one.  x lines up to 1024 cells stay whole (they may be
-// updated in place).
-inline TileCut tile_cut(int dir, int n, int nline, int other, bool per, const Rates& rate) {
-  TileCut best{};
-  best.us = 1e300;
-  auto consider = [&](int tx, int cols, int nseg, int limit) {
-    const int seglen = (n + nseg - 1) / nseg;
-    if ((n + seglen - 1) / seglen != nseg) return;
-    const int rows = nseg == 1 ? n : !per && nseg == 2 ? seglen + 1 : seglen + 2;
-    if (rows * cols > limit) return;
-    const int waves = (rows * cols + 63) / 64;
-    const double wgs = (double)nseg * ((nline + cols - 1) / cols) * other;
-    const double rounds = wgs <= 1024 ? (double)(((int64_t)wgs + 255) / 256) : wgs / 256;
-    const double eq = (0.75 * waves + 0.25 * rows * cols / 64.0) * (waves > 4 ? rate.pack[std::min(waves, 8) - 5] : 1.0) *
-                      (dir > 0 && cols == 4 ? rate.narrow : 1.0);
-    const double us = 5.0 + rate.tile * std::max(rounds * eq / 4, (double)((waves + 3) / 4));
-    if (us < best.us) best = TileCut{tx, TilePlan{cols, rows, nseg, seglen}, waves * 64, us};
-  };
-  if (dir == 0) {
-    for (int cols = 1; cols <= std::max(1, std::min(nline, 512 / n)); cols++) consider(0, cols, 1, MAX_THREADS);
-    for (int nseg = 2; best.us == 1e300; nseg++) consider(0, 1, nseg, MAX_THREADS);
-  } else {
-    for (int x = 0; x < 3; x++)
-      for (int nseg = 1; nseg <= std::max(1, n / 14); nseg++) consider(x, TX_OF[x], nseg, 512);
-  }
-  return best;
-}
-
-// Cut of a column-walker sweep (a lane walks a segment of its column; y and z):
-// segments of at most 32 cells, and shorter (down to 16) where that is needed
-// for ~4 waves per SIMD.  Modelled time: every wave reconstructs two cells more
-// than its segment has.
-struct WalkCut {
-  int bx, nseg, seglen;
-  double us;
-};
-inline WalkCut walk_cut(int n, int nx, int other, const Rates& rate) {
-  WalkCut w{};
-  w.bx = (nx + 63) / 64;
-  const int64_t layer = (int64_t)w.bx * other;
-  const int nseg = (int)std::max<int64_t>(1, std::min<int64_t>(std::max<int64_t>((4096 + layer - 1) / layer, (n + 31) / 32),
-                                                               std::max(1, n / 16)));
-  w.seglen = (n + nseg - 1) / nseg;
-  w.nseg = (n + w.seglen - 1) / w.seglen;
-  w.us = (w.seglen + 2) * std::max(rate.walk * (double)(layer * w.nseg) / 1024.0 + rate.walk_0, rate.walk_least);
-  return w;
 }
 
 }  // namespace awfl_tile

@@ -1,5 +1,7 @@
 // Prints what awflcloud_amd/csrc/awfl_cut.hpp answers, one line per line of
-// standard input: "adj n lines" -> lines per work-group.
+// standard input: "adj n lines" -> lines per work-group; "tile dir n nline other
+// periodic whole" -> lines, rows, segments, segment length, threads and LDS bytes of
+// an FP64 tile.
 #include <cstdio>
 #include <cstring>
 
@@ -13,6 +15,12 @@ int main() {
       long long lines;
       if (std::scanf("%d %lld", &n, &lines) != 2) return 1;
       std::printf("%d\n", awfl_cut::adj_cols(n, lines));
+    } else if (!std::strcmp(what, "tile")) {
+      int dir, n, nline, other, per, whole;
+      if (std::scanf("%d %d %d %d %d %d", &dir, &n, &nline, &other, &per, &whole) != 6) return 1;
+      const awfl_cut::TileCut t = awfl_cut::tile_cut(dir, n, nline, other, per, awfl_cut::rates_f64(dir), whole);
+      std::printf("%d %d %d %d %d %zu\n", t.p.cols, t.p.rows, t.p.nseg, t.p.seglen, t.threads,
+                  sizeof(double) * awfl_cut::lds_elems(t.p, 2));
     } else {
       return 1;
     }

@@ -33,3 +33,33 @@ def test_adjoint_lines_of_five_waves_share_a_group(cuts):
         for lines in (257, 312, 1008, 6400):
             assert cuts(["adj %d %d" % (n, lines)]) == [["2"]]
         assert cuts(["adj %d 224" % n]) == [["1"]]
+
+
+def _check_tile(n, per, cut, lanes):
+    cols, rows, nseg, seglen, threads, lds = (int(v) for v in cut)
+    assert cols >= 1 and cols * rows <= threads <= lanes and threads % 64 == 0 and lds <= 160 * 1024
+    assert nseg * seglen >= n and (nseg - 1) * seglen < n            # every segment has a cell
+    # a segment holds its neighbours' end cells too, where the line has them
+    assert rows >= (n if nseg == 1 else seglen + (1 if not per and nseg == 2 else 2))
+    return cols, nseg
+
+
+def test_tiles_fit(cuts):
+    asked = [(d, n, nline, other, per, 0) for d in (0, 1, 2) for n in list(range(1, 600)) + [683, 700, 768, 1000, 1024, 1027, 1364]
+             for nline, other in ((1, 1), (37, 5), (160, 64)) for per in (0, 1)]
+    for a, cut in zip(asked, cuts(["tile %d %d %d %d %d %d" % a for a in asked])):
+        _check_tile(a[1], a[4], cut, 512)
+
+
+def test_lines_updated_in_place_are_whole(cuts):
+    asked = [(0, n, nline, 5, per, 1) for n in range(1, 1025) for nline in (1, 160) for per in (0, 1)]
+    for a, cut in zip(asked, cuts(["tile %d %d %d %d %d %d" % a for a in asked])):
+        assert _check_tile(a[1], a[4], cut, 1024)[1] == 1
+
+
+def test_long_x_lines_run_in_segments(cuts):
+    # a group of nine waves or more was slower than the segments at each of these
+    for n in (513, 560, 600, 640, 700, 800, 1000, 1024):
+        for nline, other in ((48, 32), (160, 64)):
+            (cut,) = cuts(["tile 0 %d %d %d 1 0" % (n, nline, other)])
+            assert int(cut[2]) >= 2 and int(cut[4]) <= 256
