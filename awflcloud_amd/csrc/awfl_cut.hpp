@@ -2,6 +2,7 @@
 // code alone, with the timings that they rest on.
 #pragma once
 #include <algorithm>
+#include <cmath>
 #include <cstddef>
 #include <cstdint>
 
@@ -27,31 +28,50 @@ constexpr int TX_OF[3] = {4, 8, 16};
 // Rates of a sweep's kernels for the models below, in microseconds: a tile's
 // wave (one cell a lane), the factor of 4-line tiles (short runs of memory),
 // the factors of work-groups of 5 to 8 waves (how they pack on a CU), and the
-// column walker's step with x waves on a SIMD, max(walk_least, walk x + walk_0).
+// column walker's step with x waves on a SIMD, max(walk_least, walk x + walk_0); x
+// up to whole_x counts as the next whole number (a SIMD's last round costs as much
+// with one wave on a few of them as on all).
 struct Rates {
   double tile, narrow, pack[4];
   double walk, walk_0, walk_least;
+  double whole_x;
 };
 
-// Rates of the (5, 3) kernels, which the cuts of the other orders share (a
-// ratio of the two kernels' times is all that they decide).  Fitted to sweeps
-// of 64x64x32 to 512x512x256 cells, every cut timed: best tiles 9 us at 64x64x32
-// (y and z; the walkers 55), 43 and 45 at 128x128x64 (57 and 62), 84 and 92 at
-// 160x160x80 (124 and 131), 147 and 161 at 192x192x96 (160 and 167), 228 and 271
-// at 96x300x200 (319 and 364), 340 and 393 at 256x256x128 (330 and 340).  The z
-// kernel has 112 registers, four waves per SIMD, which work-groups of five to
-// eight waves fill badly.
-inline const Rates& rates_f64(int dir) {
-  static constexpr Rates xy{2.55, 1.03, {1.15, 1.18, 1.12, 1.07}, 2.3, 0.8, 3.2};
-  static constexpr Rates z{2.6, 1.03, {1.4, 1.33, 1.2, 1.15}, 2.35, 0.9, 3.4};
-  return dir == 2 ? z : xy;
+// FP64.  The (5, 3) rates are fitted to sweeps of 64x64x32 to 512x512x256 cells,
+// every cut timed: best tiles 9 us at 64x64x32 (y and z; the walkers 55), 43 and 45
+// at 128x128x64 (57 and 62), 84 and 92 at 160x160x80 (124 and 131), 147 and 161 at
+// 192x192x96 (160 and 167), 228 and 271 at 96x300x200 (319 and 364), 340 and 393 at
+// 256x256x128 (330 and 340).  The z kernel has 112 registers, four waves per SIMD,
+// which work-groups of five to eight waves fill badly.  At (3, 2) the walkers are
+// ahead earlier, in z above all, which rates of their own say (the tile's factors, and
+// so its cut, are (5, 3)'s).  Fitted to 860 grids of 0.02 to 12 million cells, both
+// forms timed: z tile and walker 355 and 284 us at 1000x160x64, 230 and 183 at
+// 600x160x64, 157 and 116 at 1101x616x6, 34 and 42 at 128x128x64, 92 and 106 at
+// 512x100x60.  They choose the slower form by more than 2% at 14 (y) and 17 (z) of the
+// grids; (5, 3)'s did at 31 and 68, by up to 31%.
+inline const Rates& rates_f64(int dir, int ord) {
+  static constexpr Rates xy{2.55, 1.03, {1.15, 1.18, 1.12, 1.07}, 2.3, 0.8, 3.2, 0.0};
+  static constexpr Rates z{2.6, 1.03, {1.4, 1.33, 1.2, 1.15}, 2.35, 0.9, 3.4, 0.0};
+  static constexpr Rates y3{2.42, 1.03, {1.15, 1.18, 1.12, 1.07}, 1.77, 1.25, 3.24, 8.0};
+  static constexpr Rates z3{1.51, 1.03, {1.4, 1.33, 1.2, 1.15}, 1.08, 0.62, 2.51, 8.0};
+  if (ord == 3) return dir < 2 ? y3 : z3;
+  return dir < 2 ? xy : z;
 }
 
-// Rates of the FP32 kernels for the cuts.  Fitted to: tiles 8 us at 64x64x32 (y
-// and z; the walkers 46 and 43), 25 at 120x100x60 (51 and 56), 33 at 128x128x64
-// (48), 108 and 112-128 at 192x192x96 (103 and 104), 234 and 260 at 256x256x128
-// (230 and 218), 1947 and 1999 at 512x512x256 (1545 and 1609).
-constexpr Rates RATES_F32{1.75, 1.2, {1.15, 1.18, 1.12, 1.07}, 1.4, 1.0, 2.7};
+// FP32.  Fitted at (5, 3) to: tiles 8 us at 64x64x32 (y and z; the walkers 46 and
+// 43), 25 at 120x100x60 (51 and 56), 33 at 128x128x64 (48), 108 and 112-128 at
+// 192x192x96 (103 and 104), 234 and 260 at 256x256x128 (230 and 218), 1947 and 1999 at
+// 512x512x256 (1545 and 1609).  At (3, 2) to 860 grids as above:
+// z 162 (tile) and 140 (walker) at 600x160x64, 102 and 78 at 192x192x96, 24 and 35 at
+// 128x128x64, 94 and 80 at 518x102x66; y 59 and 55 at 512x100x60, 102 and 78 at
+// 192x192x96, 156 and 185 at 96x300x200.  Slower by more than 2% at 16 (y) and 20 (z) of
+// them; with (5, 3)'s 27 and 33, by up to 45%.
+inline const Rates& rates_f32(int dir, int ord) {
+  static constexpr Rates yz{1.75, 1.2, {1.15, 1.18, 1.12, 1.07}, 1.4, 1.0, 2.7, 0.0};
+  static constexpr Rates y3{1.60, 1.2, {1.15, 1.18, 1.12, 1.07}, 0.92, 1.79, 0.87, 0.0};
+  static constexpr Rates z3{1.35, 1.2, {1.15, 1.18, 1.12, 1.07}, 0.89, 1.06, 3.08, 0.0};
+  return ord != 3 ? yz : dir == 1 ? y3 : z3;
+}
 
 struct TileCut {
   int tx;                     // index into TX_OF (y, z)
@@ -114,7 +134,9 @@ inline WalkCut walk_cut(int n, int nx, int other, const Rates& rate) {
                                                                std::max(1, n / 16)));
   w.seglen = (n + nseg - 1) / nseg;
   w.nseg = (n + w.seglen - 1) / w.seglen;
-  w.us = (w.seglen + 2) * std::max(rate.walk * (double)(layer * w.nseg) / 1024.0 + rate.walk_0, rate.walk_least);
+  double x = (double)(layer * w.nseg) / 1024.0;
+  if (x <= rate.whole_x) x = std::ceil(x);
+  w.us = (w.seglen + 2) * std::max(rate.walk * x + rate.walk_0, rate.walk_least);
   return w;
 }
 

@@ -994,7 +994,7 @@ static int launch_tile(awfl_ctx* c, const double* in, double* out, const SweepK&
   const int bc = dir == 0 ? c->cfg.bc_x : dir == 1 ? c->cfg.bc_y : c->cfg.bc_z;
   const awfl_cut::TileCut cut = known ? *known
                                       : awfl_cut::tile_cut(dir, n, nline, other, bc == AWFL_BC_PERIODIC,
-                                                           awfl_cut::rates_f64(dir), in == out);
+                                                           awfl_cut::rates_f64(dir, c->cfg.ord), in == out);
   const TileFn k = dir == 0 ? f.x : f.yz[dir - 1][cut.tx];
   const size_t lds = sizeof(double) * awfl_cut::lds_elems(cut.p, c->hs);
   if (lds > 64 * 1024)
@@ -1014,7 +1014,7 @@ static int launch_cells(awfl_ctx* c, const double* in, double* out, const SweepK
   const int n = dir == 1 ? c->cfg.ny : c->cfg.nz;
   const int other = dir == 1 ? c->cfg.nz : c->cfg.ny;
   const int bc = dir == 1 ? c->cfg.bc_y : c->cfg.bc_z;
-  const awfl_cut::Rates& rate = awfl_cut::rates_f64(dir);
+  const awfl_cut::Rates& rate = awfl_cut::rates_f64(dir, c->cfg.ord);
   const awfl_cut::TileCut cut = awfl_cut::tile_cut(dir, n, c->cfg.nx, other, bc == AWFL_BC_PERIODIC, rate);
   const awfl_cut::WalkCut walk = awfl_cut::walk_cut(n, c->cfg.nx, other, rate);
   if (cut.us <= walk.us) return launch_tile(c, in, out, K, dir, v->tile[tend], &cut);

@@ -1,7 +1,7 @@
 // Prints what awflcloud_amd/csrc/awfl_cut.hpp answers, one line per line of
 // standard input: "adj n lines" -> lines per work-group; "tile dir n nline other
 // periodic whole" -> lines, rows, segments, segment length, threads and LDS bytes of
-// an FP64 tile.
+// an FP64 tile; "form bits dir ord nx ny nz periodic" -> the faster form by the models.
 #include <cstdio>
 #include <cstring>
 
@@ -18,9 +18,15 @@ int main() {
     } else if (!std::strcmp(what, "tile")) {
       int dir, n, nline, other, per, whole;
       if (std::scanf("%d %d %d %d %d %d", &dir, &n, &nline, &other, &per, &whole) != 6) return 1;
-      const awfl_cut::TileCut t = awfl_cut::tile_cut(dir, n, nline, other, per, awfl_cut::rates_f64(dir), whole);
+      const awfl_cut::TileCut t = awfl_cut::tile_cut(dir, n, nline, other, per, awfl_cut::rates_f64(dir, 5), whole);
       std::printf("%d %d %d %d %d %zu\n", t.p.cols, t.p.rows, t.p.nseg, t.p.seglen, t.threads,
                   sizeof(double) * awfl_cut::lds_elems(t.p, 2));
+    } else if (!std::strcmp(what, "form")) {
+      int bits, dir, ord, nx, ny, nz, per;
+      if (std::scanf("%d %d %d %d %d %d %d", &bits, &dir, &ord, &nx, &ny, &nz, &per) != 7) return 1;
+      const awfl_cut::Rates& r = bits == 64 ? awfl_cut::rates_f64(dir, ord) : awfl_cut::rates_f32(dir, ord);
+      const int n = dir == 1 ? ny : nz, other = dir == 1 ? nz : ny;
+      std::puts(awfl_cut::tile_cut(dir, n, nx, other, per, r).us <= awfl_cut::walk_cut(n, nx, other, r).us ? "tile" : "walker");
     } else {
       return 1;
     }

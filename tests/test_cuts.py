@@ -63,3 +63,37 @@ def test_long_x_lines_run_in_segments(cuts):
         for nline, other in ((48, 32), (160, 64)):
             (cut,) = cuts(["tile 0 %d %d %d 1 0" % (n, nline, other)])
             assert int(cut[2]) >= 2 and int(cut[4]) <= 256
+
+
+# bits, direction, ord, grid, the form that was measured faster
+MEASURED = [
+    (64, 2, 3, (1000, 160, 64), "walker"),
+    (64, 2, 3, (600, 160, 64), "walker"),
+    (64, 2, 3, (1101, 616, 6), "walker"),
+    (64, 2, 3, (512, 256, 128), "walker"),
+    (64, 2, 3, (512, 100, 60), "tile"),
+    (64, 2, 3, (128, 128, 64), "tile"),
+    (64, 2, 3, (64, 64, 32), "tile"),
+    (64, 1, 3, (1000, 160, 64), "walker"),
+    (64, 1, 3, (130, 96, 64), "tile"),
+    (64, 1, 3, (541, 2, 340), "walker"),
+    (64, 2, 5, (256, 256, 128), "walker"),
+    (64, 2, 5, (96, 300, 200), "tile"),
+    (32, 2, 3, (600, 160, 64), "walker"),
+    (32, 2, 3, (192, 192, 96), "walker"),
+    (64, 2, 3, (332, 317, 5), "walker"),
+    (64, 2, 3, (1214, 40, 75), "walker"),
+    (32, 2, 3, (518, 102, 66), "walker"),
+    (32, 2, 3, (795, 186, 30), "walker"),
+    (32, 1, 3, (760, 22, 216), "walker"),
+    (32, 2, 3, (100, 90, 75), "tile"),
+    (32, 2, 3, (128, 128, 64), "tile"),
+    (32, 1, 3, (512, 100, 60), "walker"),
+    (32, 2, 5, (512, 512, 256), "walker"),
+    (32, 2, 5, (128, 128, 64), "tile"),
+]
+
+
+@pytest.mark.parametrize("bits,d,ord,grid,form", MEASURED)
+def test_form_is_the_one_measured_faster(cuts, bits, d, ord, grid, form):
+    assert cuts(["form %d %d %d %d %d %d %d" % ((bits, d, ord) + grid + (int(d < 2),))]) == [[form]]
