@@ -89,7 +89,9 @@ struct TileCut {
 // segments: a group of 9 to 16 waves leaves a CU's places empty and its barriers
 // uncovered (160 x 64 lines at (5, 3), whole against the best segments: 513 cells
 // 336 and 219 us, 640 356 and 273, 800 435 and 328, 1024 456 and 427; at (3, 2) 249
-// and 158, 269 and 194, 328 and 234, 345 and 311).
+// and 158, 269 and 194, 328 and 234, 345 and 311).  Short x lines fill a wave where
+// there are as many (8x91x9, one line against 8 to a group: 11.1 and 6.0 us at (5, 3),
+// 8.1 and 5.3 at (3, 2)).
 inline TileCut tile_cut(int dir, int n, int nline, int other, bool per, const Rates& rate, bool whole = false) {
   TileCut best{};
   best.us = 1e300;
@@ -108,7 +110,8 @@ inline TileCut tile_cut(int dir, int n, int nline, int other, bool per, const Ra
   };
   if (dir == 0) {
     if (whole || n <= 512)
-      for (int cols = 1; cols <= std::max(1, std::min(nline, 512 / n)); cols++) consider(0, cols, 1, MAX_THREADS);
+      for (int cols = std::max(1, std::min(nline, 64 / n)); cols <= std::max(1, std::min(nline, 512 / n)); cols++)
+        consider(0, cols, 1, MAX_THREADS);
     else
       for (int nseg = 2; nseg <= n / 64; nseg++) consider(0, 1, nseg, 512);
   } else {

@@ -65,6 +65,12 @@ def test_long_x_lines_run_in_segments(cuts):
             assert int(cut[2]) >= 2 and int(cut[4]) <= 256
 
 
+def test_short_x_lines_fill_a_wave(cuts):
+    for n, nline, other in ((8, 91, 9), (2, 100, 50), (6, 50, 6), (16, 40, 30), (20, 60, 60), (33, 40, 30)):
+        (cut,) = cuts(["tile 0 %d %d %d 1 0" % (n, nline, other)])
+        assert int(cut[0]) >= 64 // n
+
+
 # bits, direction, ord, grid, the form that was measured faster
 MEASURED = [
     (64, 2, 3, (1000, 160, 64), "walker"),
