@@ -144,6 +144,67 @@ inline WalkCut walk_cut(int n, int nx, int other, const Rates& rate) {
 }
 
 // ---------------------------------------------------------------------------
+// tracer tiles and walkers (k_tile_tr, k_walk_tr in awfl_tracers.hip)
+// ---------------------------------------------------------------------------
+constexpr int TT_MAX = 1024;    // lanes of a work-group
+
+constexpr int tt_stride(int ntr) { return ntr | 1; }
+inline size_t tt_lds(int n, int cols, int hs, int ntr) {
+  const size_t ts = tt_stride(ntr);
+  return sizeof(double) * cols * ((5 + ts) * (n + 2 * hs) + (5 + 2 * ts) * (n + 1));
+}
+
+// Lines per work-group of a tile, and its modelled cost per cell in waves of
+// full lanes: the idle lanes of the waves, the waves a CU holds (16, by the
+// registers; work-groups of 5 to 8 waves fit twice, larger ones and those that
+// fill the LDS once, and a lone group idles at its barriers), and in y and z the
+// runs of `cols` neighbouring lines that a load covers.  Measured, y at
+// 256x256x128 with 3 tracers: 1 line 791 us, 2 (8 waves) 662, 3 (12 waves) 953, 4
+// (16 waves) 856; z: 1 line 1110, 2 747, 3 (6 waves) 974, 4 (8 waves) 670, 5 (10
+// waves) 1065, 6 (12 waves) 915, 8 (16 waves) 835.
+struct TtCut {
+  int cols;
+  double cost;
+};
+inline TtCut tt_cut(int dir, int n, int64_t lines, int hs, int ntr) {
+  TtCut best{0, 1e300};
+  for (int m = 1; m * n <= TT_MAX && (m == 1 || (lines + m - 1) / m >= 256); m++) {
+    const int waves = (m * n + 63) / 64;
+    const size_t lds = tt_lds(n, m, hs, ntr);
+    if (lds > 160 * 1024) break;
+    const int groups = (int)std::min<size_t>(waves <= 4 ? 16 / waves : waves <= 8 ? 2 : 1, 160 * 1024 / lds);
+    const double runs = dir == 0 || m >= 4 ? 1.0 : m == 3 ? 1.05 : m == 2 ? 1.11 : 1.33;
+    // a small grid needs fewer waves than a CU holds, but whole rounds of groups
+    const double need = std::min(16.0, (double)lines * n / 64 / 256);
+    const double held = std::max(1.0, need / (groups * waves)) * (groups == 1 ? 1.4 : 1.0);
+    const int64_t wgs = (lines + m - 1) / m;
+    const double rounds = wgs <= 1024 && wgs >= 256 ? (wgs + 255) / 256 * 256.0 / wgs : 1.0;
+    const double cost = 64.0 * waves / (m * n) * held * rounds * runs * (waves == 1 ? 1.06 : waves == 2 ? 1.03 : 1.0);
+    if (cost < best.cost * 0.999) best = TtCut{m, cost};
+  }
+  return best;
+}
+
+// Tile or walker for y and z lines, of `groups` walker work-groups: the walker's
+// waves take steps of 64 cells of a line, the tile pays for idle lanes and short runs
+// but not for the walker's head, tail and carries.  Around the line at (5, 3): y at n =
+// 256 (cost 1.11 of the walker's) 662 against 704 us, 210 (1.33) 225 and 240, 150 (1.42)
+// 486 and 552, 400 (1.5) 78 and 71, 300 (1.6) 607 and 422; z at 128 (1.0) 670 and 777,
+// 150 (1.42) 577 and 566, 180 (1.42) 238 and 230.  The walker of (3, 2) gains more on its
+// tile where that takes single y lines and there are few tracers (so that the walker's
+// LDS lets a CU hold its waves), once the grid fills the chip: 39x456x215 with one tracer
+// 303 (tile) and 231 us, 92x449x80 with three 364 and 287, 59x189x181 with three 171 and
+// 157; but with five 520 and 594 at 237x147x116.  A grid with fewer walker groups than
+// CUs waits for one walk: 17x520x10 with five tracers 24 (tile) and 91 us, 57x6x388
+// with eight 48 and 101 (z).
+inline bool tt_tile(const TtCut& cut, int dir, int ord, int n, int64_t groups, int ntr) {
+  if (groups <= 192) return true;
+  const double walker = (n + 63) / 64 * 64.0 / n;
+  const bool quick = dir == 2 || (ord == 3 && ntr < 4 && groups > 1024);
+  return cut.cost < (quick ? 1.3 : 1.45) * walker;
+}
+
+// ---------------------------------------------------------------------------
 // sweep adjoint (k_adj_tile in awfl_adjoint.hip)
 // ---------------------------------------------------------------------------
 // Cells of a line, lanes of a work-group: the twelve waves that a CU holds.  The

@@ -43,6 +43,7 @@
 #include <algorithm>
 
 #include "awfl_cell.hpp"
+#include "awfl_cut.hpp"
 #include "awfl_internal.hpp"
 #include "awfl_profiles.hpp"
 
@@ -441,16 +442,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
 // 128x128x64 with 5 tracers 86, 95 and 95 against 128, 148 and 177; at 64x64x32
 // 15 against 16, 22 and 35.
 // ---------------------------------------------------------------------------
-constexpr int TT_MAX = 1024;    // lanes of a work-group
-
-inline int tt_stride(int ntr) { return ntr | 1; }
-inline size_t tt_lds(int n, int cols, int hs, int ntr) {
-  const size_t ts = tt_stride(ntr);
-  return sizeof(double) * cols * ((5 + ts) * (n + 2 * hs) + (5 + 2 * ts) * (n + 1));
-}
-
 template <int ORD, int NGLL, int DIR, bool TEND>
-__global__ __launch_bounds__(TT_MAX) __attribute__((amdgpu_waves_per_eu(4))) void k_tile_tr(
+__global__ __launch_bounds__(awfl_cut::TT_MAX) __attribute__((amdgpu_waves_per_eu(4))) void k_tile_tr(
     const double* __restrict__ in, const double* __restrict__ tr_in, double* __restrict__ out,
     double* __restrict__ tr_out, Grid G, SweepK K, int ntr, unsigned pos, int cols) {
   constexpr int hs = (ORD - 1) / 2;
@@ -458,7 +451,7 @@ __global__ __launch_bounds__(TT_MAX) __attribute__((amdgpu_waves_per_eu(4))) voi
   constexpr int NA = NGLL;
   extern __shared__ double sm[];
   const int n = axis_n(G, DIR);
-  const int ts = ntr | 1;
+  const int ts = awfl_cut::tt_stride(ntr);
   const bool per = G.bc[DIR] == AWFL_BC_PERIODIC;
   const int t = threadIdx.x;
   const int col = DIR == 0 ? t / n : t % cols;
@@ -689,37 +682,6 @@ __global__ __launch_bounds__(TT_MAX) __attribute__((amdgpu_waves_per_eu(4))) voi
       else tr_out[q * G.sl + o] = tr_in[q * G.sl + o] + K.dt * td;
     }
   }
-}
-
-// Lines per work-group of a tile, and its modelled cost per cell in waves of
-// full lanes: the idle lanes of the waves, the waves a CU holds (16, by the
-// registers; work-groups of 5 to 8 waves fit twice, larger ones and those that
-// fill the LDS once, and a lone group idles at its barriers), and in y and z the
-// runs of `cols` neighbouring lines that a load covers.  Measured, y at
-// 256x256x128 with 3 tracers: 1 line 791 us, 2 (8 waves) 662, 3 (12 waves) 953, 4
-// (16 waves) 856; z: 1 line 1110, 2 747, 3 (6 waves) 974, 4 (8 waves) 670, 5 (10
-// waves) 1065, 6 (12 waves) 915, 8 (16 waves) 835.
-struct TtCut {
-  int cols;
-  double cost;
-};
-inline TtCut tt_cut(int dir, int n, int64_t lines, int hs, int ntr) {
-  TtCut best{0, 1e300};
-  for (int m = 1; m * n <= TT_MAX && (m == 1 || (lines + m - 1) / m >= 256); m++) {
-    const int waves = (m * n + 63) / 64;
-    const size_t lds = tt_lds(n, m, hs, ntr);
-    if (lds > 160 * 1024) break;
-    const int groups = (int)std::min<size_t>(waves <= 4 ? 16 / waves : waves <= 8 ? 2 : 1, 160 * 1024 / lds);
-    const double runs = dir == 0 || m >= 4 ? 1.0 : m == 3 ? 1.05 : m == 2 ? 1.11 : 1.33;
-    // a small grid needs fewer waves than a CU holds, but whole rounds of groups
-    const double need = std::min(16.0, (double)lines * n / 64 / 256);
-    const double held = std::max(1.0, need / (groups * waves)) * (groups == 1 ? 1.4 : 1.0);
-    const int64_t wgs = (lines + m - 1) / m;
-    const double rounds = wgs <= 1024 && wgs >= 256 ? (wgs + 255) / 256 * 256.0 / wgs : 1.0;
-    const double cost = 64.0 * waves / (m * n) * held * rounds * runs * (waves == 1 ? 1.06 : waves == 2 ? 1.03 : 1.0);
-    if (cost < best.cost * 0.999) best = TtCut{m, cost};
-  }
-  return best;
 }
 
 // ---------------------------------------------------------------------------
@@ -1406,21 +1368,14 @@ int launch_sweep_tr(awfl_ctx* c, const double* in, const double* tr_in, double* 
   const bool walks = dir > 0 && n >= 8 && v->wupd[dir - 1];
   const size_t lds = sizeof(double) * (size_t)(5 * W + ntr * W + 10 * n + 2 * ntr * n + (dir == 2 ? 2 : 1) * n);
   if (!walks && lds > 160 * 1024) return fail(c, AWFL_E_UNSUPPORTED, "tracers: line too long for the tracer sweep's LDS");
-  // Tile or walker: the walker's waves take steps of 64 cells of a line, the tile
-  // pays for idle lanes and short runs but not for the walker's head, tail and
-  // carries.  Around the line: y at n = 256 (cost 1.11 of the walker's) 662
-  // against 704 us, 210 (1.33) 225 and 240, 150 (1.42) 486 and 552, 400 (1.5)
-  // 78 and 71, 300 (1.6) 607 and 422; z at 128 (1.0) 670 and 777, 150 (1.42) 577
-  // and 566, 180 (1.42) 238 and 230.
   if (KernelTt k = v->tile[tend][dir]) {
-    const int64_t lines = nc / n;
-    const TtCut cut = tt_cut(dir, n, lines, c->hs, ntr);
-    const double walker = (n + 63) / 64 * 64.0 / n;
-    if (cut.cols && (!walks || cut.cost < (dir == 1 ? 1.45 : 1.3) * walker)) {
-      const size_t tlds = tt_lds(n, cut.cols, c->hs, ntr);
+    const awfl_cut::TtCut cut = awfl_cut::tt_cut(dir, n, nc / n, c->hs, ntr);
+    const int64_t groups = (int64_t)((c->cfg.nx + WK_WX - 1) / WK_WX) * (dir == 1 ? c->cfg.nz : c->cfg.ny);
+    if (cut.cols && (!walks || awfl_cut::tt_tile(cut, dir, c->cfg.ord, n, groups, ntr))) {
+      const size_t tlds = awfl_cut::tt_lds(n, cut.cols, c->hs, ntr);
       if (tlds > 64 * 1024)
         HIP_TRY(c, hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)tlds));
-      k<<<(unsigned)((lines + cut.cols - 1) / cut.cols), (cut.cols * n + 63) / 64 * 64, tlds, c->stream>>>(
+      k<<<(unsigned)((nc / n + cut.cols - 1) / cut.cols), (cut.cols * n + 63) / 64 * 64, tlds, c->stream>>>(
           in, tr_in, out, tr_out, c->grid(), sweep_constants(c, dt, dir), ntr, c->tpos, cut.cols);
       LAUNCH_CHECK(c);
       return AWFL_OK;

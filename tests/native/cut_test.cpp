@@ -1,7 +1,8 @@
 // Prints what awflcloud_amd/csrc/awfl_cut.hpp answers, one line per line of
 // standard input: "adj n lines" -> lines per work-group; "tile dir n nline other
 // periodic whole" -> lines, rows, segments, segment length, threads and LDS bytes of
-// an FP64 tile; "form bits dir ord nx ny nz periodic" -> the faster form by the models.
+// an FP64 tile; "form bits dir ord nx ny nz periodic" -> the faster form by the models;
+// "tracers dir ord nx ny nz ntr" -> form, lines per work-group of the tile and its LDS bytes.
 #include <cstdio>
 #include <cstring>
 
@@ -27,6 +28,14 @@ int main() {
       const awfl_cut::Rates& r = bits == 64 ? awfl_cut::rates_f64(dir, ord) : awfl_cut::rates_f32(dir, ord);
       const int n = dir == 1 ? ny : nz, other = dir == 1 ? nz : ny;
       std::puts(awfl_cut::tile_cut(dir, n, nx, other, per, r).us <= awfl_cut::walk_cut(n, nx, other, r).us ? "tile" : "walker");
+    } else if (!std::strcmp(what, "tracers")) {
+      int dir, ord, nx, ny, nz, ntr;
+      if (std::scanf("%d %d %d %d %d %d", &dir, &ord, &nx, &ny, &nz, &ntr) != 6) return 1;
+      const int n = dir == 0 ? nx : dir == 1 ? ny : nz;
+      const awfl_cut::TtCut t = awfl_cut::tt_cut(dir, n, (long long)nx * ny * nz / n, (ord - 1) / 2, ntr);
+      const bool tile = t.cols && (dir == 0 || n < 8 ||
+                                   awfl_cut::tt_tile(t, dir, ord, n, (long long)((nx + 3) / 4) * (dir == 1 ? nz : ny), ntr));
+      std::printf("%s %d %zu\n", tile ? "tile" : "walker", t.cols, awfl_cut::tt_lds(n, t.cols, (ord - 1) / 2, ntr));
     } else {
       return 1;
     }

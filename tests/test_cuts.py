@@ -103,3 +103,31 @@ MEASURED = [
 @pytest.mark.parametrize("bits,d,ord,grid,form", MEASURED)
 def test_form_is_the_one_measured_faster(cuts, bits, d, ord, grid, form):
     assert cuts(["form %d %d %d %d %d %d %d" % ((bits, d, ord) + grid + (int(d < 2),))]) == [[form]]
+
+
+def test_tracer_tiles_fit(cuts):
+    asked = [(d, o, nx, ny, nz, ntr) for d in (0, 1, 2) for o in (3, 5) for ntr in (0, 1, 3, 8)
+             for nx, ny, nz in ((1, 1, 1), (7, 5, 6), (63, 65, 64), (1024, 2, 3), (2, 1025, 9), (3, 4, 700), (300, 200, 100))]
+    for a, (form, cols, lds) in zip(asked, cuts(["tracers %d %d %d %d %d %d" % a for a in asked])):
+        n = a[2 + a[0]]
+        assert form == "tile" or a[0] == 0 or n >= 8          # shorter lines have no walker
+        assert int(cols) * n <= 1024 and (form == "walker" or int(lds) <= 160 * 1024)
+
+
+# direction, ord, grid, tracers, the form that was measured faster
+@pytest.mark.parametrize("d,ord,grid,ntr,form", [
+    (1, 3, (39, 456, 215), 1, "walker"),
+    (1, 3, (92, 449, 80), 3, "walker"),
+    (1, 3, (59, 189, 181), 3, "walker"),
+    (1, 3, (237, 147, 116), 5, "tile"),
+    (1, 3, (170, 249, 7), 2, "tile"),
+    (1, 3, (17, 520, 10), 5, "tile"),
+    (2, 3, (57, 6, 388), 8, "tile"),
+    (2, 3, (51, 11, 367), 1, "tile"),
+    (1, 5, (256, 256, 128), 3, "tile"),
+    (2, 5, (256, 256, 128), 3, "tile"),
+    (1, 5, (155, 287, 109), 3, "walker"),
+    (2, 5, (778, 23, 267), 3, "walker"),
+])
+def test_tracer_form_is_the_one_measured_faster(cuts, d, ord, grid, ntr, form):
+    assert cuts(["tracers %d %d %d %d %d %d" % ((d, ord) + grid + (ntr,))])[0][0] == form
