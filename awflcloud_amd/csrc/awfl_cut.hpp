@@ -143,6 +143,16 @@ inline WalkCut walk_cut(int n, int nx, int other, const Rates& rate) {
   return w;
 }
 
+// Groups of two waves with m lines each, of which some of the 256 CUs get a second
+// one: the two share a SIMD, which four waves alone do not.  The WENO3 adjoint along 36
+// cells of 636 lines takes 13.4 us by twos (318 groups) and 10.9 one by one, three
+// tracers along 63 cells of 770 lines 11.2 and 9.7.  Grids on which groups of one wave
+// leave a SIMD one at most do without.
+inline bool pairs_collide(int n, int m, int64_t lines) {
+  const int64_t groups = (lines + m - 1) / m;
+  return n <= 64 && m * n > 64 && m * n <= 128 && groups > 256 && groups <= 512 && lines <= 1024 * (64 / n);
+}
+
 // ---------------------------------------------------------------------------
 // tracer tiles and walkers (k_tile_tr, k_walk_tr in awfl_tracers.hip)
 // ---------------------------------------------------------------------------
@@ -170,6 +180,7 @@ inline TtCut tt_cut(int dir, int n, int64_t lines, int hs, int ntr) {
   TtCut best{0, 1e300};
   for (int m = 1; m * n <= TT_MAX && (m == 1 || (lines + m - 1) / m >= 256); m++) {
     const int waves = (m * n + 63) / 64;
+    if (dir == 0 && pairs_collide(n, m, lines)) continue;
     const size_t lds = tt_lds(n, m, hs, ntr);
     if (lds > 160 * 1024) break;
     const int groups = (int)std::min<size_t>(waves <= 4 ? 16 / waves : waves <= 8 ? 2 : 1, 160 * 1024 / lds);
@@ -233,6 +244,7 @@ inline int adj_cols(int n, int64_t lines) {
   double cost = 1e300;
   for (int m = 1; m * n <= 256 && (m == 1 || (lines + m - 1) / m >= 256); m++) {
     const int waves = (m * n + 63) / 64;
+    if (pairs_collide(n, m, lines)) continue;
     const double e = slack[waves] * waves / m;
     if (e < cost) {
       cost = e;

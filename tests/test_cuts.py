@@ -35,6 +35,15 @@ def test_adjoint_lines_of_five_waves_share_a_group(cuts):
         assert cuts(["adj %d 224" % n]) == [["1"]]
 
 
+def test_small_grids_without_colliding_pairs(cuts):
+    # two groups of two waves on a CU share a SIMD: slower at each of these, by the
+    # adjoint (cells of a line, lines) and by three tracers along x
+    for n, lines in ((36, 636), (45, 650), (43, 585), (34, 864)):
+        assert cuts(["adj %d %d" % (n, lines)]) == [["1"]]
+    for grid in ((63, 5, 154), (34, 12, 72), (40, 30, 30)):
+        assert cuts(["tracers 0 3 %d %d %d 3" % grid])[0][1] == "1"
+
+
 def _check_tile(n, per, cut, lanes):
     cols, rows, nseg, seglen, threads, lds = (int(v) for v in cut)
     assert cols >= 1 and cols * rows <= threads <= lanes and threads % 64 == 0 and lds <= 160 * 1024
