@@ -1017,7 +1017,7 @@ static int launch_cells(awfl_ctx* c, const double* in, double* out, const SweepK
   const awfl_cut::Rates& rate = awfl_cut::rates_f64(dir, c->cfg.ord);
   const awfl_cut::TileCut cut = awfl_cut::tile_cut(dir, n, c->cfg.nx, other, bc == AWFL_BC_PERIODIC, rate);
   const awfl_cut::WalkCut walk = awfl_cut::walk_cut(n, c->cfg.nx, other, rate);
-  if (cut.us <= walk.us) return launch_tile(c, in, out, K, dir, v->tile[tend], &cut);
+  if (c->form ? c->form == 1 : cut.us <= walk.us) return launch_tile(c, in, out, K, dir, v->tile[tend], &cut);
   v->col[dir - 1][tend]<<<dim3(walk.bx, other, walk.nseg), 64, 0, c->stream>>>(in, out, c->grid(), K, walk.seglen);
   LAUNCH_CHECK(c);
   return AWFL_OK;
@@ -1224,6 +1224,13 @@ static void timing_free(awfl_ctx* c) {
   c->t_ev.clear();
   c->t_dir.clear();
   c->t_n = 0;
+}
+
+int awfl_set_sweep_form(awfl_ctx* c, int form) {
+  if (!c) return AWFL_E_ARG;
+  if (form < 0 || form > 2) return fail(c, AWFL_E_ARG, "form must be 0 (by rule), 1 (tiles) or 2 (walkers)");
+  c->form = form;
+  return AWFL_OK;
 }
 
 int awfl_sweep_timing(awfl_ctx* c, int max_sweeps) {

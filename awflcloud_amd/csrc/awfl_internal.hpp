@@ -142,6 +142,7 @@ struct awfl_ctx {
   std::vector<hipEvent_t> t_ev;
   std::vector<int> t_dir;
   int t_n = 0;
+  int form = 0;                     // of y and z sweeps: 0 by rule, 1 tiles, 2 walkers (awfl_set_sweep_form)
   std::string err;
   Grid grid() const;
   int64_t state_elems() const {

@@ -488,7 +488,7 @@ int launch_sweep_f32(awfl_ctx* c, const float* s, const float* cs, float* so, fl
   const awfl_cut::Rates& rate = awfl_cut::rates_f32(dir, c->cfg.ord);
   const awfl_cut::TileCut cut = awfl_cut::tile_cut(dir, n, c->cfg.nx, other, bc == AWFL_BC_PERIODIC, rate);
   const awfl_cut::WalkCut walk = awfl_cut::walk_cut(n, c->cfg.nx, other, rate);
-  if (walk.us < cut.us) {
+  if (c->form ? c->form == 2 : walk.us < cut.us) {
     v->col[dir - 1]<<<dim3(walk.bx, other, walk.nseg), 64, 0, c->stream>>>(s, cs, so, co, F, K, walk.seglen);
     LAUNCH_CHECK(c);
     return AWFL_OK;

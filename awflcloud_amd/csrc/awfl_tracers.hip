@@ -1371,7 +1371,8 @@ int launch_sweep_tr(awfl_ctx* c, const double* in, const double* tr_in, double* 
   if (KernelTt k = v->tile[tend][dir]) {
     const awfl_cut::TtCut cut = awfl_cut::tt_cut(dir, n, nc / n, c->hs, ntr);
     const int64_t groups = (int64_t)((c->cfg.nx + WK_WX - 1) / WK_WX) * (dir == 1 ? c->cfg.nz : c->cfg.ny);
-    if (cut.cols && (!walks || awfl_cut::tt_tile(cut, dir, c->cfg.ord, n, groups, ntr))) {
+    const bool tile = c->form ? c->form == 1 : awfl_cut::tt_tile(cut, dir, c->cfg.ord, n, groups, ntr);
+    if (cut.cols && (!walks || tile)) {
       const size_t tlds = awfl_cut::tt_lds(n, cut.cols, c->hs, ntr);
       if (tlds > 64 * 1024)
         HIP_TRY(c, hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)tlds));

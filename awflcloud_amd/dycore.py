@@ -103,6 +103,7 @@ _SIGNATURES = {
     "awfl_apply_tendencies": ([_P, _P, _P, _D, C.c_int], C.c_int),
     "awfl_time_step": ([_P, _P, _D], C.c_int),
     "awfl_time_step_noalloc": ([_P, _P, _D], C.c_int),
+    "awfl_set_sweep_form": ([_P, C.c_int], C.c_int),
     "awfl_sweep_timing": ([_P, C.c_int], C.c_int),
     "awfl_sweep_times": ([_P, C.POINTER(C.c_double), C.POINTER(C.c_int64)], C.c_int),
     "awfl_time_step_branches": ([_P, _P, _D, _P, C.c_int], C.c_int),
@@ -280,6 +281,11 @@ class Dycore:
         n = (C.c_int64 * 3)()
         self._check(self.L.awfl_sweep_times(self.h, ms, n))
         return list(ms), list(n)
+
+    def set_sweep_form(self, form):
+        """the form of the y and z sweeps: 0 by rules on the grid, 1 tiles, 2
+        column walkers (awfl_set_sweep_form)"""
+        self._check(self.L.awfl_set_sweep_form(self.h, int(form)))
 
     def time_step_noalloc(self, state, dt):
         """time_step without any allocation (awfl_time_step_noalloc): its

@@ -130,6 +130,12 @@ int awfl_time_step_branches(awfl_ctx* ctx, double* d_state, double dt, unsigned 
  * ms and the number of timed sweeps since the previous call. */
 int awfl_sweep_timing(awfl_ctx* ctx, int max_sweeps);
 int awfl_sweep_times(awfl_ctx* ctx, double ms[3], int64_t count[3]);
+/* Diagnostic, no counterpart in the reference: the form of this context's y and z
+ * sweeps at (ord, ngll) = (3, 2) and (5, 3), FP64, FP32 and with tracers.  0 (the
+ * default): by rules on the grid; 1: tiles; 2: column walkers (with tracers only for
+ * lines of 8 cells and more).  The forms give the same FP64 states and tendencies, bit
+ * for bit; FP32 and tracers to rounding. */
+int awfl_set_sweep_form(awfl_ctx* ctx, int form);
 /* awfl_time_step that allocates nothing: no counterpart in the reference.
  * For callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  The same
