@@ -3,12 +3,16 @@
 // of the Euler fluxes, time averaging of the cell-edge states, and the
 // upwind characteristic Riemann flux.
 //
-// Every routine restates the reference's formula in the reference's operation
-// order (the FP64 CPU oracle follows the same order), with three arithmetic
-// changes that keep the result within a few ulp per operation: divisions by
-// constants or by a value used several times become multiplications by a
-// reciprocal (compile-time, launch-time, or rcp() refined to ~1 ulp);
-// (rho theta)^GAMMA uses pow_gamma(); products and sums contract to FMA.
+// The values are the reference's formulas', in forms of fewer operations: WENO5 and
+// WENO3 in differences of the stencil (reconstruct_w5, reconstruct_w3), the general
+// reconstruction with folded maps (weno_coefs), the transform by the normal velocity's
+// Taylor coefficients (cell_transform), the flux in differences of the two sides
+// (riemann); reciprocals (rcp(), ~1 ulp) for divisions, several from one where they go
+// together, and (rho theta)^GAMMA by pow_gamma().  Multiply-adds of the difference
+// forms, the transform and the flux are written out (fm) with the compiler's own
+// contraction off, so that every kernel rounds them alike; the general reconstruction
+// contracts as the compiler chooses.  The reference's operation order is the CPU
+// oracle's and, for test builds, awfl_cell_ref.hpp's.
 //   WENO ..................... WenoLimiter.h:12-25, 93-172
 //   reconstruction ........... Spatial_euler3d_cons_expl_cart_fv_Agrid.h (S:) 1800-1833
 //   level-0 products ......... S:704-715, 1067-1078, 1428-1440

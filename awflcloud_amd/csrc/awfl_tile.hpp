@@ -19,7 +19,8 @@
 // barrier, so whole lines may be updated in place.
 //
 // What bounds it: instruction issue (and the clock the FP64 load leaves).  One
-// cell per lane takes 96-106 registers in FP64, four or five waves per SIMD.
+// cell per lane takes 96 registers in FP64 x and y, five waves per SIMD, and 112 in z,
+// four.
 // Work-groups are best four waves or fewer: the more of them a CU holds, the
 // less a barrier costs (y at 256x256x128 in segments: 330 us with four waves,
 // 371 with seven, 396 with six).  LDS holds a cell's 5 values contiguously:

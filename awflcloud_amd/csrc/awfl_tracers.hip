@@ -25,8 +25,9 @@
 // (k_walk_tr: four x-adjacent lines per work-group walked in 64-cell steps);
 // WENO9/ADER5, and x lines past a tile, run one line per work-group with the
 // line in LDS (k_sweep_tr).  All run the production sweep's statements
-// (cell_edges / riemann) for the state, so the state they return is
-// awfl_sweep's up to the compiler's contraction choices in these kernels.
+// (cell_edges / riemann) for the state: it is awfl_sweep's bit for bit in WENO3 and
+// WENO5, whose multiply-adds are written out, and to the compiler's contraction
+// choices in WENO9.
 // Departures from the source text, where it cannot run as written:
 //   T1 the limiter forms every cell's reduction factor from the unlimited
 //      fluxes and then applies it to the faces it is upwind of; the
@@ -1365,6 +1366,8 @@ int launch_sweep_tr(awfl_ctx* c, const double* in, const double* tr_in, double* 
   const int n = dir == 0 ? c->cfg.nx : dir == 1 ? c->cfg.ny : c->cfg.nz;
   const int W = n + 2 * c->hs, ntr = c->ntr;
   const int64_t nc = (int64_t)c->cfg.nx * c->cfg.ny * c->cfg.nz;
+  // (where no walker takes a line, what the line kernel's LDS cannot hold is refused,
+  // also of the lines that run as tiles, which take a little less)
   const bool walks = dir > 0 && n >= 8 && v->wupd[dir - 1];
   const size_t lds = sizeof(double) * (size_t)(5 * W + ntr * W + 10 * n + 2 * ntr * n + (dir == 2 ? 2 : 1) * n);
   if (!walks && lds > 160 * 1024) return fail(c, AWFL_E_UNSUPPORTED, "tracers: line too long for the tracer sweep's LDS");
