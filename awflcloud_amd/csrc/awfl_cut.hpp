@@ -205,14 +205,17 @@ inline TtCut tt_cut(int dir, int n, int64_t lines, int hs, int ntr) {
 // tile where that takes single y lines and there are few tracers (so that the walker's
 // LDS lets a CU hold its waves), once the grid fills the chip: 39x456x215 with one tracer
 // 303 (tile) and 231 us, 92x449x80 with three 364 and 287, 59x189x181 with three 171 and
-// 157; but with five 520 and 594 at 237x147x116.  A grid with fewer walker groups than
-// CUs waits for one walk: 17x520x10 with five tracers 24 (tile) and 91 us, 57x6x388
-// with eight 48 and 101 (z).
+// 157; but with five 520 and 594 at 237x147x116.  Two tracers take the tile's LDS of
+// three and leave it behind by pairs of lines as well (cost 1.11): 156x228x160 398 and 368
+// us, 288x237x52 250 and 221, where one and three are even or ahead (66x210x76 80 and
+// 106).  A grid with fewer walker groups than CUs waits for one walk: 17x520x10 with five
+// tracers 24 (tile) and 91 us, 57x6x388 with eight 48 and 101 (z).
 inline bool tt_tile(const TtCut& cut, int dir, int ord, int n, int64_t groups, int ntr) {
   if (groups <= 192) return true;
   const double walker = (n + 63) / 64 * 64.0 / n;
-  const bool quick = dir == 2 || (ord == 3 && ntr < 4 && groups > 1024);
-  return cut.cost < (quick ? 1.3 : 1.45) * walker;
+  const bool quick = ord == 3 && ntr < 4 && groups > 1024;
+  const double line = dir == 2 ? 1.3 : !quick ? 1.45 : ntr == 2 ? 1.05 : 1.3;
+  return cut.cost < line * walker;
 }
 
 // ---------------------------------------------------------------------------

@@ -128,6 +128,10 @@ def test_tracer_tiles_fit(cuts):
     (1, 3, (39, 456, 215), 1, "walker"),
     (1, 3, (92, 449, 80), 3, "walker"),
     (1, 3, (59, 189, 181), 3, "walker"),
+    (1, 3, (156, 228, 160), 2, "walker"),
+    (1, 3, (288, 237, 52), 2, "walker"),
+    (1, 3, (66, 210, 76), 3, "tile"),
+    (1, 3, (224, 134, 62), 2, "tile"),
     (1, 3, (237, 147, 116), 5, "tile"),
     (1, 3, (170, 249, 7), 2, "tile"),
     (1, 3, (17, 520, 10), 5, "tile"),
